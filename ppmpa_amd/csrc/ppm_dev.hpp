@@ -79,14 +79,13 @@ __device__ __forceinline__ float chan(float4 c, uint32_t wl) {
 // (element, pass, stream tag, block) so that the FP64 oracle draws the same
 // numbers.
 
+// Each round's two products are taken whole (one v_mad_u64_u32 instead of a
+// low and a high multiplication, all of them quarter-rate).
 __device__ __forceinline__ uint4 philox4x32_10(uint4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int i = 0; i < 10; ++i) {
-    uint32_t lo0 = PHILOX_M0 * c.x;
-    uint32_t hi0 = __umulhi(PHILOX_M0, c.x);
-    uint32_t lo1 = PHILOX_M1 * c.z;
-    uint32_t hi1 = __umulhi(PHILOX_M1, c.z);
-    c = make_uint4(hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0);
+    const uint64_t p0 = (uint64_t)PHILOX_M0 * c.x, p1 = (uint64_t)PHILOX_M1 * c.z;
+    c = make_uint4((uint32_t)(p1 >> 32) ^ c.y ^ k0, (uint32_t)p1, (uint32_t)(p0 >> 32) ^ c.w ^ k1, (uint32_t)p0);
     k0 += PHILOX_W0;
     k1 += PHILOX_W1;
   }
@@ -118,7 +117,50 @@ struct Rng {
     uint32_t v = j == 0 ? blk.x : (j == 1 ? blk.y : (j == 2 ? blk.z : blk.w));
     return u01(v);
   }
+
+  // The next four draws without consuming them, w.d[k] being the k-th, from
+  // one new block computed at one place: lanes of a wave stand at different
+  // draws of their blocks, and next() at each draw's own place had the wave
+  // compute a block nearly every time.  used(w, m) then consumes the first m
+  // (m <= 4).
+  struct Window {
+    float d[4];
+    uint4 b;  // block n / 4 when n % 4 == 0, else the one after it
+  };
+  __device__ __forceinline__ Window peek4() const {
+    const uint32_t j = n & 3u;
+    Window w;
+    w.b = philox4x32_10(make_uint4(c0, c1, c2, (n + 3u) >> 2), k0, k1);
+    const bool j1 = (j & 1u) != 0u, j2 = (j & 2u) != 0u;
+    // v[0..6]: the draws from the current block's start (j > 0: blk then w.b)
+    const uint32_t v0 = j == 0u ? w.b.x : blk.x, v1 = j == 0u ? w.b.y : blk.y, v2 = j == 0u ? w.b.z : blk.z;
+    const uint32_t v3 = j == 0u ? w.b.w : blk.w;
+    const uint32_t s0 = j2 ? v2 : v0, s1 = j2 ? v3 : v1, s2 = j2 ? w.b.x : v2, s3 = j2 ? w.b.y : v3;
+    const uint32_t s4 = j2 ? w.b.z : w.b.x;
+    w.d[0] = u01(j1 ? s1 : s0);
+    w.d[1] = u01(j1 ? s2 : s1);
+    w.d[2] = u01(j1 ? s3 : s2);
+    w.d[3] = u01(j1 ? s4 : s3);
+    return w;
+  }
+  __device__ __forceinline__ void used(const Window& w, uint32_t m) {
+    const uint32_t j = n & 3u;
+    const bool moved = j == 0u || j + m > 4u;  // draw n + m lies in w.b (or starts a block of its own)
+    blk.x = moved ? w.b.x : blk.x;
+    blk.y = moved ? w.b.y : blk.y;
+    blk.z = moved ? w.b.z : blk.z;
+    blk.w = moved ? w.b.w : blk.w;
+    n += m;
+  }
 };
+
+// Draws s and s + 1 (s even) of the stream (seed, elem, pass, tag).
+__device__ __forceinline__ void rng_pair(uint64_t seed, uint32_t elem, uint32_t pass, uint32_t tag, uint32_t s,
+                                         float& u0, float& u1) {
+  const uint4 b = philox4x32_10(make_uint4(elem, pass, tag, s >> 2), (uint32_t)seed, (uint32_t)(seed >> 32));
+  u0 = u01((s & 2u) != 0u ? b.z : b.x);
+  u1 = u01((s & 2u) != 0u ? b.w : b.y);
+}
 
 // ---------------------------------------------------------------------------
 // Scene view passed by value to every kernel.
@@ -555,26 +597,32 @@ __device__ __forceinline__ float schlick(float f0, float c) { return f0 + (1.0f 
 
 // generate_random_dir_by_angle (algebra.rs:225-235) + diffuse_reflection
 // (surface.rs:408-417): uniform on the sphere, flipped into n's hemisphere.
-__device__ __forceinline__ V3 diffuse_reflection(V3 n, Rng& rng) {
-  float phi = TWO_PI_F * rng.next();
-  float xi = 2.0f * rng.next() - 1.0f;
+// u0, u1: the two uniform draws.
+__device__ __forceinline__ V3 diffuse_reflection(V3 n, float u0, float u1) {
+  float phi = TWO_PI_F * u0;
+  float xi = 2.0f * u1 - 1.0f;
   float xi2 = __builtin_amdgcn_sqrtf(fmaxf(1.0f - xi * xi, 0.0f));
   const float sp = __sinf(phi), cp = __cosf(phi);  // = __sincosf, without its pointer outputs
   V3 d = normalize_or(mk(xi2 * cp, xi, xi2 * sp), mk(0.0f, 1.0f, 0.0f));
   return sel(dot(n, d) > 0.0f, d, -d);
 }
+__device__ __forceinline__ V3 diffuse_reflection(V3 n, Rng& rng) {
+  const float u0 = rng.next();
+  const float u1 = rng.next();
+  return diffuse_reflection(n, u0, u1);
+}
 
 // reflection_glossy (physics.rs:232-261).  xi1 = xi0^(pw c0) is formed as
 // exp(t) with 1 - xi1 = -expm1(t), t = pw c0 ln xi0, so that the tiny
 // deviation of near-mirror surfaces (pw ~ 1e-5) keeps float precision.
-__device__ __forceinline__ V3 reflection_glossy(V3 n, V3 r, float pw, Rng& rng) {
+// xi0, u1: the two uniform draws.
+__device__ __forceinline__ V3 reflection_glossy(V3 n, V3 r, float pw, float xi0, float u1) {
   V3 u;
   if (!normalize(cross(mk(0.00424f, 1.0f, 0.00764f), r), u))
     u = normalize_or(cross(mk(1.0f, 0.00424f, 0.00764f), r), mk(1.0f, 0.0f, 0.0f));
   V3 v = cross(u, r);
   float c0 = dot(n, r);
-  float xi0 = rng.next();
-  float xi2 = TWO_PI_F * rng.next();
+  float xi2 = TWO_PI_F * u1;
   float e = pw * c0;
   float xi1, one_m;
   if (xi0 == 0.0f) {  // 0^e: 1 when e == 0, else 0
