@@ -36,7 +36,14 @@ struct ppm_ctx {
   int n_cu = 256;
   std::string err;
   hipStream_t aux[AUX_N] = {};
+  unsigned char* stage = nullptr;      // STAGE_BYTES of pinned host memory (ctx_stage)
+  hipEvent_t stage_ev[2] = {};         // one per half of it
 };
+
+// Pinned host memory a context keeps for bringing results to the caller's
+// arrays: kernels write one half of it while the host empties the other.
+constexpr size_t STAGE_BYTES = 8u << 20;
+constexpr size_t STAGE_HALF = STAGE_BYTES / 2 - 256;  // payload of a half; its last 256 bytes hold flags
 
 struct ppm_scene {
   ppm_ctx* ctx = nullptr;
@@ -132,6 +139,22 @@ void ctx_stream_renew(ppm_ctx* c, int i) {
     (void)hipStreamDestroy(c->aux[i]);
   }
   c->aux[i] = nullptr;
+}
+
+// The context's pinned staging memory and its events (made on first use,
+// kept until ppm_destroy).
+hipError_t ctx_stage(ppm_ctx* c) {
+  hipError_t e;
+  if (!c->stage && (e = hipHostMalloc((void**)&c->stage, STAGE_BYTES, hipHostMallocDefault)) != hipSuccess) {
+    c->stage = nullptr;
+    return e;
+  }
+  for (hipEvent_t& v : c->stage_ev)
+    if (!v && (e = hipEventCreateWithFlags(&v, hipEventDisableTiming)) != hipSuccess) {
+      v = nullptr;
+      return e;
+    }
+  return hipSuccess;
 }
 
 ppm_status fail(ppm_ctx* c, ppm_status s, const std::string& msg) {
@@ -471,6 +494,12 @@ void ppm_destroy(ppm_ctx* c) {
       (void)hipStreamDestroy(a);
       a = nullptr;
     }
+  if (c->stage) {
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipHostFree(c->stage);
+  }
+  for (hipEvent_t v : c->stage_ev)
+    if (v) (void)hipEventDestroy(v);
   if (c->own_stream && c->stream) {
     (void)hipStreamSynchronize(c->stream);
     (void)hipStreamDestroy(c->stream);
@@ -1841,21 +1870,15 @@ static hipError_t pipe_states(ppm_session* s, std::vector<PassState>& h) {
   return e;
 }
 
-// Sum and sum of squares over all passes: the pipelines' FP64 sums added
-// in pipeline order.
-static hipError_t merged_sums(ppm_session* s, std::vector<double>& sum, std::vector<double>* sq) {
+// Sum over all passes: the pipelines' FP64 sums added in pipeline order.
+static hipError_t merged_sum(ppm_session* s, std::vector<double>& sum) {
   const uint64_t n3 = 3ull * s->pipes[0].eb.n_pix;
   sum.assign(n3, 0.0);
-  if (sq) sq->assign(n3, 0.0);
   std::vector<double> a(n3);
   for (Pipe& p : s->pipes) {
-    hipError_t e = hipMemcpy(a.data(), p.sum, sizeof(double) * n3, hipMemcpyDeviceToHost);
+    const hipError_t e = hipMemcpy(a.data(), p.sum, sizeof(double) * n3, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return e;
     for (uint64_t i = 0; i < n3; ++i) sum[i] += a[i];
-    if (sq) {
-      if ((e = hipMemcpy(a.data(), p.sumsq, sizeof(double) * n3, hipMemcpyDeviceToHost)) != hipSuccess) return e;
-      for (uint64_t i = 0; i < n3; ++i) (*sq)[i] += a[i];
-    }
   }
   return hipSuccess;
 }
@@ -2013,7 +2036,7 @@ ppm_status ppm_session_backward(ppm_session* s, const double* grad_image, double
   if (grad_light) {
     // the image is proportional to the light scale: dL/ds = sum g * mean / s
     std::vector<double> sum;
-    HIP_TRY(c, merged_sums(s, sum, nullptr));
+    HIP_TRY(c, merged_sum(s, sum));
     double acc = 0.0;
     for (size_t i = 0; i < sum.size(); ++i) acc += grad_image[i] * (sum[i] / K);
     *grad_light = sc->light_scale > 0.0 ? acc / sc->light_scale : 0.0;
@@ -2035,21 +2058,46 @@ ppm_status ppm_session_radius2(ppm_session* s, double* r2) {
 ppm_status ppm_session_image(ppm_session* s, double* mean_out, double* var_out, uint32_t* passes_done) {
   if (!s) return PPM_E_INVALID;
   ppm_ctx* c = s->ctx;
-  std::vector<PassState> h;
-  HIP_TRY(c, pipe_states(s, h));
   if (passes_done) *passes_done = s->passes_done;
-  for (const PassState& x : h) {
-    if (x.overflow)
-      return fail(c, PPM_E_RANGE, "capacity exceeded during a pass: " + overflow_text(x.overflow));
-    if (x.nonfinite) return fail(c, PPM_E_NONFINITE, "non-finite photon position (photonmap.rs:26)");
+  HIP_TRY(c, ctx_stage(c));
+  ImageSrc src;
+  src.n_pipes = (uint32_t)s->pipes.size();
+  for (uint32_t j = 0; j < src.n_pipes; ++j) {
+    src.sum[j] = s->pipes[j].sum;
+    src.sumsq[j] = s->pipes[j].sumsq;
+    src.st[j] = s->pipes[j].st;
   }
-  std::vector<double> sum, sq;
-  HIP_TRY(c, merged_sums(s, sum, &sq));
-  const uint64_t n3 = sum.size();
-  const double n = (double)s->passes_done;
-  for (uint64_t i = 0; i < n3; ++i) {
-    if (mean_out) mean_out[i] = n > 0 ? sum[i] / n : 0.0;
-    if (var_out) var_out[i] = n > 1 ? std::max(0.0, (sq[i] - sum[i] * sum[i] / n) / (n - 1.0)) : 0.0;
+  // chunks of the image alternate between the halves of the staging memory:
+  // k_image writes one while the other is copied out
+  const uint64_t n3 = 3ull * s->pipes[0].eb.n_pix;
+  const uint32_t outs = (mean_out ? 1u : 0u) + (var_out ? 1u : 0u);
+  const uint64_t per = outs ? STAGE_HALF / (sizeof(double) * outs) : n3;
+  const uint64_t chunks = outs ? (n3 + per - 1) / per : 1;
+  auto half = [&](uint64_t k) { return c->stage + (k & 1u) * (STAGE_BYTES / 2); };
+  auto flags = [&](uint64_t k) { return reinterpret_cast<uint32_t*>(half(k) + STAGE_HALF); };
+  auto queue = [&](uint64_t k) -> hipError_t {
+    double* d = reinterpret_cast<double*>(half(k));
+    const uint64_t n = outs ? std::min(per, n3 - k * per) : 0;
+    const hipError_t e = launch_image(c->stream, src, k * per, (uint32_t)n, s->passes_done, mean_out ? d : nullptr,
+                                      var_out ? d + (mean_out ? n : 0) : nullptr, flags(k));
+    return e != hipSuccess ? e : hipEventRecord(c->stage_ev[k & 1u], c->stream);
+  };
+  HIP_TRY(c, queue(0));
+  for (uint64_t k = 0; k < chunks; ++k) {
+    if (k + 1 < chunks) HIP_TRY(c, queue(k + 1));
+    hipError_t e = hipEventSynchronize(c->stage_ev[k & 1u]);
+    const uint32_t over = e == hipSuccess ? flags(k)[0] : 0u, bad = e == hipSuccess ? flags(k)[1] : 0u;
+    if (e != hipSuccess || over || bad) {
+      const hipError_t e2 = hipStreamSynchronize(c->stream);  // the queued chunk still writes the staging memory
+      if (e == hipSuccess) e = e2;
+      HIP_TRY(c, e);
+      if (over) return fail(c, PPM_E_RANGE, "capacity exceeded during a pass: " + overflow_text(over));
+      return fail(c, PPM_E_NONFINITE, "non-finite photon position (photonmap.rs:26)");
+    }
+    const double* d = reinterpret_cast<const double*>(half(k));
+    const uint64_t n = outs ? std::min(per, n3 - k * per) : 0;
+    if (mean_out) std::memcpy(mean_out + k * per, d, n * sizeof(double));
+    if (var_out) std::memcpy(var_out + k * per, d + (mean_out ? n : 0), n * sizeof(double));
   }
   return PPM_OK;
 }

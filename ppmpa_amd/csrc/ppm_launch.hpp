@@ -279,6 +279,21 @@ hipError_t launch_bvh_build(hipStream_t s, const DevShape* shapes, const uint32_
                             uint32_t* ghist, uint32_t* totals, uint32_t sort_blocks, Node* pbox, DevShape* bprims,
                             Node* nodes);
 
+// The mean and variance of `passes` passes from the FP64 sums of a session's
+// pipelines (added in pipeline order), values [base, base + n) of the image's
+// 3 per pixel: to mean and var (either may be null; host memory the GPU can
+// write), and the OR of the pipelines' overflow and nonfinite words to
+// flags[0..1].
+constexpr uint32_t MAX_PIPES = 4;
+struct ImageSrc {
+  const double* sum[MAX_PIPES] = {};
+  const double* sumsq[MAX_PIPES] = {};
+  const PassState* st[MAX_PIPES] = {};
+  uint32_t n_pipes = 0;
+};
+hipError_t launch_image(hipStream_t s, const ImageSrc& src, uint64_t base, uint32_t n, uint32_t passes, double* mean,
+                        double* var, uint32_t* flags);
+
 // One scene of a batch: everything its pass kernels read (device memory).
 struct BatchItem {
   SceneBuf sc;
