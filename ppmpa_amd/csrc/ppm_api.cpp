@@ -19,15 +19,17 @@
 
 using namespace ppm;
 
-// Streams a context makes for its sessions and batches on first use and
-// keeps until ppm_destroy, so that creating and destroying sessions creates
-// and destroys no streams: AUX_PIPE + j - 1 runs pass pipeline j >= 1 (its
-// graph launches), AUX_EYE + j the eye branch of pipeline j (forked into a
-// pass graph's capture, or used directly without graphs), AUX_CAPTURE and
-// AUX_CAPTURE2 the streams pass graphs are captured on.  Calls on a context
-// never overlap (each returns once its work is done), so its sessions and
-// batches may share them.
-constexpr int AUX_PIPE = 0, AUX_EYE = 3, AUX_CAPTURE = 7, AUX_CAPTURE2 = 8, AUX_N = 9;
+// Streams of a context beside its own, kept until ppm_destroy, so that
+// creating and destroying sessions creates and destroys no streams: AUX_PIPE
+// + j - 1 runs pass pipeline j >= 1 (pipeline 0 runs on the context's
+// stream), AUX_CAPTURE is the stream pass graphs are captured on (made on
+// first use).  The pipelines' streams are made with the context, right after
+// its own: HIP spreads a process's streams over four hardware queues in the
+// order they are made, and two pipelines on one queue run one after the
+// other (four pipelines whose streams were made after a capture stream: as
+// slow as two).  Calls on a context never overlap (each returns once its
+// work is done), so its sessions and batches may share them.
+constexpr int AUX_PIPE = 0, AUX_CAPTURE = MAX_PIPES - 1, AUX_N = MAX_PIPES;
 
 struct ppm_ctx {
   int device = 0;
@@ -38,6 +40,8 @@ struct ppm_ctx {
   hipStream_t aux[AUX_N] = {};
   unsigned char* stage = nullptr;      // STAGE_BYTES of pinned host memory (ctx_stage)
   hipEvent_t stage_ev[2] = {};         // one per half of it
+  void* work = nullptr;                // the device block calls lay their buffers out in (Work)
+  size_t work_bytes = 0;
 };
 
 // Pinned host memory a context keeps for bringing results to the caller's
@@ -61,6 +65,7 @@ struct ppm_scene {
 
 struct ppm_photons {
   ppm_ctx* ctx = nullptr;
+  void* mem = nullptr;  // pb's arrays and st
   uint64_t cap = 0;
   PhotonBuf pb;
   PassState* st = nullptr;
@@ -72,6 +77,8 @@ struct ppm_photons {
 
 struct ppm_map {
   ppm_ctx* ctx = nullptr;
+  void* mem = nullptr;       // the tree's arrays, the sort's and st
+  void* grid_mem = nullptr;  // the grid's cells and sort state (first grid build)
   MapBuf m;
   PassState* st = nullptr;
   double power = 1.0;
@@ -90,15 +97,16 @@ struct ppm_map {
 // pass graph.  Passes of different pipelines run at once, as the reference's
 // iterator runs NPARA pm | rt processes at once (util/iterator.rb:18,90-117).
 struct Pipe {
+  void* mem = nullptr;  // all of the pipeline's buffers (pipe_alloc)
   PhotonBuf pb;
   MapBuf map;
   EyeBuf eb;
   double* sum = nullptr;
-  double* sumsq = nullptr;
+  double* sumsq = nullptr;  // right after sum
   PassState* st = nullptr;
+  PassState* st_adj = nullptr;   // the state of ppm_session_backward's replay
   hipStream_t stream = nullptr;  // this pipeline's passes, in order
-  hipStream_t s2 = nullptr;      // the eye branch of its passes
-  hipEvent_t evf = nullptr, evj = nullptr, done = nullptr;
+  hipEvent_t done = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
@@ -112,6 +120,9 @@ struct ppm_session {
   double power = 0.0;
   uint32_t passes_done = 0;
   std::vector<Pipe> pipes;  // pass p (from cfg.first_pass) runs on pipes[p % K]
+  std::vector<DevLight> lights_host;  // what `lights` holds
+  float4* gimg = nullptr;   // ppm_session_backward: the image gradient and the
+  double* grad = nullptr;   // material gradients (made on first use)
   hipEvent_t ev[10] = {};
   ppm_timings t{};
 };
@@ -183,22 +194,91 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
+// Several buffers laid out in one allocation: a layout function runs twice,
+// first to add up the size (base null), then, after alloc(), to set the
+// pointers.
+struct Arena {
+  unsigned char* base = nullptr;
+  size_t used = 0;
+  template <typename T>
+  void take(T** p, uint64_t count) {
+    *p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+    used += ((count ? count : 1) * sizeof(T) + 255) & ~(size_t)255;
+  }
+};
+// A device block of the context's; when memory runs out, once more without
+// the block it keeps for its calls.
+hipError_t block_alloc(ppm_ctx* c, void** mem, size_t bytes) {
+  hipError_t e = hipMalloc(mem, bytes ? bytes : 1);
+  if (e == hipErrorOutOfMemory && c->work) {
+    (void)hipGetLastError();
+    dfree(c->work);
+    c->work_bytes = 0;
+    e = hipMalloc(mem, bytes ? bytes : 1);
+  }
+  if (e != hipSuccess) *mem = nullptr;
+  return e;
+}
+
+// layout(arena) twice around one allocation; *mem is to be freed with dfree.
+template <typename F>
+hipError_t arena_alloc(ppm_ctx* c, void** mem, F&& layout, size_t* bytes = nullptr) {
+  Arena a;
+  layout(a);
+  if (bytes) *bytes = a.used;
+  const hipError_t e = block_alloc(c, mem, a.used);
+  if (e != hipSuccess) return e;
+  a.base = static_cast<unsigned char*>(*mem);
+  a.used = 0;
+  layout(a);
+  return hipSuccess;
+}
+
+// The device buffers of one call (which ends with its work done), laid out in
+// the block that the context keeps from call to call: grown to the largest
+// call so far, but at most WORK_KEEP bytes (a larger call allocates and frees
+// its own), given back by ppm_destroy and by block_alloc when memory runs
+// out.  Allocating them per call cost more than the calls' kernels: an eye
+// pass of 640x480 over 500k photons 22.1 -> 2.1 ms.
+constexpr size_t WORK_KEEP = 2ull << 30;
+struct Work {
+  void* own = nullptr;
+  template <typename F>
+  hipError_t get(ppm_ctx* c, F&& layout) {
+    Arena a;
+    layout(a);
+    void* m = c->work;
+    if (a.used > WORK_KEEP) {
+      const hipError_t e = block_alloc(c, &own, a.used);
+      if (e != hipSuccess) return e;
+      m = own;
+    } else if (a.used > c->work_bytes) {
+      dfree(c->work);
+      c->work_bytes = 0;
+      const hipError_t e = block_alloc(c, &c->work, a.used);
+      if (e != hipSuccess) return e;
+      c->work_bytes = a.used;
+      m = c->work;
+    }
+    a.base = static_cast<unsigned char*>(m);
+    a.used = 0;
+    layout(a);
+    return hipSuccess;
+  }
+  Work() = default;
+  Work(const Work&) = delete;
+  Work& operator=(const Work&) = delete;
+  ~Work() { dfree(own); }
+};
+
 // One-sweep sort state for up to cap keys (the look-back words count keys + 1
-// in 31 bits).
-hipError_t onesweep_alloc(OneSweep& o, uint64_t cap, int n_cu) {
-  if (cap >= 0x7FFFFFFFull) return hipErrorInvalidValue;
+// in 31 bits); ctl is cleared by the kernels that write keys.
+void onesweep_layout(Arena& a, OneSweep& o, uint64_t cap, int n_cu) {
   o.cap = cap;
   o.tiles = (uint32_t)std::max<uint64_t>(1, (cap + OS_TILE - 1) / OS_TILE);
   o.blocks = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)n_cu * OS_BLOCKS_PER_CU, o.tiles));
-  hipError_t e;
-  if ((e = dalloc(&o.ctl, OS_CTL_WORDS)) != hipSuccess) return e;
-  if ((e = hipMemset(o.ctl, 0, sizeof(uint32_t) * OS_CTL_WORDS)) != hipSuccess) return e;
-  return dalloc(&o.look, (uint64_t)OS_MAX_DIGITS * o.tiles * 256u);
-}
-
-void onesweep_free(OneSweep& o) {
-  dfree(o.ctl);
-  dfree(o.look);
+  a.take(&o.ctl, OS_CTL_WORDS);
+  a.take(&o.look, (uint64_t)OS_MAX_DIGITS * o.tiles * 256u);
 }
 
 float4 f4(const double v[3], float w = 0.0f) { return make_float4((float)v[0], (float)v[1], (float)v[2], w); }
@@ -248,62 +328,36 @@ ppm_status check_cfg_depth(ppm_ctx* c, int max_depth) {
 }
 
 // A map for cap photons: the box tree (grid = false) or the per-pass grid.
-hipError_t map_alloc(MapBuf& m, uint64_t cap, int n_cu, bool grid) {
+void map_layout(Arena& a, MapBuf& m, uint64_t cap, int n_cu, bool grid) {
   m.cap = cap;
   m.sort_blocks = (uint32_t)std::min<uint64_t>(4096, std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)n_cu * 4,
                                                                                                 (cap + 2047) / 2048)));
-  hipError_t e;
   // the grid's gathers read up to GRID_READ_SLACK records past the last photon
-  if ((e = dalloc(&m.sorted, cap + GRID_READ_SLACK)) != hipSuccess) return e;
-  if ((e = dalloc(&m.src_idx, cap)) != hipSuccess) return e;
+  a.take(&m.sorted, cap + GRID_READ_SLACK);
+  a.take(&m.src_idx, cap);
   if (grid) {
     m.cells_max = (uint32_t)std::min<uint64_t>(GRID_MAX_BUCKETS, next_pow2(std::max<uint64_t>(cap, 1024)));
-    if ((e = dalloc(&m.cells, m.cells_max)) != hipSuccess) return e;
-    if ((e = onesweep_alloc(m.os, cap, n_cu)) != hipSuccess) return e;
+    a.take(&m.cells, m.cells_max);
+    onesweep_layout(a, m.os, cap, n_cu);
   } else {
     const uint64_t leaves = (cap + LEAF - 1) / LEAF;
     m.lpad_max = next_pow2(leaves > 0 ? leaves : 1);
-    if ((e = dalloc(&m.nodes, 2ull * m.lpad_max)) != hipSuccess) return e;
+    a.take(&m.nodes, 2ull * m.lpad_max);
+    a.take(&m.ghist, 256ull * m.sort_blocks);
+    a.take(&m.totals, 256);
   }
   for (int i = 0; i < 2; ++i) {
-    if ((e = dalloc(&m.keys[i], cap)) != hipSuccess) return e;
-    if ((e = dalloc(&m.vals[i], cap)) != hipSuccess) return e;
+    a.take(&m.keys[i], cap);
+    a.take(&m.vals[i], cap);
   }
-  if ((e = dalloc(&m.ghist, 256ull * m.sort_blocks)) != hipSuccess) return e;
-  if ((e = dalloc(&m.totals, 256)) != hipSuccess) return e;
-  return hipSuccess;
 }
 
-void map_free(MapBuf& m) {
-  dfree(m.sorted);
-  dfree(m.sorted64);
-  dfree(m.src_idx);
-  dfree(m.nodes);
-  dfree(m.cells);
-  for (int i = 0; i < 2; ++i) {
-    dfree(m.keys[i]);
-    dfree(m.vals[i]);
-  }
-  dfree(m.ghist);
-  dfree(m.totals);
-  onesweep_free(m.os);
-}
-
-hipError_t photons_alloc(PhotonBuf& pb, uint64_t cap, uint32_t max_regions) {
+void photons_layout_mem(Arena& a, PhotonBuf& pb, uint64_t cap, uint32_t max_regions) {
   pb.cap = cap;
   pb.max_regions = max_regions;
-  hipError_t e;
-  if ((e = dalloc(&pb.rec, cap)) != hipSuccess) return e;
-  if ((e = dalloc(&pb.count, max_regions)) != hipSuccess) return e;
-  if ((e = dalloc(&pb.offset, max_regions)) != hipSuccess) return e;
-  return hipSuccess;
-}
-
-void photons_free(PhotonBuf& pb) {
-  dfree(pb.rec);
-  dfree(pb.rec64);
-  dfree(pb.count);
-  dfree(pb.offset);
+  a.take(&pb.rec, cap);
+  a.take(&pb.count, max_regions);
+  a.take(&pb.offset, max_regions);
 }
 
 // Region layout of a traced pass: one region per tracing wave.
@@ -341,21 +395,31 @@ uint32_t cam_tiles_max(const DevCamera& cam) {
 // The eye buffers at tile shape `shift` (sized for any shape by eye_alloc);
 // the tiles' query counts of earlier passes, which only order the eye's
 // work, start again from zero.
-hipError_t eye_set_tiles(EyeBuf& eb, DevCamera& cam, uint32_t shift) {
+bool eye_tiles(EyeBuf& eb, DevCamera& cam, uint32_t shift) {
   uint32_t tx = 0;
   const uint32_t tiles = cam_tiles(cam, shift, &tx);
-  if (tiles > eb.tiles_cap) return hipErrorInvalidValue;
+  if (tiles > eb.tiles_cap) return false;
   cam.tile_shift = (int32_t)shift;
   cam.tiles_x = (int32_t)tx;
   eb.n_tiles = tiles;
   eb.q_primary = tiles * 64u;
   eb.q_fine = eb.q_primary >= QUERY_FINE_PIXELS ? 1u : 0u;
+  return true;
+}
+hipError_t eye_set_tiles(EyeBuf& eb, DevCamera& cam, uint32_t shift) {
+  if (!eye_tiles(eb, cam, shift)) return hipErrorInvalidValue;
   return hipMemset(eb.tile_count, 0, sizeof(uint32_t) * eb.tiles_cap);
 }
 
-hipError_t eye_alloc(EyeBuf& eb, const DevCamera& cam, int max_depth, int n_cu) {
-  // buffers for the most tiles any tile shape needs, so that a batch can
-  // tune the shape without reallocating
+// The eye's buffers, for the most tiles any tile shape needs, so that a batch
+// can tune the shape without reallocating.  What only the eye kernel and the
+// query sort use (the pending pool, the dense positions, the sort's keys) and
+// the results that the shade writes after them share memory with each other
+// and, in a pass, with the traced records (pb; null: none): those are written
+// after the query sort and read for the last time by the grid's sort, before
+// the shade.  A pass runs its stages in that order, or trace and grid first.
+void eye_layout(Arena& a, EyeBuf& eb, const DevCamera& cam, int max_depth, int n_cu, PhotonBuf* pb, uint64_t pcap,
+                uint32_t max_regions) {
   const uint32_t tiles = cam_tiles_max(cam);
   eb.tiles_cap = tiles;
   eb.q_primary = tiles * 64u;
@@ -363,44 +427,45 @@ hipError_t eye_alloc(EyeBuf& eb, const DevCamera& cam, int max_depth, int n_cu) 
   eb.sec_max = (uint32_t)std::max(1, std::min(2 * max_depth, 32));
   eb.n_pix = (uint32_t)cam.xreso * (uint32_t)cam.yreso;
   eb.ovf_cap = 2u * eb.n_pix + 1024u;
-  const uint64_t inplace = (uint64_t)eb.q_primary * (1u + eb.sec_max);
-  hipError_t e;
-  if ((e = dalloc(&eb.q, inplace + eb.ovf_cap)) != hipSuccess) return e;
-  if ((e = dalloc(&eb.qpos, inplace + eb.ovf_cap)) != hipSuccess) return e;
-  if ((e = dalloc(&eb.sec_count, eb.q_primary)) != hipSuccess) return e;
-  if ((e = dalloc(&eb.pix, eb.n_pix)) != hipSuccess) return e;
-  if ((e = dalloc(&eb.tile_count, tiles)) != hipSuccess) return e;
-  if ((e = hipMemset(eb.tile_count, 0, sizeof(uint32_t) * tiles)) != hipSuccess) return e;
-  if ((e = dalloc(&eb.tile_off, tiles)) != hipSuccess) return e;
-  if ((e = dalloc(&eb.tile_order, tiles)) != hipSuccess) return e;
-  for (int i = 0; i < 2; ++i) {
-    if ((e = dalloc(&eb.qkeys[i], inplace + eb.ovf_cap)) != hipSuccess) return e;
-    if ((e = dalloc(&eb.qvals[i], inplace + eb.ovf_cap)) != hipSuccess) return e;
-  }
-  if ((e = onesweep_alloc(eb.qos, inplace + eb.ovf_cap, n_cu)) != hipSuccess) return e;
-  if ((e = dalloc(&eb.res, inplace + eb.ovf_cap)) != hipSuccess) return e;
+  const uint64_t slots = (uint64_t)eb.q_primary * (1u + eb.sec_max) + eb.ovf_cap;
   eb.estack_lanes = 64u * std::max<uint32_t>(1, std::min<uint32_t>(tiles, (uint32_t)n_cu * EYE_WAVES_PER_CU_MAX));
   eb.estack_depth = (uint32_t)std::max(1, std::min(max_depth, MAX_DEPTH_LIMIT));
-  if ((e = dalloc(&eb.estack, 3ull * eb.estack_depth * eb.estack_lanes)) != hipSuccess) return e;
-  DevCamera c = cam;
-  return eye_set_tiles(eb, c, (uint32_t)cam.tile_shift);
+  a.take(&eb.q, slots);
+  a.take(&eb.sec_count, eb.q_primary);
+  a.take(&eb.pix, eb.n_pix);
+  a.take(&eb.tile_count, tiles);
+  a.take(&eb.tile_off, tiles);
+  a.take(&eb.tile_order, tiles);
+  a.take(&eb.qvals[0], slots);  // the sorted order, read by the shade
+  onesweep_layout(a, eb.qos, slots, n_cu);
+  const size_t at = a.used;
+  size_t end = at;
+  auto overlay = [&](auto&& f) {
+    a.used = at;
+    f();
+    end = std::max(end, a.used);
+  };
+  overlay([&] {
+    a.take(&eb.qpos, slots);
+    a.take(&eb.qkeys[0], slots);
+    a.take(&eb.qkeys[1], slots);
+    a.take(&eb.qvals[1], slots);
+    a.take(&eb.estack, 3ull * eb.estack_depth * eb.estack_lanes);
+  });
+  overlay([&] { a.take(&eb.res, slots); });
+  if (pb) overlay([&] { photons_layout_mem(a, *pb, pcap, max_regions); });
+  a.used = end;
 }
 
-void eye_free(EyeBuf& eb) {
-  dfree(eb.q);
-  dfree(eb.qpos);
-  dfree(eb.sec_count);
-  dfree(eb.pix);
-  dfree(eb.tile_count);
-  dfree(eb.tile_off);
-  dfree(eb.tile_order);
-  for (int i = 0; i < 2; ++i) {
-    dfree(eb.qkeys[i]);
-    dfree(eb.qvals[i]);
-  }
-  onesweep_free(eb.qos);
-  dfree(eb.res);
-  dfree(eb.estack);
+// The eye's buffers alone and a pass state (one pass outside a session).
+hipError_t eye_work(ppm_ctx* c, Work& w, EyeBuf& eb, PassState** st, const DevCamera& cam, int max_depth) {
+  const hipError_t e = w.get(c, [&](Arena& a) {
+    a.take(st, 1);
+    eye_layout(a, eb, cam, max_depth, c->n_cu, nullptr, 0, 0);
+  });
+  if (e != hipSuccess) return e;
+  DevCamera cm = cam;
+  return eye_set_tiles(eb, cm, (uint32_t)cam.tile_shift);
 }
 
 // What the overflow flags of a pass state say (device-side bits 1 photon
@@ -482,6 +547,13 @@ ppm_status ppm_create(ppm_ctx** out, int device, void* hip_stream) {
     }
     c->own_stream = true;
   }
+  for (int i = AUX_PIPE; i < AUX_CAPTURE; ++i) {
+    hipStream_t s;
+    if (ctx_stream(c, i, &s) != hipSuccess) {
+      ppm_destroy(c);
+      return PPM_E_HIP;
+    }
+  }
   *out = c;
   return PPM_OK;
 }
@@ -494,10 +566,9 @@ void ppm_destroy(ppm_ctx* c) {
       (void)hipStreamDestroy(a);
       a = nullptr;
     }
-  if (c->stage) {
-    (void)hipStreamSynchronize(c->stream);
-    (void)hipHostFree(c->stage);
-  }
+  if (c->stage || c->work) (void)hipStreamSynchronize(c->stream);
+  if (c->stage) (void)hipHostFree(c->stage);
+  dfree(c->work);
   for (hipEvent_t v : c->stage_ev)
     if (v) (void)hipEventDestroy(v);
   if (c->own_stream && c->stream) {
@@ -1036,8 +1107,10 @@ ppm_status ppm_photons_create(ppm_ctx* c, uint64_t capacity, ppm_photons** out) 
   ppm_photons* p = new ppm_photons();
   p->ctx = c;
   p->cap = capacity;
-  hipError_t e = photons_alloc(p->pb, capacity, 8192);
-  if (e == hipSuccess) e = dalloc(&p->st, 1);
+  hipError_t e = arena_alloc(c, &p->mem, [&](Arena& a) {
+    photons_layout_mem(a, p->pb, capacity, 8192);
+    a.take(&p->st, 1);
+  });
   if (e != hipSuccess) {
     ppm_photons_destroy(p);
     return fail(c, PPM_E_OOM, hipGetErrorString(e));
@@ -1059,8 +1132,8 @@ ppm_status ppm_photons_create(ppm_ctx* c, uint64_t capacity, ppm_photons** out) 
 void ppm_photons_destroy(ppm_photons* p) {
   if (!p) return;
   if (p->ctx) (void)hipStreamSynchronize(p->ctx->stream);
-  photons_free(p->pb);
-  dfree(p->st);
+  dfree(p->pb.rec64);
+  dfree(p->mem);
   delete p;
 }
 
@@ -1200,8 +1273,10 @@ ppm_status ppm_map_create(ppm_ctx* c, uint64_t capacity, ppm_map** out) {
   if (capacity == 0 || capacity > 0x7FFFFFFFull) return fail(c, PPM_E_RANGE, "capacity must be in [1, 2^31)");
   ppm_map* m = new ppm_map();
   m->ctx = c;
-  hipError_t e = map_alloc(m->m, capacity, c->n_cu, false);
-  if (e == hipSuccess) e = dalloc(&m->st, 1);
+  const hipError_t e = arena_alloc(c, &m->mem, [&](Arena& a) {
+    map_layout(a, m->m, capacity, c->n_cu, false);
+    a.take(&m->st, 1);
+  });
   if (e != hipSuccess) {
     ppm_map_destroy(m);
     return fail(c, PPM_E_OOM, hipGetErrorString(e));
@@ -1213,8 +1288,9 @@ ppm_status ppm_map_create(ppm_ctx* c, uint64_t capacity, ppm_map** out) {
 void ppm_map_destroy(ppm_map* m) {
   if (!m) return;
   if (m->ctx) (void)hipStreamSynchronize(m->ctx->stream);
-  map_free(m->m);
-  dfree(m->st);
+  dfree(m->m.sorted64);
+  dfree(m->mem);
+  dfree(m->grid_mem);
   dfree(m->hook_mat);
   delete m;
 }
@@ -1252,11 +1328,14 @@ ppm_status ppm_map_build_grid(ppm_ctx* c, const ppm_scene* sc, const ppm_photons
   const double* hi = sc ? sc->bmax : ph->bmax;
   if (!sc && !ph->has_bounds) return fail(c, PPM_E_INVALID, "no bounds for the grid");
   m->built = false;
-  if (!m->m.cells) {
-    m->m.cells_max = (uint32_t)std::min<uint64_t>(GRID_MAX_BUCKETS, next_pow2(std::max<uint64_t>(m->m.cap, 1024)));
-    HIP_TRY(c, dalloc(&m->m.cells, m->m.cells_max));
-  }
-  if (!m->m.os.ctl) HIP_TRY(c, onesweep_alloc(m->m.os, m->m.cap, c->n_cu));
+  if (m->m.cap >= 0x7FFFFFFFull) HIP_TRY(c, hipErrorInvalidValue);  // the sort's look-back words count 31 bits
+  if (!m->grid_mem)
+    HIP_TRY(c, arena_alloc(c, &m->grid_mem, [&](Arena& a) {
+              m->m.cells_max =
+                  (uint32_t)std::min<uint64_t>(GRID_MAX_BUCKETS, next_pow2(std::max<uint64_t>(m->m.cap, 1024)));
+              a.take(&m->m.cells, m->m.cells_max);
+              onesweep_layout(a, m->m.os, m->m.cap, c->n_cu);
+            }));
   if (!m->hook_mat) {
     DevMaterial air;
     std::memset(&air, 0, sizeof(air));
@@ -1526,13 +1605,13 @@ ppm_status ppm_trace_eye(ppm_ctx* c, const ppm_scene* sc, const ppm_map* m, uint
   if (pfilter < 0 || pfilter > 2) return fail(c, PPM_E_INVALID, "bad photon filter");
   if (m->grid && r2 > m->grid_r2) return fail(c, PPM_E_INVALID, "r2 exceeds the radius the grid was built for");
   EyeBuf eb;
+  Work work;
   PassState* st = nullptr;
   hipError_t e = hipSuccess;
   std::vector<float4> h;
   PassState hs;
   do {
-    if ((e = eye_alloc(eb, sc->buf.cam, max_depth, c->n_cu)) != hipSuccess) break;
-    if ((e = dalloc(&st, 1)) != hipSuccess) break;
+    if ((e = eye_work(c, work, eb, &st, sc->buf.cam, max_depth)) != hipSuccess) break;
     if ((e = hipMemcpyAsync(&hs, m->st, sizeof(PassState), hipMemcpyDeviceToHost, c->stream)) != hipSuccess) break;
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) break;
     hs.pass = pass;
@@ -1562,8 +1641,6 @@ ppm_status ppm_trace_eye(ppm_ctx* c, const ppm_scene* sc, const ppm_map* m, uint
     if ((e = hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, c->stream)) != hipSuccess) break;
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) break;
   } while (0);
-  eye_free(eb);
-  dfree(st);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
   if (hs.overflow) return fail(c, PPM_E_RANGE, "gather query buffer overflow");
   for (size_t p = 0; p < h.size(); ++p) {
@@ -1580,13 +1657,13 @@ ppm_status ppm_trace_classic(ppm_ctx* c, const ppm_scene* sc, uint64_t seed, uin
   for (int k = 0; k < 3; ++k)
     if (!std::isfinite(ambient[k])) return fail(c, PPM_E_INVALID, "bad ambient radiance");
   EyeBuf eb;
+  Work work;
   PassState* st = nullptr;
   hipError_t e = hipSuccess;
   std::vector<float4> h;
   PassState hs = host_state();
   do {
-    if ((e = eye_alloc(eb, sc->buf.cam, CLASSIC_DEPTH, c->n_cu)) != hipSuccess) break;
-    if ((e = dalloc(&st, 1)) != hipSuccess) break;
+    if ((e = eye_work(c, work, eb, &st, sc->buf.cam, CLASSIC_DEPTH)) != hipSuccess) break;
     hs.pass = pass;
     if ((e = hipMemcpy(st, &hs, sizeof(hs), hipMemcpyHostToDevice)) != hipSuccess) break;
     const float4 amb = make_float4((float)ambient[0], (float)ambient[1], (float)ambient[2], 0.0f);
@@ -1598,8 +1675,6 @@ ppm_status ppm_trace_classic(ppm_ctx* c, const ppm_scene* sc, uint64_t seed, uin
     if ((e = hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, c->stream)) != hipSuccess) break;
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) break;
   } while (0);
-  eye_free(eb);
-  dfree(st);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
   if (hs.overflow) return fail(c, PPM_E_RANGE, "gather query buffer overflow");
   for (size_t p = 0; p < h.size(); ++p) {
@@ -1626,29 +1701,47 @@ void ppm_session_destroy(ppm_session* s) {
   for (Pipe& p : s->pipes) {
     // the streams are the context's (ctx_stream): waited for, not destroyed
     if (p.stream) (void)hipStreamSynchronize(p.stream);
-    if (p.s2) (void)hipStreamSynchronize(p.s2);
     pipe_drop_graph(p);
-    for (hipEvent_t e : {p.evf, p.evj, p.done})
-      if (e) (void)hipEventDestroy(e);
-    photons_free(p.pb);
-    map_free(p.map);
-    eye_free(p.eb);
-    dfree(p.sum);
-    dfree(p.sumsq);
-    dfree(p.st);
+    if (p.done) (void)hipEventDestroy(p.done);
+    dfree(p.mem);
   }
+  dfree(s->gimg);
+  dfree(s->grad);
   for (auto& e : s->ev)
     if (e) (void)hipEventDestroy(e);
   dfree(s->lights);
   delete s;
 }
 
-// Pipelines of a session: cfg.pipelines, else 2 when a pass is large enough
-// (at least 256k photons or 256k pixels) for two passes in flight to keep
-// the GPU busier than one, else 1.
-static uint32_t session_pipelines(const ppm_pass_cfg& cfg, uint64_t n_emit, uint64_t n_pix) {
-  if (cfg.pipelines) return std::min<uint32_t>(cfg.pipelines, 4);
-  return (n_emit >= (1u << 18) || n_pix >= (1u << 18)) ? 2u : 1u;
+// All buffers of one pass pipeline, in one allocation.
+static hipError_t pipe_alloc(ppm_ctx* c, Pipe& p, const DevCamera& cam, uint64_t n_emit, int max_depth,
+                             size_t* bytes) {
+  const uint64_t cap = photons_needed(n_emit, max_depth, c->n_cu);
+  return arena_alloc(c, &p.mem, [&](Arena& a) {
+    a.take(&p.st, 1);
+    a.take(&p.st_adj, 1);
+    eye_layout(a, p.eb, cam, max_depth, c->n_cu, &p.pb, cap, trace_waves(n_emit, c->n_cu));
+    map_layout(a, p.map, cap, c->n_cu, true);
+    const uint64_t n3 = 3ull * p.eb.n_pix;
+    a.take(&p.sum, 2 * n3);
+    p.sumsq = p.sum ? p.sum + n3 : nullptr;
+  }, bytes);
+}
+
+// Before the first pass: sums cleared, pass states as new with the photon
+// power, and (tiles) the tiles' query counts of earlier passes cleared.
+static hipError_t session_clear(ppm_session* s, bool tiles) {
+  PipesInit in;
+  in.n_pipes = (uint32_t)s->pipes.size();
+  in.n_sums = 6ull * s->pipes[0].eb.n_pix;
+  in.n_tiles = tiles ? s->pipes[0].eb.tiles_cap : 0u;
+  in.power = s->power;
+  for (uint32_t j = 0; j < in.n_pipes; ++j) {
+    in.sums[j] = s->pipes[j].sum;
+    in.tiles[j] = s->pipes[j].eb.tile_count;
+    in.st[j] = s->pipes[j].st;
+  }
+  return launch_pipes_init(s->ctx->stream, in);
 }
 
 // own_streams = false: a batch's session, whose passes the batch launches on
@@ -1676,50 +1769,56 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
     return fail(c, PPM_E_RANGE, "photons per pass must be in [1, 2^25] (the record's photon index)");
   }
   const uint64_t cap = photons_needed(total, cfg->max_depth, c->n_cu);
-  if (cap > 0x7FFFFFFFull) {
+  if (cap >= 0x7FFFFFFFull) {
     delete s;
-    return fail(c, PPM_E_RANGE, "n_photon * max_depth must stay below 2^31");
+    return fail(c, PPM_E_RANGE, "n_photon * max_depth must stay below 2^31 - 1");
   }
   s->sbuf = sc->buf;
   s->sbuf.n_emit_total = (uint32_t)total;
-  const uint64_t n_pix = (uint64_t)sc->buf.cam.xreso * (uint64_t)sc->buf.cam.yreso;
-  s->cfg.pipelines = session_pipelines(s->cfg, total, n_pix);
-  s->pipes.resize(s->cfg.pipelines);
+  // Automatic: MAX_PIPES pipelines, one per hardware queue.  A pass is a chain
+  // of kernels that rarely fill the GPU alone, and four passes in flight, each
+  // a plain chain on a queue of its own, beat one or two whose eye branch was
+  // forked beside the photon branch (ms per pass: 160x120 and 20k photons
+  // 0.35 -> 0.20, 256x256 and 200k 0.335 -> 0.154, caustic box 0.665 ->
+  // 0.637, 327k-triangle mesh 56 -> 53; three: 0.28, 0.18, 0.67, 69).  Fewer
+  // when the GPU's memory does not hold that many: at most half of what is
+  // free, except the first.
+  const bool automatic = cfg->pipelines == 0;
+  uint32_t want = automatic ? MAX_PIPES : cfg->pipelines;
   hipError_t e = hipSuccess;
-  do {
+  s->pipes.reserve(want);
+  size_t free0 = 0, total_mem = 0, per = 0;
+  if (automatic) (void)hipMemGetInfo(&free0, &total_mem);
+  for (uint32_t j = 0; j < want; ++j) {
+    if (automatic && j > 0 && (j + 1) * per > free0 / 2) break;
+    Pipe p;
+    e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, &per);
+    if (e == hipErrorOutOfMemory && automatic && j > 0) {
+      (void)hipGetLastError();
+      e = hipSuccess;
+      break;
+    }
+    if (e != hipSuccess) break;
+    photons_layout(p.pb, total, cfg->max_depth, c->n_cu);
+    s->pipes.push_back(p);
+  }
+  s->cfg.pipelines = (uint32_t)s->pipes.size();
+  if (e == hipSuccess) do {
     if ((e = dalloc(&s->lights, L.size())) != hipSuccess) break;
     if ((e = hipMemcpy(s->lights, L.data(), sizeof(DevLight) * L.size(), hipMemcpyHostToDevice)) != hipSuccess) break;
     s->sbuf.lights = s->lights;
-    for (Pipe& p : s->pipes) {
-      if ((e = photons_alloc(p.pb, cap, trace_waves(total, c->n_cu))) != hipSuccess) break;
-      photons_layout(p.pb, total, cfg->max_depth, c->n_cu);
-      if ((e = map_alloc(p.map, cap, c->n_cu, true)) != hipSuccess) break;
-      if ((e = eye_alloc(p.eb, sc->buf.cam, cfg->max_depth, c->n_cu)) != hipSuccess) break;
-      const uint64_t n3 = 3ull * p.eb.n_pix;
-      if ((e = dalloc(&p.sum, n3)) != hipSuccess) break;
-      if ((e = dalloc(&p.sumsq, n3)) != hipSuccess) break;
-      if ((e = hipMemset(p.sum, 0, sizeof(double) * n3)) != hipSuccess) break;
-      if ((e = hipMemset(p.sumsq, 0, sizeof(double) * n3)) != hipSuccess) break;
-      if ((e = dalloc(&p.st, 1)) != hipSuccess) break;
-      PassState h = host_state();
-      if ((e = hipMemcpy(p.st, &h, sizeof(h), hipMemcpyHostToDevice)) != hipSuccess) break;
-      // pipeline 0 runs on the context's stream: K pipelines then use 2K
-      // streams in all, which HIP spreads over that many hardware queues
-      // (GPU_MAX_HW_QUEUES, 4 by default) when K <= 2
-      const int j = (int)(&p - &s->pipes[0]);
-      if (j == 0 || !own_streams)
-        p.stream = c->stream;
-      else if ((e = ctx_stream(c, AUX_PIPE + j - 1, &p.stream)) != hipSuccess)
-        break;
-      if (!own_streams) continue;
-      if ((e = ctx_stream(c, AUX_EYE + j, &p.s2)) != hipSuccess) break;
-      if ((e = hipEventCreateWithFlags(&p.evf, hipEventDisableTiming)) != hipSuccess) break;
-      if ((e = hipEventCreateWithFlags(&p.evj, hipEventDisableTiming)) != hipSuccess) break;
-      if ((e = hipEventCreateWithFlags(&p.done, hipEventDisableTiming)) != hipSuccess) break;
+    s->lights_host = L;
+    for (size_t j = 0; j < s->pipes.size(); ++j) {
+      Pipe& p = s->pipes[j];
+      eye_tiles(p.eb, s->sbuf.cam, (uint32_t)sc->buf.cam.tile_shift);
+      p.stream = j == 0 || !own_streams ? c->stream : c->aux[AUX_PIPE + j - 1];
+      if (own_streams && (e = hipEventCreateWithFlags(&p.done, hipEventDisableTiming)) != hipSuccess) break;
     }
     if (e != hipSuccess) break;
     for (auto& ev : s->ev)
       if ((e = hipEventCreate(&ev)) != hipSuccess) break;
+    if (e != hipSuccess) break;
+    e = session_clear(s, true);
   } while (0);
   if (e != hipSuccess) {
     ppm_session_destroy(s);
@@ -1733,11 +1832,10 @@ ppm_status ppm_session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass_cf
   return session_create(c, sc, cfg, out, true);
 }
 
-// Enqueue the kernels of one pass of pipeline p on stream st.  The eye
-// branch (eye rays, query order) depends only on the pass state, so it runs
-// on p.s2 beside the photon branch (trace, grid build) and joins before the
-// gather; ev != nullptr (stage timing) runs every stage in order on st and
-// records its events.
+// Enqueue the kernels of one pass of pipeline j on stream st, one after the
+// other: the eye rays and the order of their queries, then the photons, their
+// grid, the gather and the sums.  ev != nullptr (stage timing) records its
+// events between the stages, the photons first.
 static hipError_t enqueue_pass(ppm_session* s, uint32_t j, hipStream_t st, hipEvent_t* ev) {
   const ppm_pass_cfg& cfg = s->cfg;
   const ppm_scene* sc = s->scene;
@@ -1747,42 +1845,31 @@ static hipError_t enqueue_pass(ppm_session* s, uint32_t j, hipStream_t st, hipEv
   const float4 bmax = make_float4((float)sc->bmax[0], (float)sc->bmax[1], (float)sc->bmax[2], 0.f);
   const int n_cu = s->ctx->n_cu;
   const uint32_t K = (uint32_t)s->pipes.size();
-  if (ev && (e = hipEventRecord(ev[0], st)) != hipSuccess) return e;
-  if ((e = launch_pass_begin(st, p.st, cfg.first_pass + j, cfg.radius0 * cfg.radius0, cfg.alpha, s->power, K)) !=
-      hipSuccess)
+  auto mark = [&](int k) { return ev ? hipEventRecord(ev[k], st) : hipSuccess; };
+  auto eye = [&] {
+    return launch_eye(st, s->sbuf, p.st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, n_cu);
+  };
+  auto order = [&] { return launch_query_prep(st, s->sbuf, p.map, p.st, p.eb); };
+  if ((e = mark(0)) != hipSuccess) return e;
+  if ((e = launch_pass_begin(st, p.st, cfg.first_pass + j, cfg.radius0 * cfg.radius0, cfg.alpha, K)) != hipSuccess)
     return e;
-  if (!ev) {
-    if ((e = hipEventRecord(p.evf, st)) != hipSuccess) return e;
-    if ((e = hipStreamWaitEvent(p.s2, p.evf, 0)) != hipSuccess) return e;
-    if ((e = launch_eye(p.s2, s->sbuf, p.st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, n_cu)) != hipSuccess)
-      return e;
-    if ((e = launch_query_prep(p.s2, s->sbuf, p.map, p.st, p.eb)) != hipSuccess) return e;
-    if ((e = hipEventRecord(p.evj, p.s2)) != hipSuccess) return e;
-  }
+  if (!ev && ((e = eye()) != hipSuccess || (e = order()) != hipSuccess)) return e;
   if ((e = launch_trace_photons(st, s->sbuf, p.st, p.pb, cfg.seed, cfg.use_classic, cfg.max_depth)) != hipSuccess)
     return e;
-  if (ev && (e = hipEventRecord(ev[1], st)) != hipSuccess) return e;
+  if ((e = mark(1)) != hipSuccess) return e;
   if ((e = launch_grid_build(st, p.map, p.st, p.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total)) != hipSuccess) return e;
-  if (ev && (e = hipEventRecord(ev[2], st)) != hipSuccess) return e;
-  if (ev) {
-    if ((e = launch_eye(st, s->sbuf, p.st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, n_cu)) != hipSuccess)
-      return e;
-    if ((e = hipEventRecord(ev[3], st)) != hipSuccess) return e;
-    if ((e = launch_query_prep(st, s->sbuf, p.map, p.st, p.eb)) != hipSuccess) return e;
-  } else if ((e = hipStreamWaitEvent(st, p.evj, 0)) != hipSuccess) {
-    return e;
-  }
+  if ((e = mark(2)) != hipSuccess) return e;
+  if (ev && ((e = eye()) != hipSuccess || (e = mark(3)) != hipSuccess || (e = order()) != hipSuccess)) return e;
   if ((e = launch_gather(st, s->sbuf, p.map, p.st, p.eb, cfg.pfilter, cfg.use_classic, n_cu, p.sum, p.sumsq,
                          ev ? ev + 4 : nullptr, true)) != hipSuccess)
     return e;
   if ((e = launch_pass_end(st, p.st)) != hipSuccess) return e;
-  if (ev && (e = hipEventRecord(ev[6], st)) != hipSuccess) return e;
-  return hipSuccess;
+  return mark(6);
 }
 
 // The pass graph of pipeline j, captured once.  A capture that fails
-// part-way leaves no graph behind, and the capture stream and the eye
-// stream forked into it are replaced by fresh ones.
+// part-way leaves no graph behind, and the capture stream is replaced by a
+// fresh one.
 static hipError_t pipe_graph(ppm_session* s, uint32_t j) {
   Pipe& p = s->pipes[j];
   if (p.exec) return hipSuccess;
@@ -1800,10 +1887,6 @@ static hipError_t pipe_graph(ppm_session* s, uint32_t j) {
   if (e != hipSuccess) {
     pipe_drop_graph(p);
     ctx_stream_renew(c, AUX_CAPTURE);
-    ctx_stream_renew(c, AUX_EYE + (int)j);
-    p.s2 = nullptr;
-    const hipError_t e4 = ctx_stream(c, AUX_EYE + (int)j, &p.s2);
-    (void)e4;  // a missing eye stream fails the next capture, not this report
   }
   return e;
 }
@@ -1830,8 +1913,8 @@ ppm_status ppm_session_run(ppm_session* s, uint32_t n_pass) {
     }
   } else {
     if (graph)
-      for (uint32_t j = 0; j < K; ++j) {
-        const hipError_t e = pipe_graph(s, j);
+      for (uint32_t i = 0; i < std::min(n_pass, K); ++i) {
+        const hipError_t e = pipe_graph(s, (s->passes_done + i) % K);
         if (e != hipSuccess) return fail(c, PPM_E_HIP, std::string("graph capture: ") + hipGetErrorString(e));
       }
     // every pipeline starts after the context stream's earlier work and the
@@ -1911,17 +1994,13 @@ ppm_status ppm_session_reset(ppm_session* s) {
   const uint64_t total = assign_photons(L, sc->total_flux, s->cfg.n_photon, &power);
   if (total != s->sbuf.n_emit_total) return fail(c, PPM_E_INVALID, "the scene's photon counts changed; create a new session");
   HIP_TRY(c, hipStreamSynchronize(c->stream));
-  HIP_TRY(c, hipMemcpy(s->lights, L.data(), sizeof(DevLight) * L.size(), hipMemcpyHostToDevice));
-  s->power = power;
-  const PassState h = host_state();
-  for (Pipe& p : s->pipes) {
-    const uint64_t n3 = 3ull * p.eb.n_pix;
-    HIP_TRY(c, hipMemset(p.sum, 0, sizeof(double) * n3));
-    HIP_TRY(c, hipMemset(p.sumsq, 0, sizeof(double) * n3));
-    HIP_TRY(c, hipMemcpy(p.st, &h, sizeof(h), hipMemcpyHostToDevice));
-    // the captured pass has the photon power as an argument: capture again
-    pipe_drop_graph(p);
+  if (L.size() != s->lights_host.size() || std::memcmp(L.data(), s->lights_host.data(), sizeof(DevLight) * L.size()) != 0) {
+    HIP_TRY(c, hipMemcpy(s->lights, L.data(), sizeof(DevLight) * L.size(), hipMemcpyHostToDevice));
+    s->lights_host = L;
   }
+  // the photon power goes with the pass states, so the captured passes stay
+  s->power = power;
+  HIP_TRY(c, session_clear(s, false));
   s->passes_done = 0;
   s->t = ppm_timings{};
   return PPM_OK;
@@ -1944,7 +2023,6 @@ static hipError_t session_set_tiles(ppm_session* s, uint32_t shift) {
   for (Pipe& p : s->pipes) {
     hipError_t e;
     if (p.stream && (e = hipStreamSynchronize(p.stream)) != hipSuccess) return e;
-    if (p.s2 && (e = hipStreamSynchronize(p.s2)) != hipSuccess) return e;
   }
   for (Pipe& p : s->pipes) {
     const hipError_t e = eye_set_tiles(p.eb, s->sbuf.cam, shift);
@@ -1969,8 +2047,7 @@ ppm_status ppm_session_backward(ppm_session* s, const double* grad_image, double
   if (K == 0) return fail(c, PPM_E_INVALID, "backward before any pass");
   const ppm_pass_cfg& cfg = s->cfg;
   const ppm_scene* sc = s->scene;
-  Pipe& p0 = s->pipes[0];
-  const uint32_t n_pix = p0.eb.n_pix;
+  const uint32_t n_pix = s->pipes[0].eb.n_pix;
   const uint32_t nm = s->sbuf.n_mats;
   // dL/d(pass image) = dL/d(mean image) / K
   std::vector<float4> g(n_pix);
@@ -1979,58 +2056,50 @@ ppm_status ppm_session_backward(ppm_session* s, const double* grad_image, double
     if (!finite3(v)) return fail(c, PPM_E_NONFINITE, "non-finite image gradient");
     g[p] = make_float4((float)(v[0] / K), (float)(v[1] / K), (float)(v[2] / K), 0.0f);
   }
-  float4* gimg = nullptr;
-  float *adj_sorted = nullptr, *adj_slot = nullptr;
-  double* grad = nullptr;
-  PassState* st = nullptr;
+  if (!s->gimg) HIP_TRY(c, dalloc(&s->gimg, n_pix));
+  if (!s->grad) HIP_TRY(c, dalloc(&s->grad, 3ull * nm));
+  HIP_TRY(c, hipMemcpy(s->gimg, g.data(), sizeof(float4) * n_pix, hipMemcpyHostToDevice));
+  HIP_TRY(c, hipMemset(s->grad, 0, sizeof(double) * 3 * nm));
   const float4 bmin = make_float4((float)sc->bmin[0], (float)sc->bmin[1], (float)sc->bmin[2], 0.f);
   const float4 bmax = make_float4((float)sc->bmax[0], (float)sc->bmax[1], (float)sc->bmax[2], 0.f);
-  hipStream_t q = c->stream;
-  hipError_t e;
-  if ((e = dalloc(&gimg, n_pix)) == hipSuccess && (e = dalloc(&adj_sorted, p0.map.cap)) == hipSuccess &&
-      (e = dalloc(&adj_slot, p0.pb.cap)) == hipSuccess && (e = dalloc(&grad, 3ull * nm)) == hipSuccess &&
-      (e = dalloc(&st, 1)) == hipSuccess &&
-      (e = hipMemcpy(gimg, g.data(), sizeof(float4) * n_pix, hipMemcpyHostToDevice)) == hipSuccess &&
-      (e = hipMemset(grad, 0, sizeof(double) * 3 * nm)) == hipSuccess) {
-    const PassState h = host_state();
-    e = hipMemcpy(st, &h, sizeof(h), hipMemcpyHostToDevice);
-    // replay the session's passes from their seeds (the passes' only
-    // checkpoint), each followed by its adjoint
-    for (uint32_t k = 0; k < K && e == hipSuccess; ++k) {
-      if ((e = launch_pass_begin(q, st, cfg.first_pass, cfg.radius0 * cfg.radius0, cfg.alpha, s->power)) != hipSuccess)
-        break;
-      // the eye branch beside the photon branch, as in a forward pass
-      if ((e = hipEventRecord(p0.evf, q)) != hipSuccess || (e = hipStreamWaitEvent(p0.s2, p0.evf, 0)) != hipSuccess)
-        break;
-      if ((e = launch_eye(p0.s2, s->sbuf, st, p0.eb, cfg.seed, cfg.use_classic, cfg.max_depth, c->n_cu)) !=
-          hipSuccess)
-        break;
-      if ((e = launch_query_prep(p0.s2, s->sbuf, p0.map, st, p0.eb)) != hipSuccess) break;
-      if ((e = hipEventRecord(p0.evj, p0.s2)) != hipSuccess) break;
-      if ((e = launch_trace_photons(q, s->sbuf, st, p0.pb, cfg.seed, cfg.use_classic, cfg.max_depth)) != hipSuccess)
-        break;
-      if ((e = launch_grid_build(q, p0.map, st, p0.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total)) != hipSuccess) break;
-      if ((e = hipStreamWaitEvent(q, p0.evj, 0)) != hipSuccess) break;
-      if ((e = launch_gather(q, s->sbuf, p0.map, st, p0.eb, cfg.pfilter, cfg.use_classic, c->n_cu, nullptr,
-                             nullptr, nullptr, true)) != hipSuccess)
-        break;
-      if ((e = launch_adjoint(q, s->sbuf, p0.map, st, p0.pb, p0.eb, cfg.pfilter, c->n_cu, cfg.seed,
-                              cfg.use_classic, cfg.max_depth, gimg, adj_sorted, adj_slot, grad)) != hipSuccess)
-        break;
-      e = launch_pass_end(q, st);
-    }
-    // an error may leave the eye branch running: drain it before the frees
-    const hipError_t e2 = hipStreamSynchronize(p0.s2);
+  PassState h = host_state();
+  h.power = s->power;
+  const uint32_t NP = std::min<uint32_t>(K, (uint32_t)s->pipes.size());
+  hipError_t e = hipSuccess;
+  for (uint32_t j = 0; j < NP && e == hipSuccess; ++j)
+    e = hipMemcpy(s->pipes[j].st_adj, &h, sizeof(h), hipMemcpyHostToDevice);
+  // replay the session's passes from their seeds (the passes' only
+  // checkpoint), each followed by its adjoint: pass k on pipeline k mod NP,
+  // NP passes in flight as in the forward run.  The pipelines' streams start
+  // after the copies above (done) and the context stream's earlier work (a
+  // session's calls return once theirs is done).
+  for (uint32_t k = 0; k < K && e == hipSuccess; ++k) {
+    const uint32_t j = k % NP;
+    Pipe& p = s->pipes[j];
+    hipStream_t q = p.stream;
+    PassState* st = p.st_adj;
+    // the adjoint's scratch: the photon sort's keys, done with by then
+    float* adj_sorted = reinterpret_cast<float*>(p.map.keys[0]);
+    float* adj_slot = reinterpret_cast<float*>(p.map.keys[1]);
+    if ((e = launch_pass_begin(q, st, cfg.first_pass + j, cfg.radius0 * cfg.radius0, cfg.alpha, NP)) != hipSuccess) break;
+    if ((e = launch_eye(q, s->sbuf, st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, c->n_cu)) != hipSuccess) break;
+    if ((e = launch_query_prep(q, s->sbuf, p.map, st, p.eb)) != hipSuccess) break;
+    if ((e = launch_trace_photons(q, s->sbuf, st, p.pb, cfg.seed, cfg.use_classic, cfg.max_depth)) != hipSuccess) break;
+    if ((e = launch_grid_build(q, p.map, st, p.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total)) != hipSuccess) break;
+    if ((e = launch_gather(q, s->sbuf, p.map, st, p.eb, cfg.pfilter, cfg.use_classic, c->n_cu, nullptr, nullptr,
+                           nullptr, true)) != hipSuccess)
+      break;
+    if ((e = launch_adjoint(q, s->sbuf, p.map, st, p.pb, p.eb, cfg.pfilter, c->n_cu, cfg.seed, cfg.use_classic,
+                            cfg.max_depth, s->gimg, adj_sorted, adj_slot, s->grad)) != hipSuccess)
+      break;
+    e = launch_pass_end(q, st);
+  }
+  for (uint32_t j = 0; j < NP; ++j) {  // also after an error: nothing keeps running on the buffers
+    const hipError_t e2 = hipStreamSynchronize(s->pipes[j].stream);
     if (e == hipSuccess) e = e2;
-    if (e == hipSuccess) e = hipStreamSynchronize(q);
   }
   std::vector<double> hg(3ull * nm, 0.0);
-  if (e == hipSuccess) e = hipMemcpy(hg.data(), grad, sizeof(double) * hg.size(), hipMemcpyDeviceToHost);
-  dfree(gimg);
-  dfree(adj_sorted);
-  dfree(adj_slot);
-  dfree(grad);
-  dfree(st);
+  if (e == hipSuccess && !hg.empty()) e = hipMemcpy(hg.data(), s->grad, sizeof(double) * hg.size(), hipMemcpyDeviceToHost);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
   for (size_t i = 0; i < hg.size(); ++i) grad_albedo[i] = hg[i];
   if (grad_light) {
@@ -2167,7 +2236,6 @@ hipError_t batch_layout(ppm_batch* b) {
     it.seed = s->cfg.seed;
     it.r2_first = s->cfg.radius0 * s->cfg.radius0;
     it.alpha = s->cfg.alpha;
-    it.power = s->power;
     it.mscale = morton_scale(s->sbuf.bmin, s->sbuf.bmax, QUERY_MORTON_MAX);
     it.first_pass = s->cfg.first_pass;
     it.pass_stride = b->K;
@@ -2238,32 +2306,24 @@ hipError_t batch_round(ppm_batch* b, uint32_t act, uint32_t q) {
   if (!b->exec[gi]) {
     uint32_t blocks[BK_KINDS];
     for (int k = 0; k < BK_KINDS; ++k) blocks[k] = b->htab[(size_t)k * (n + 1) + act];
-    // captured on the context's capture streams; the fork/join events live
-    // only while the graph is captured.  A capture that fails part-way
-    // leaves no graph behind and replaces both capture streams.
-    hipStream_t cap = nullptr, cap2 = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
+    // captured on the context's capture stream.  A capture that fails
+    // part-way leaves no graph behind and replaces that stream.
+    hipStream_t cap = nullptr;
     hipError_t e = ctx_stream(b->ctx, AUX_CAPTURE, &cap);
-    if (e == hipSuccess) e = ctx_stream(b->ctx, AUX_CAPTURE2, &cap2);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
     if (e == hipSuccess) e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
       const hipError_t e2 =
-          launch_batch_pass(cap, cap2, fork, join, b->items + (size_t)q * n, b->tab, blocks, act, n, b->bvh, b->dyn);
+          launch_batch_pass(cap, b->items + (size_t)q * n, b->tab, blocks, act, n, b->bvh, b->dyn);
       const hipError_t e3 = hipStreamEndCapture(cap, &b->graph[gi]);
       e = e2 != hipSuccess ? e2 : e3;
     }
     if (e == hipSuccess) e = hipGraphInstantiate(&b->exec[gi], b->graph[gi], nullptr, nullptr, 0);
-    if (join) (void)hipEventDestroy(join);
-    if (fork) (void)hipEventDestroy(fork);
     if (e != hipSuccess) {
       if (b->exec[gi]) (void)hipGraphExecDestroy(b->exec[gi]);
       if (b->graph[gi]) (void)hipGraphDestroy(b->graph[gi]);
       b->exec[gi] = nullptr;
       b->graph[gi] = nullptr;
       ctx_stream_renew(b->ctx, AUX_CAPTURE);
-      ctx_stream_renew(b->ctx, AUX_CAPTURE2);
       return e;
     }
   }
@@ -2272,15 +2332,9 @@ hipError_t batch_round(ppm_batch* b, uint32_t act, uint32_t q) {
 
 // Every scene back to before its first pass.
 hipError_t batch_reset(ppm_batch* b) {
-  const PassState h = host_state();
   for (ppm_session* s : b->sess) {
-    for (Pipe& p : s->pipes) {
-      const uint64_t n3 = 3ull * p.eb.n_pix;
-      hipError_t e;
-      if ((e = hipMemsetAsync(p.sum, 0, sizeof(double) * n3, b->ctx->stream)) != hipSuccess) return e;
-      if ((e = hipMemsetAsync(p.sumsq, 0, sizeof(double) * n3, b->ctx->stream)) != hipSuccess) return e;
-      if ((e = hipMemcpyAsync(p.st, &h, sizeof(h), hipMemcpyHostToDevice, b->ctx->stream)) != hipSuccess) return e;
-    }
+    const hipError_t e = session_clear(s, false);
+    if (e != hipSuccess) return e;
     s->passes_done = 0;
   }
   b->rounds_done = 0;
@@ -2350,8 +2404,8 @@ ppm_status ppm_batch_create(ppm_ctx* c, uint32_t n, const ppm_scene* const* scen
   b->ps[0] = c->stream;
   e = hipSuccess;
   for (uint32_t q = 1; q < b->K && e == hipSuccess; ++q) {
-    e = ctx_stream(c, AUX_PIPE + (int)q - 1, &b->ps[q]);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&b->pdone[q], hipEventDisableTiming);
+    b->ps[q] = c->aux[AUX_PIPE + (int)q - 1];
+    e = hipEventCreateWithFlags(&b->pdone[q], hipEventDisableTiming);
   }
   if (e != hipSuccess || (e = dalloc(&b->items, (uint64_t)b->K * n)) != hipSuccess ||
       (e = dalloc(&b->tab, (uint64_t)BK_KINDS * (n + 1))) != hipSuccess ||

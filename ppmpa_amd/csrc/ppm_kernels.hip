@@ -62,19 +62,18 @@ __host__ __device__ inline SceneView make_view(const SceneBuf& b) {
 // steps through the passes in between, so r2 of every pass is the same FP64
 // product as in a single pipeline.
 __device__ __forceinline__ void k_pass_begin_body(PassState* st, uint32_t first_pass, double r2_first, double alpha,
-                                                  double power, uint32_t stride, Blk blk) {
+                                                  uint32_t stride, Blk blk) {
   if (blk.b != 0) return;
   if (threadIdx.x < 16) st->work[threadIdx.x >> 3][threadIdx.x & 7u][0] = 0;
   if (threadIdx.x != 0) return;
   uint32_t pass = st->pass;
-  double a = st->alpha, r2 = st->r2, pw = st->power;
+  double a = st->alpha, r2 = st->r2;
+  const double pw = st->power;
   if (pass == 0) {
     pass = first_pass;
     a = alpha;
-    pw = power;
     st->alpha = alpha;
     st->r2_first = r2_first;
-    st->power = power;
     r2 = r2_first;
     for (uint32_t k = 1; k < first_pass; ++k) r2 *= ((double)k + alpha) / ((double)k + 1.0);
   } else {
@@ -95,9 +94,8 @@ __device__ __forceinline__ void k_pass_begin_body(PassState* st, uint32_t first_
   st->tiles_back = 0;
 }
 
-__global__ void k_pass_begin(PassState* st, uint32_t first_pass, double r2_first, double alpha, double power,
-                             uint32_t stride) {
-  k_pass_begin_body(st, first_pass, r2_first, alpha, power, stride, Blk{blockIdx.x, gridDim.x});
+__global__ void k_pass_begin(PassState* st, uint32_t first_pass, double r2_first, double alpha, uint32_t stride) {
+  k_pass_begin_body(st, first_pass, r2_first, alpha, stride, Blk{blockIdx.x, gridDim.x});
 }
 
 __device__ __forceinline__ void k_pass_end_body(PassState* st, Blk blk) {
@@ -110,9 +108,30 @@ __global__ void k_pass_end(PassState* st) {
   k_pass_end_body(st, Blk{blockIdx.x, gridDim.x});
 }
 
+// One launch for a session's pipelines (block row blockIdx.y = pipeline).
+__global__ __launch_bounds__(256) void k_pipes_init(PipesInit in) {
+  const uint32_t j = blockIdx.y, stride = gridDim.x * blockDim.x;
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint64_t i = t; i < in.n_sums; i += stride) in.sums[j][i] = 0.0;
+  for (uint32_t i = t; i < in.n_tiles; i += stride) in.tiles[j][i] = 0u;
+  if (blockIdx.x == 0) {
+    uint32_t* w = reinterpret_cast<uint32_t*>(in.st[j]);
+    for (uint32_t i = threadIdx.x; i < sizeof(PassState) / 4u; i += blockDim.x) w[i] = 0u;
+    __syncthreads();
+    if (threadIdx.x == 0) in.st[j]->power = in.power;
+  }
+}
+
+hipError_t launch_pipes_init(hipStream_t s, const PipesInit& in) {
+  if (in.n_pipes == 0 || in.n_pipes > MAX_PIPES) return hipErrorInvalidValue;
+  const uint32_t blocks = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(1, (in.n_sums + 1023) / 1024));
+  hipLaunchKernelGGL(k_pipes_init, dim3(blocks, in.n_pipes), dim3(256), 0, s, in);
+  return hipGetLastError();
+}
+
 hipError_t launch_pass_begin(hipStream_t s, PassState* st, uint32_t first_pass, double r2_first, double alpha,
-                             double power, uint32_t stride) {
-  hipLaunchKernelGGL(k_pass_begin, dim3(1), dim3(64), 0, s, st, first_pass, r2_first, alpha, power, stride);
+                             uint32_t stride) {
+  hipLaunchKernelGGL(k_pass_begin, dim3(1), dim3(64), 0, s, st, first_pass, r2_first, alpha, stride);
   return hipGetLastError();
 }
 hipError_t launch_pass_end(hipStream_t s, PassState* st) {
@@ -2950,7 +2969,7 @@ __device__ __forceinline__ BatchItem load_item(const BatchItem* items, uint32_t 
 __global__ void kb_pass_begin(const BatchItem* items, uint32_t n) {
   if (blockIdx.x >= n) return;
   const BatchItem it = load_item(items, blockIdx.x);
-  k_pass_begin_body(it.st, it.first_pass, it.r2_first, it.alpha, it.power, it.pass_stride, Blk{0u, 1u});
+  k_pass_begin_body(it.st, it.first_pass, it.r2_first, it.alpha, it.pass_stride, Blk{0u, 1u});
 }
 
 __global__ void kb_pass_end(const BatchItem* items, uint32_t n) {
@@ -3099,36 +3118,31 @@ __global__ __launch_bounds__(256) void kb_accumulate(const BatchItem* items, con
 
 #undef BATCH_PROLOGUE
 
-hipError_t launch_batch_pass(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent_t join,
-                             const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
+hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
                              uint32_t n_all, bool bvh, uint32_t dyn) {
-  // blocks[k] = total blocks of kind k over the first n scenes.  The eye
-  // branch (tile order, eye trace, query sort) runs on s2 beside the photon
-  // branch (trace, grid build): the two touch disjoint buffers and counters.
+  // blocks[k] = total blocks of kind k over the first n scenes.  One chain of
+  // launches: the rounds of the other pipelines run beside it.
   const dim3 T256(256), T1024(1024), T64(64), TOS(OS_THREADS);
   hipError_t e;
   hipLaunchKernelGGL(kb_pass_begin, dim3(n), T64, 0, s, items, n);
-  if ((e = hipEventRecord(fork, s)) != hipSuccess) return e;
-  if ((e = hipStreamWaitEvent(s2, fork, 0)) != hipSuccess) return e;
-  hipLaunchKernelGGL(kb_tile_order, dim3(blocks[BK_PIX]), T256, 0, s2, items, tab, n, n_all);
+  hipLaunchKernelGGL(kb_tile_order, dim3(blocks[BK_PIX]), T256, 0, s, items, tab, n, n_all);
   switch ((bvh ? (dyn != 0u ? 2 : 1) : 0)) {
     case 2:
-      hipLaunchKernelGGL(kb_eye<2>, dim3(blocks[BK_EYE]), T256, dyn, s2, items, tab, n, n_all);
+      hipLaunchKernelGGL(kb_eye<2>, dim3(blocks[BK_EYE]), T256, dyn, s, items, tab, n, n_all);
       break;
     case 1:
-      hipLaunchKernelGGL(kb_eye<1>, dim3(blocks[BK_EYE]), T256, 0, s2, items, tab, n, n_all);
+      hipLaunchKernelGGL(kb_eye<1>, dim3(blocks[BK_EYE]), T256, 0, s, items, tab, n, n_all);
       break;
     default:
-      hipLaunchKernelGGL(kb_eye<0>, dim3(blocks[BK_EYE]), T256, 0, s2, items, tab, n, n_all);
+      hipLaunchKernelGGL(kb_eye<0>, dim3(blocks[BK_EYE]), T256, 0, s, items, tab, n, n_all);
   }
-  hipLaunchKernelGGL(kb_tile_count, dim3(blocks[BK_PIX]), T256, 0, s2, items, tab, n, n_all);
-  hipLaunchKernelGGL(kb_scan_tiles, dim3(n), T1024, 0, s2, items, n);
-  hipLaunchKernelGGL(kb_query_keys, dim3(blocks[BK_QKEYS]), T256, 0, s2, items, tab, n, n_all);
-  hipLaunchKernelGGL(kb_os_hist, dim3(blocks[BK_QHIST]), T1024, 0, s2, items, tab, n, n_all, 1);
+  hipLaunchKernelGGL(kb_tile_count, dim3(blocks[BK_PIX]), T256, 0, s, items, tab, n, n_all);
+  hipLaunchKernelGGL(kb_scan_tiles, dim3(n), T1024, 0, s, items, n);
+  hipLaunchKernelGGL(kb_query_keys, dim3(blocks[BK_QKEYS]), T256, 0, s, items, tab, n, n_all);
+  hipLaunchKernelGGL(kb_os_hist, dim3(blocks[BK_QHIST]), T1024, 0, s, items, tab, n, n_all, 1);
   for (uint32_t p = 0; p < QUERY_KEY_BITS / 8u; ++p)
-    hipLaunchKernelGGL(kb_os_scatter<false>, dim3(blocks[BK_QOS]), TOS, 0, s2, items, tab, n, n_all, 1, p);
+    hipLaunchKernelGGL(kb_os_scatter<false>, dim3(blocks[BK_QOS]), TOS, 0, s, items, tab, n, n_all, 1, p);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = hipEventRecord(join, s2)) != hipSuccess) return e;
   switch ((bvh ? (dyn != 0u ? 2 : 1) : 0)) {
     case 2:
       hipLaunchKernelGGL(kb_trace<2>, dim3(blocks[BK_TRACE]), T256, dyn, s, items, tab, n, n_all);
@@ -3151,7 +3165,6 @@ hipError_t launch_batch_pass(hipStream_t s, hipStream_t s2, hipEvent_t fork, hip
   hipLaunchKernelGGL(kb_grid_clear, dim3(blocks[BK_CLEAR]), T256, 0, s, items, tab, n, n_all);
   hipLaunchKernelGGL(kb_grid_cells, dim3(blocks[BK_LEAVES]), T256, 0, s, items, tab, n, n_all);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = hipStreamWaitEvent(s, join, 0)) != hipSuccess) return e;
   switch ((bvh ? (dyn != 0u ? 2 : 1) : 0)) {
     case 2:
       hipLaunchKernelGGL(kb_shade<2>, dim3(blocks[BK_SHADE]), T256, dyn, s, items, tab, n, n_all);

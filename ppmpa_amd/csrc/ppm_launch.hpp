@@ -150,10 +150,26 @@ constexpr uint32_t EYE_WAVES_PER_CU = 6;
 constexpr uint32_t SHADE_BLOCKS_PER_CU = 5;
 constexpr uint32_t TRACE_WAVES_PER_CU = 8;
 
+// Pass pipelines of a session or batch at most.
+constexpr uint32_t MAX_PIPES = 4;
+
+// Pipelines back to before their first pass: each one's n_sums FP64 sums and
+// its n_tiles tile counts cleared, its state zeroed but for the photon power.
+struct PipesInit {
+  double* sums[MAX_PIPES] = {};
+  uint32_t* tiles[MAX_PIPES] = {};
+  PassState* st[MAX_PIPES] = {};
+  uint64_t n_sums = 0;
+  uint32_t n_tiles = 0, n_pipes = 0;
+  double power = 0.0;
+};
+hipError_t launch_pipes_init(hipStream_t s, const PipesInit& in);
+
 // Next pass of the state (the first one: first_pass); a state that runs
 // every stride-th pass advances by stride.
+// The photon power is in the state already.
 hipError_t launch_pass_begin(hipStream_t s, PassState* st, uint32_t first_pass, double r2_first, double alpha,
-                             double power, uint32_t stride = 1);
+                             uint32_t stride);
 hipError_t launch_pass_end(hipStream_t s, PassState* st);
 
 // Number of tracing waves (= photon regions) used for n photons.
@@ -284,7 +300,6 @@ hipError_t launch_bvh_build(hipStream_t s, const DevShape* shapes, const uint32_
 // 3 per pixel: to mean and var (either may be null; host memory the GPU can
 // write), and the OR of the pipelines' overflow and nonfinite words to
 // flags[0..1].
-constexpr uint32_t MAX_PIPES = 4;
 struct ImageSrc {
   const double* sum[MAX_PIPES] = {};
   const double* sumsq[MAX_PIPES] = {};
@@ -304,7 +319,7 @@ struct BatchItem {
   double* sum;
   double* sumsq;
   uint64_t seed;
-  double r2_first, alpha, power;
+  double r2_first, alpha;
   float4 mscale;             // Morton scale of the scene bounds (QUERY_MORTON_MAX + 1 cells per axis)
   uint32_t first_pass;       // this pipeline's first pass
   uint32_t pass_stride;      // passes between two of this pipeline's (the batch's pipelines)
@@ -344,8 +359,7 @@ hipError_t launch_adjoint(hipStream_t s, const SceneBuf& sc, const MapBuf& m, Pa
 
 // One pass of the first n scenes of a batch (scenes sorted by pass count,
 // so the scenes still running are a prefix); blocks[k] = tab[k*(n_all+1)+n].
-hipError_t launch_batch_pass(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent_t join,
-                             const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
+hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
                              uint32_t n_all, bool bvh, uint32_t dyn);  // dyn: the BVH kernels' dynamic LDS
 
 // Test hook: nearest hit of n rays (unit directions).
