@@ -673,6 +673,50 @@ static hipError_t upload_lin_boxes(SceneBuf& b, const std::vector<DevShape>& lin
   return e;
 }
 
+// The list as rays test it (LinRec).
+static LinRec lin_rec(const DevShape& s) {
+  LinRec r;
+  std::memset(&r, 0, sizeof(r));
+  uint32_t kind = LIN_FULL;
+  r.a = s.p;
+  auto axis = [](const float4& v) {  // the only nonzero component, or -1
+    const float c[3] = {v.x, v.y, v.z};
+    int at = -1;
+    for (int k = 0; k < 3; ++k)
+      if (c[k] != 0.0f) at = at < 0 ? k : 3;
+    return at == 3 ? -1 : at;
+  };
+  if (s.kind == SHAPE_POINT) {
+    kind = LIN_NONE;
+  } else if (s.kind == SHAPE_SPHERE) {
+    kind = LIN_SPHERE;
+    r.b.x = s.radius * s.radius;
+  } else if (s.kind == SHAPE_PLAIN) {
+    kind = LIN_PLAIN;
+    r.a = s.n;
+    r.b.x = s.dist;
+  } else if (s.kind == SHAPE_PARALLELOGRAM) {
+    const int i = axis(s.d1), j = axis(s.d2);
+    if (i >= 0 && j >= 0 && i != j) {
+      const float d1[3] = {s.d1.x, s.d1.y, s.d1.z}, d2[3] = {s.d2.x, s.d2.y, s.d2.z};
+      kind = LIN_RECT + (uint32_t)(2 * i + (j > i ? j - 1 : j));
+      r.b.x = d1[i];
+      r.b.y = d2[j];
+    }
+  }
+  std::memcpy(&r.a.w, &kind, sizeof(kind));
+  r.b.w = s.p.w;
+  return r;
+}
+static hipError_t upload_lin_recs(SceneBuf& b, const std::vector<DevShape>& lin) {
+  std::vector<LinRec> recs(std::max<size_t>(lin.size(), 1));
+  std::memset(recs.data(), 0, recs.size() * sizeof(LinRec));
+  for (size_t i = 0; i < lin.size(); ++i) recs[i] = lin_rec(lin[i]);
+  hipError_t e = dalloc(&b.lin_rec, recs.size());
+  if (e == hipSuccess) e = hipMemcpy(b.lin_rec, recs.data(), recs.size() * sizeof(LinRec), hipMemcpyHostToDevice);
+  return e;
+}
+
 // Shapes tested one by one and, when the scene asks for one (or has at least
 // BVH_MIN_PRIMS bounded shapes in automatic mode), the device-built BVH over
 // the bounded shapes whose box sides are all within a quarter of the scene's
@@ -681,7 +725,8 @@ static hipError_t upload_lin_boxes(SceneBuf& b, const std::vector<DevShape>& lin
 static ppm_status scene_layout(ppm_ctx* c, ppm_scene* sc, const std::vector<DevShape>& shapes, int flags) {
   const ppm_status r = scene_layout_bvh(c, sc, shapes, flags);
   if (r != PPM_OK) return r;
-  const hipError_t e = upload_lin_boxes(sc->buf, sc->lin_host);
+  hipError_t e = upload_lin_boxes(sc->buf, sc->lin_host);
+  if (e == hipSuccess) e = upload_lin_recs(sc->buf, sc->lin_host);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
   return PPM_OK;
 }
@@ -1014,6 +1059,7 @@ void ppm_scene_destroy(ppm_scene* sc) {
   dfree(sc->buf.bvh);
   dfree(sc->buf.bprims);
   dfree(sc->buf.lin_box);
+  dfree(sc->buf.lin_rec);
   delete sc;
 }
 

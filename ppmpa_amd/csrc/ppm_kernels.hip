@@ -35,6 +35,7 @@ __host__ __device__ inline SceneView make_view(const SceneBuf& b) {
   v.mats = b.mats;
   v.lights = b.lights;
   v.lin = b.lin;
+  v.lin_rec = b.lin_rec;
   v.lin_box = b.lin_box;
   v.bvh = b.bvh;
   v.bprims = b.bprims;

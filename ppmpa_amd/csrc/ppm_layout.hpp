@@ -72,6 +72,21 @@ struct alignas(16) DevShape {
   float4 d2;
 };
 
+// What a ray's test of a shape of the list (SceneBuf::lin) needs, in list
+// order: a = (x, y, z, kind bits), b = (s0, s1, 0, scene index bits).
+//   LIN_RECT + k  a parallelogram with axis-aligned sides s0 along axis i and
+//                 s1 along axis j at corner a, (i, j) = (x,y) (x,z) (y,x) (y,z)
+//                 (z,x) (z,y) for k = 0..5
+//   LIN_SPHERE    centre a, s0 = radius^2
+//   LIN_PLAIN     normal a, s0 = dist
+//   LIN_FULL      any other shape: tested from its full record
+//   LIN_NONE      a point (never hit)
+enum : uint32_t { LIN_RECT = 0, LIN_SPHERE = 6, LIN_PLAIN = 7, LIN_FULL = 8, LIN_NONE = 9 };
+struct alignas(16) LinRec {
+  float4 a;
+  float4 b;
+};
+
 struct alignas(16) DevMaterial {
   uint32_t surface;
   float diff;         // diffuseness / scatterness
