@@ -1196,6 +1196,41 @@ __device__ __forceinline__ V3 tss_point(const SceneView& sc, uint32_t li, int s)
   return mk(t.x, t.y, t.z);
 }
 
+// What the shadow rays from p to light L share: the candidates, which of
+// them still have to be tested (shadow_need), and their unions over the wave.
+struct LightSetup {
+  uint64_t cand, need_o, need_s, wu_o, wu_s;
+  LightSelf self;
+};
+__device__ __forceinline__ LightSetup light_setup(const SceneView& sc, const DevLight& L, V3 p) {
+  LightSetup u;
+  u.cand = occluder_candidates(sc, L, p);
+  u.self.self = __float_as_uint(L.pos.w);
+  u.self.nq = cross(mk(L.d1), mk(L.d2));
+  u.self.nqn = sqrtf(dot(u.self.nq, u.self.nq));
+  // the union of the candidates of the wave's active lanes (one ballot per
+  // shape): the 25 samples then loop over these shapes only, instead of
+  // every shape with a per-lane test (caustic shade 0.75 -> 0.64 ms)
+  uint64_t wunion = 0;
+  const uint32_t nb = min(sc.n_lin, CAND_BITS);
+  for (uint32_t i = 0; i < nb; ++i)
+    if (__ballot(((u.cand >> i) & 1ull) != 0)) wunion |= 1ull << i;
+  shadow_need(sc, L, p, u.cand, wunion, u.self.self, u.need_o, u.need_s);
+  u.wu_o = u.wu_s = 0;
+  for (uint64_t w = wunion; w != 0; w &= w - 1) {
+    const uint32_t i = (uint32_t)__builtin_ctzll(w);
+    if (__ballot(((u.need_o >> i) & 1ull) != 0)) u.wu_o |= 1ull << i;
+    if (__ballot(((u.need_s >> i) & 1ull) != 0)) u.wu_s |= 1ull << i;
+  }
+  return u;
+}
+
+template <int BV, bool BVH = (BV != 0)>
+__device__ __forceinline__ bool sample_lit(const SceneView& sc, V3 p, V3 n, V3 ld, const LightSetup& u, uint32_t& occ,
+                                           float& cos0sq, float& sqd) {
+  return sample_lit<BV>(sc, p, n, ld, u.cand, u.need_o, u.need_s, u.wu_o, u.wu_s, u.self, occ, cos0sq, sqd);
+}
+
 template <int BV, bool BVH = (BV != 0)>
 __device__ C3 direct_light(const SceneView& sc, V3 p, V3 n) {
   C3 sum{0.0f, 0.0f, 0.0f};
@@ -1203,35 +1238,65 @@ __device__ C3 direct_light(const SceneView& sc, V3 p, V3 n) {
     const DevLight L = ldc(sc.lights, li);
     if (L.kind != LIGHT_PARALLELOGRAM) continue;
     const V3 ln = mk(L.nvec);
-    const uint64_t cand = occluder_candidates(sc, L, p);
-    LightSelf ls;
-    ls.self = __float_as_uint(L.pos.w);
-    ls.nq = cross(mk(L.d1), mk(L.d2));
-    ls.nqn = sqrtf(dot(ls.nq, ls.nq));
-    // the union of the candidates of the wave's active lanes (one ballot per
-    // shape): the 25 samples then loop over these shapes only, instead of
-    // every shape with a per-lane test (caustic shade 0.75 -> 0.64 ms)
-    uint64_t wunion = 0;
-    const uint32_t nb = min(sc.n_lin, CAND_BITS);
-    for (uint32_t i = 0; i < nb; ++i)
-      if (__ballot(((cand >> i) & 1ull) != 0)) wunion |= 1ull << i;
-    uint64_t need_o, need_s;
-    shadow_need(sc, L, p, cand, wunion, ls.self, need_o, need_s);
-    uint64_t wu_o = 0, wu_s = 0;
-    for (uint64_t w = wunion; w != 0; w &= w - 1) {
-      const uint32_t i = (uint32_t)__builtin_ctzll(w);
-      if (__ballot(((need_o >> i) & 1ull) != 0)) wu_o |= 1ull << i;
-      if (__ballot(((need_s >> i) & 1ull) != 0)) wu_s |= 1ull << i;
-    }
+    const LightSetup u = light_setup(sc, L, p);
     C3 prev{0.0f, 0.0f, 0.0f};
     uint32_t occ = ~0u;  // the BVH primitive that shadowed the last sample
     for (int s = 0; s < 25; ++s) {
       const V3 ld = tss_point(sc, li, s) - p;
       if (!(dot(ln, ld) < 0.0f)) continue;  // light.rs:129-131
       float csq, sqd;
-      if (!sample_lit<BV>(sc, p, n, ld, cand, need_o, need_s, wu_o, wu_s, ls, occ, csq, sqd)) continue;
+      if (!sample_lit<BV>(sc, p, n, ld, u, occ, csq, sqd)) continue;
       sum = sum + prev * csq;
       prev = light_radiance(L, sqd);
+    }
+  }
+  return sum;
+}
+
+// --- four lanes per query ------------------------------------------------------
+// A quad (lanes 4 q .. 4 q + 3) works on one query, all four lanes with the
+// same control flow: each takes every fourth item, and the items' terms are
+// then added in their order by all four, so the sums are those of one lane.
+template <int K>
+__device__ __forceinline__ float quad_get(float v) {  // lane K's value of the quad
+  const int x = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(x, x, K * 0x55, 0xF, 0xF, true));
+}
+
+// One step of the ordered sum of direct_light over the quad's four samples.
+template <int K>
+__device__ __forceinline__ void quad_light(float lit, float csq, C3 rad, C3& prev, C3& sum) {
+  const bool l = quad_get<K>(lit) != 0.0f;
+  const C3 t = sum + prev * quad_get<K>(csq);
+  sum = C3{l ? t.r : sum.r, l ? t.g : sum.g, l ? t.b : sum.b};
+  const C3 r{quad_get<K>(rad.r), quad_get<K>(rad.g), quad_get<K>(rad.b)};
+  prev = C3{l ? r.r : prev.r, l ? r.g : prev.g, l ? r.b : prev.b};
+}
+
+// Σ over the lights of the direct term, as direct_light, the 25 samples of a
+// light spread over the quad.
+template <int BV, bool BVH = (BV != 0)>
+__device__ C3 direct_light_quad(const SceneView& sc, V3 p, V3 n) {
+  C3 sum{0.0f, 0.0f, 0.0f};
+  const uint32_t sub = __lane_id() & 3u;
+  for (uint32_t li = 0; li < sc.n_lights; ++li) {
+    const DevLight L = ldc(sc.lights, li);
+    if (L.kind != LIGHT_PARALLELOGRAM) continue;
+    const LightSetup ls = light_setup(sc, L, p);
+    C3 prev{0.0f, 0.0f, 0.0f};
+    uint32_t occ = ~0u;  // the BVH primitive that shadowed the lane's last sample
+    for (uint32_t s0 = 0; s0 < 25u; s0 += 4u) {
+      const uint32_t s = s0 + sub;
+      float lit = 0.0f, csq = 0.0f, sqd = 1.0f;
+      if (s < 25u) {
+        const V3 ld = mk(sc.lights[li].tss[s]) - p;
+        if (dot(mk(L.nvec), ld) < 0.0f && sample_lit<BV>(sc, p, n, ld, ls, occ, csq, sqd)) lit = 1.0f;
+      }
+      const C3 rad = light_radiance(L, sqd);
+      quad_light<0>(lit, csq, rad, prev, sum);
+      quad_light<1>(lit, csq, rad, prev, sum);
+      quad_light<2>(lit, csq, rad, prev, sum);
+      quad_light<3>(lit, csq, rad, prev, sum);
     }
   }
   return sum;

@@ -1447,62 +1447,11 @@ hipError_t launch_grid_build(hipStream_t s, MapBuf& m, PassState* st, const Phot
   return hipGetLastError();
 }
 
-// Every photon of the pass's grid within the ball (q, r2): on_photon(j, pm,
-// dm, d2) for each sorted index j with dist2_nc(q, p_j) <= r2, each once.
-// Buckets are visited in cell order (x fastest, then y, then z), photons in
-// sorted order within a bucket, so a query's sum is formed in a fixed order.
-// Per lane: no cross-lane operations, so inactive lanes may skip it.
-template <typename OnPhoton>
-__device__ __forceinline__ void grid_range_scan(const PhotonRec* ph, uint2 se, float qx, float qy, float qz, float r2,
-                                                OnPhoton& on_photon) {
-  uint32_t j = se.x;
-  // four whole records per step: their loads are in flight together
-  for (; j + 3 < se.y; j += 4) {
-    const PhotonRec p0 = ph[j], p1 = ph[j + 1], p2 = ph[j + 2], p3 = ph[j + 3];
-    const float d0 = dist2_nc(qx, qy, qz, p0.pm.x, p0.pm.y, p0.pm.z);
-    const float d1 = dist2_nc(qx, qy, qz, p1.pm.x, p1.pm.y, p1.pm.z);
-    const float d2 = dist2_nc(qx, qy, qz, p2.pm.x, p2.pm.y, p2.pm.z);
-    const float d3 = dist2_nc(qx, qy, qz, p3.pm.x, p3.pm.y, p3.pm.z);
-    if (d0 <= r2) on_photon(j, p0.pm, p0.dm, d0);
-    if (d1 <= r2) on_photon(j + 1, p1.pm, p1.dm, d1);
-    if (d2 <= r2) on_photon(j + 2, p2.pm, p2.dm, d2);
-    if (d3 <= r2) on_photon(j + 3, p3.pm, p3.dm, d3);
-  }
-  for (; j < se.y; ++j) {
-    const PhotonRec p0 = ph[j];
-    const float d0 = dist2_nc(qx, qy, qz, p0.pm.x, p0.pm.y, p0.pm.z);
-    if (d0 <= r2) on_photon(j, p0.pm, p0.dm, d0);
-  }
-}
-
-// The same scan calling on_photon(j, pm, dm, d2, inside, valid) for every
-// photon of the range, inside = (d2 <= r2), valid = true (the walk below also
-// calls it for slots past a range's end, with both false): for a callback
-// whose work is a select
-// (the shade's sum adds 0 for photons outside), with no branch per photon
-// and so none of the exec-mask work that kept the scalar units half busy.
-template <typename OnPhoton>
-__device__ __forceinline__ void grid_range_scan_all(const PhotonRec* ph, uint2 se, float qx, float qy, float qz,
-                                                    float r2, OnPhoton& on_photon) {
-  uint32_t j = se.x;
-  for (; j + 3 < se.y; j += 4) {
-    const PhotonRec p0 = ph[j], p1 = ph[j + 1], p2 = ph[j + 2], p3 = ph[j + 3];
-    const float d0 = dist2_nc(qx, qy, qz, p0.pm.x, p0.pm.y, p0.pm.z);
-    const float d1 = dist2_nc(qx, qy, qz, p1.pm.x, p1.pm.y, p1.pm.z);
-    const float d2 = dist2_nc(qx, qy, qz, p2.pm.x, p2.pm.y, p2.pm.z);
-    const float d3 = dist2_nc(qx, qy, qz, p3.pm.x, p3.pm.y, p3.pm.z);
-    on_photon(j, p0.pm, p0.dm, d0, d0 <= r2, true);
-    on_photon(j + 1, p1.pm, p1.dm, d1, d1 <= r2, true);
-    on_photon(j + 2, p2.pm, p2.dm, d2, d2 <= r2, true);
-    on_photon(j + 3, p3.pm, p3.dm, d3, d3 <= r2, true);
-  }
-  for (; j < se.y; ++j) {
-    const PhotonRec p0 = ph[j];
-    const float d0 = dist2_nc(qx, qy, qz, p0.pm.x, p0.pm.y, p0.pm.z);
-    on_photon(j, p0.pm, p0.dm, d0, d0 <= r2, true);
-  }
-}
-
+// Every photon of the pass's grid within the ball (q, r2): each sorted index j
+// with dist2_nc(q, p_j) <= r2, each once.  Buckets are visited in cell order
+// (x fastest, then y, then z), photons in sorted order within a bucket, so a
+// query's sum is formed in a fixed order.  Per lane: no cross-lane operations
+// but the callbacks' own, so inactive lanes may skip it.
 // The photons of a query's (at most) eight cell ranges se[0..7] walked in
 // one loop, as one sequence: a lane moves on to its next range when it has
 // used up the current one.  Walked range by range, a wave ran each cell's
@@ -1516,14 +1465,15 @@ __device__ __forceinline__ void grid_range_scan_all(const PhotonRec* ph, uint2 s
 // next bucket's records, or the GRID_READ_SLACK zeroed ones after the last)
 // are marked not valid.  The next step's records are loaded before the
 // current ones are tested (256x256 box, whose waves each shade one group:
-// shade 0.085 -> 0.078 ms alone; caustic 0.340 -> 0.330).  ALL: on_photon(j, pm, dm, d2, inside, valid) for
-// every slot, inside only when valid; otherwise on_photon(j, pm, dm, d2) for
-// the valid photons inside the ball.
-template <bool ALL, typename OnPhoton>
-__device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se)[8], float qx, float qy, float qz,
-                                           float r2, OnPhoton& on_photon) {
-  uint32_t k = 0, j = se[0].x, e = se[0].y;
-  auto advance = [&]() -> bool {  // j, e to the next range with photons left
+// shade 0.085 -> 0.078 ms alone; caustic 0.340 -> 0.330).
+// ALL: on_photon(j, pm, dm, d2, inside, valid) for every slot, inside only when
+// valid; otherwise on_photon(j, pm, dm, d2) for the valid photons inside the
+// ball.
+struct RangeWalk {
+  uint32_t k, j, e;
+  __device__ __forceinline__ explicit RangeWalk(const uint2 (&se)[8]) : k(0), j(se[0].x), e(se[0].y) {}
+  // j, e to the next range with photons left
+  __device__ __forceinline__ bool advance(const uint2 (&se)[8]) {
     while (j >= e) {
       if (++k >= 8u) return false;
       // range k (k differs between lanes: a chain of selects, not an index)
@@ -1534,16 +1484,21 @@ __device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se
       e = n.y;
     }
     return true;
-  };
-  if (!advance()) return;
-  const PhotonRec* p = ph + j;
+  }
+};
+template <bool ALL, typename OnPhoton>
+__device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se)[8], float qx, float qy, float qz,
+                                           float r2, OnPhoton& on_photon) {
+  RangeWalk w(se);
+  if (!w.advance(se)) return;
+  const PhotonRec* p = ph + w.j;
   PhotonRec p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
   while (true) {
-    const uint32_t j0 = j, i1 = j + 1u, i2 = j + 2u, i3 = j + 3u;
-    const bool v1 = i1 < e, v2 = i2 < e, v3 = i3 < e;
-    j += 4u;
-    const bool more = advance();
-    const PhotonRec* q = ph + (more ? j : j0);
+    const uint32_t j0 = w.j, i1 = j0 + 1u, i2 = j0 + 2u, i3 = j0 + 3u;
+    const bool v1 = i1 < w.e, v2 = i2 < w.e, v3 = i3 < w.e;
+    w.j += 4u;
+    const bool more = w.advance(se);
+    const PhotonRec* q = ph + (more ? w.j : j0);
     const PhotonRec q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
     const float d0 = dist2_nc(qx, qy, qz, p0.pm.x, p0.pm.y, p0.pm.z);
     const float d1 = dist2_nc(qx, qy, qz, p1.pm.x, p1.pm.y, p1.pm.z);
@@ -1568,20 +1523,15 @@ __device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se
   }
 }
 
-template <typename OnPhoton>
-__device__ __forceinline__ void grid_bucket_scan(const uint2* cells, const PhotonRec* ph, uint32_t b, float qx,
-                                                 float qy, float qz, float r2, OnPhoton& on_photon) {
-  grid_range_scan(ph, cells[b], qx, qy, qz, r2, on_photon);
-}
-
-// Returns false (and scans only the first three cells of an axis) if the
-// query's cells span more than three per axis, which the cell side rules out
-// for every finite point (the caller raises a flag).
-// ALL = true: on_photon(j, pm, dm, d2, inside, valid) for every photon of the
-// cells, in the same order, and for padding slots with valid = false.
-template <bool ALL = false, typename OnPhoton>
-__device__ __forceinline__ bool grid_query(const GridView& g, const uint2* cells, const PhotonRec* ph, float qx,
-                                           float qy, float qz, float r2, OnPhoton&& on_photon) {
+// walk(se) for the ranges of the query's cells, in cell order: all of them in
+// one call when the query meets at most 2 x 2 x 2 cells, which the cell side
+// makes the rule; else (float rounding at the edge of the bound) one range
+// per call.  Returns false (and walks only the first three cells of an axis)
+// if the query's cells span more than three per axis, which the cell side
+// rules out for every finite point (the caller raises a flag).
+template <typename Walk>
+__device__ __forceinline__ bool grid_ranges(const GridView& g, const uint2* cells, float qx, float qy, float qz,
+                                            Walk&& walk) {
   const float rx = g.reach + GRID_REL_MARGIN * fabsf(qx);
   const float ry = g.reach + GRID_REL_MARGIN * fabsf(qy);
   const float rz = g.reach + GRID_REL_MARGIN * fabsf(qz);
@@ -1589,8 +1539,8 @@ __device__ __forceinline__ bool grid_query(const GridView& g, const uint2* cells
   const int y0 = grid_coord(qy - ry, g.bmin.y, g.inv_c, g.lim), y1 = grid_coord(qy + ry, g.bmin.y, g.inv_c, g.lim);
   const int z0 = grid_coord(qz - rz, g.bmin.z, g.inv_c, g.lim), z1 = grid_coord(qz + rz, g.bmin.z, g.inv_c, g.lim);
   if (x1 - x0 <= 1 && y1 - y0 <= 1 && z1 - z0 <= 1) {
-    // at most 2 x 2 x 2 cells (the cell side makes this the rule): buckets in
-    // registers, a bucket met twice (two cells hashed alike) scanned once
+    // buckets in registers, a bucket met twice (two cells hashed alike)
+    // scanned once
     uint32_t b[8];
     bool v[8];
 #pragma unroll
@@ -1606,11 +1556,10 @@ __device__ __forceinline__ bool grid_query(const GridView& g, const uint2* cells
     uint2 se[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) se[k] = v[k] ? cells[b[k]] : make_uint2(0u, 0u);
-    grid_walk8<ALL>(ph, se, qx, qy, qz, r2, on_photon);
+    walk(se);
     return true;
   }
-  // three cells on some axis (float rounding at the edge of the bound): the
-  // same order, duplicates found by recomputing the earlier cells' buckets
+  // the same order, duplicates found by recomputing the earlier cells' buckets
   const bool ok = x1 - x0 <= 2 && y1 - y0 <= 2 && z1 - z0 <= 2;
   const int xe = min(x1, x0 + 2), ye = min(y1, y0 + 2), ze = min(z1, z0 + 2);
   for (int z = z0; z <= ze; ++z)
@@ -1625,13 +1574,21 @@ __device__ __forceinline__ bool grid_query(const GridView& g, const uint2* cells
               dup = dup || (earlier && grid_bucket(xx, yy, zz, g.mask) == b);
             }
         if (!dup) {
-          if constexpr (ALL)
-            grid_range_scan_all(ph, cells[b], qx, qy, qz, r2, on_photon);
-          else
-            grid_bucket_scan(cells, ph, b, qx, qy, qz, r2, on_photon);
+          uint2 se[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) se[k] = k == 0 ? cells[b] : make_uint2(0u, 0u);
+          walk(se);
         }
       }
   return ok;
+}
+
+// on_photon for the photons of the query's cells (grid_walk8).
+template <bool ALL = false, typename OnPhoton>
+__device__ __forceinline__ bool grid_query(const GridView& g, const uint2* cells, const PhotonRec* ph, float qx,
+                                           float qy, float qz, float r2, OnPhoton&& on_photon) {
+  return grid_ranges(g, cells, qx, qy, qz,
+                     [&](const uint2 (&se)[8]) { grid_walk8<ALL>(ph, se, qx, qy, qz, r2, on_photon); });
 }
 
 // ===========================================================================
@@ -2098,82 +2055,98 @@ hipError_t launch_eye(hipStream_t s, const SceneBuf& sc, PassState* st, const Ey
   return hipGetLastError();
 }
 
-// ===========================================================================
-// Wave-coherent radius query over the heap-ordered tree.  Stackless DFS:
-// descend to the left child while any lane's ball overlaps the node box;
-// otherwise step to the next sibling, climbing while at a right child.  At a
-// leaf, the 64 photons are staged once into this wave's LDS slice with
-// coalesced loads and every lane tests them from LDS (broadcast reads).
-
-struct LeafLds {
-  float4 pm[LEAF];
-  float4 dm[LEAF];
-};
-
-template <typename OnPhoton>
-__device__ __forceinline__ void wave_query(const Node* nodes, const PhotonRec* ph, uint32_t n, uint32_t depth,
-                                           bool active, float qx, float qy, float qz, float r2box, LeafLds& lds,
-                                           OnPhoton&& on_photon) {
-  const uint32_t lane = lane_id();
-  const uint32_t first_leaf = (1u << depth) - 1u;
-  uint32_t node = 0;
-  if (n == 0) return;
-  while (true) {
-    node = __builtin_amdgcn_readfirstlane(node);
-    const Node nd = ldc(nodes, node);
-    const bool ov = active && box_dist2_nc(qx, qy, qz, nd.lo, nd.hi) <= r2box;
-    if (__ballot(ov)) {
-      if (node < first_leaf) {
-        node = 2 * node + 1;
-        continue;
-      }
-      const uint32_t base = (node - first_leaf) * LEAF;
-      const uint32_t cnt = base < n ? min((uint32_t)LEAF, n - base) : 0u;
-      if (lane < cnt) {
-        const PhotonRec r = ph[base + lane];
-        lds.pm[lane] = r.pm;
-        lds.dm[lane] = r.dm;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (ov) {
-        for (uint32_t j = 0; j < cnt; ++j) on_photon(base + j, lds.pm[j], lds.dm[j]);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    while (node != 0 && (node & 1u) == 0) node = (node - 1) >> 1;
-    if (node == 0) break;
-    node += 1;
-  }
+// Ordered sum of the per-channel terms (0 when the photon does not count) of
+// each lane of the quad, lane 0's first: exact additions of v or 0, as with
+// one lane.
+template <int K>
+__device__ __forceinline__ void quad_photon(float vr, float vg, float vb, float& ar, float& ag, float& ab) {
+  ar += quad_get<K>(vr);
+  ag += quad_get<K>(vg);
+  ab += quad_get<K>(vb);
+}
+__device__ __forceinline__ void quad_photons(float vr, float vg, float vb, float& ar, float& ag, float& ab) {
+  quad_photon<0>(vr, vg, vb, ar, ag, ab);
+  quad_photon<1>(vr, vg, vb, ar, ag, ab);
+  quad_photon<2>(vr, vg, vb, ar, ag, ab);
+  quad_photon<3>(vr, vg, vb, ar, ag, ab);
 }
 
-// Gather of one query: Σ filter * max(0, -n.dir) per channel over the ball
-// (estimate_radiance, tracer.rs:179-195; photon_to_radiance, optics.rs:224-233).
-struct GatherAcc {
-  float r, g, b;
-};
-
-__device__ __forceinline__ GatherAcc gather_query(const Node* nodes, const PhotonRec* ph, uint32_t n, uint32_t depth,
-                                                  bool active, const Query& qq, float r2, int pf, LeafLds& lds) {
-  GatherAcc a{0.0f, 0.0f, 0.0f};
-  const float qx = qq.a.x, qy = qq.a.y, qz = qq.a.z;
-  const float nx = qq.b.x, ny = qq.b.y, nz = qq.b.z;
-  const float inv_r2 = 1.0f / r2;
-  wave_query(nodes, ph, n, depth, active, qx, qy, qz, r2, lds, [&](uint32_t, float4 pm, float4 dm) {
-    const float d2 = dist2_nc(qx, qy, qz, pm.x, pm.y, pm.z);
-    if (d2 <= r2) {
-      const float c = nx * dm.x + ny * dm.y + nz * dm.z;
-      const float v = c < 0.0f ? -c * filter_weight(pf, d2 * inv_r2) * dm.w : 0.0f;
-      const uint32_t wl = __float_as_uint(pm.w) & 3u;
-      a.r += wl == 0 ? v : 0.0f;
-      a.g += wl == 1 ? v : 0.0f;
-      a.b += wl == 2 ? v : 0.0f;
+// ===========================================================================
+// Radius query over the heap-ordered tree, one query per lane: the photons of
+// every leaf whose box meets the ball, leaves from left to right, photons in
+// order, on_photon(j, pm, dm) for each.  Each lane walks its own nodes, both
+// children's boxes in one step, the right one deferred on a bit trail (as in
+// the scene BVH's walk), and the lanes of a wave scan their leaves together,
+// four records per step with the next four in flight.  Bound by the latency
+// of the node loads (some 30 steps per query, shared cache lines).  Walking
+// the union of the wave's balls together, each leaf staged in LDS, made every
+// wave pass over every leaf that any of its 64 balls met: 200k texels over 1M
+// photons 3.68 ms, 0.83 ms with one lane per query, 0.49 ms with four.
+// Q: the four lanes of a quad walk the same query's nodes and take a leaf's
+// photons in turn; on_photon(j, pm, dm, valid) then is called by all four, for
+// four consecutive photons at a time.  One lane's chain of steps (up to a
+// thousand photons in a bright spot's ball) set the kernel's time.  Over the
+// pass's grid the quad lost (256x256 box: pass 0.106 -> 0.131 ms, caustic
+// 0.62 -> 0.93): there the instructions bound the gather, not the chain.
+template <bool Q, typename OnPhoton>
+__device__ __forceinline__ void tree_query(const Node* nodes, const PhotonRec* ph, uint32_t n, uint32_t depth, float qx,
+                                           float qy, float qz, float r2box, OnPhoton&& on_photon) {
+  if (n == 0) return;
+  const uint32_t first_leaf = (1u << depth) - 1u;
+  uint32_t node = 0, trail = 0;
+  bool more = true;
+  {
+    const Node nd = nodes[0];
+    more = box_dist2_nc(qx, qy, qz, nd.lo, nd.hi) <= r2box;
+  }
+  while (more) {
+    // down, or to the next deferred node, until the lane stands at a leaf
+    while (more && node < first_leaf) {
+      const uint32_t l = 2u * node + 1u;
+      const Node a = nodes[l], b = nodes[l + 1u];
+      const bool ha = box_dist2_nc(qx, qy, qz, a.lo, a.hi) <= r2box;
+      const bool hb = box_dist2_nc(qx, qy, qz, b.lo, b.hi) <= r2box;
+      if (ha && hb) trail |= 1u << heap_level(l);
+      if (ha || hb)
+        node = ha ? l : l + 1u;
+      else if (trail != 0u)
+        node = trail_pop(trail, node);
+      else
+        more = false;
     }
-  });
-  return a;
+    if (more) {
+      const uint32_t base = (node - first_leaf) * LEAF;
+      const uint32_t end = base < n ? min(base + (uint32_t)LEAF, n) : base;
+      if (base < end) {
+        constexpr uint32_t S = Q ? 16u : 4u, L = Q ? 4u : 1u;  // photons per step, lanes on a query
+        const uint32_t last = end - 1u, sub = Q ? lane_id() & 3u : 0u;
+        PhotonRec r[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) r[i] = ph[min(base + L * i + sub, last)];
+        for (uint32_t j = base; j < end; j += S) {
+          PhotonRec q[4];
+          if (j + S < end) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) q[i] = ph[min(j + S + L * i + sub, last)];
+          }
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t k = j + L * i + sub;
+            if constexpr (Q)
+              on_photon(k, r[i].pm, r[i].dm, k < end);
+            else if (k < end)
+              on_photon(k, r[i].pm, r[i].dm, true);
+          }
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i) r[i] = q[i];
+        }
+      }
+      if (trail != 0u)
+        node = trail_pop(trail, node);
+      else
+        more = false;
+    }
+  }
 }
 
 // Sort keys of the queries: one wave per tile; lane i writes its pixel's
@@ -2277,7 +2250,7 @@ template <int BV, int PF, bool BVH = (BV != 0)>
 __device__ __forceinline__ void k_shade_body(SceneView sc, const uint2* cells, const PhotonRec* ph, PassState* st,
                                                EyeBuf eb, const uint32_t* order, int pf, int uc, Blk blk) {
   const uint32_t nq = st->n_qsort;
-  const uint32_t groups = (nq + 63) / 64;
+  const uint32_t groups = (nq + 63u) / 64u;
   // The grid is sized for a full GPU, whatever the queries (their number is
   // only known on the device): the waves past one per group leave before they
   // touch the counters or copy the scene.  With 65k queries, 5120 waves asking
@@ -2294,7 +2267,7 @@ __device__ __forceinline__ void k_shade_body(SceneView sc, const uint2* cells, c
   const uint32_t per = (groups + 7u) / 8u;
   for (uint32_t gi = wave_next_part(st->work[WORK_SHADE], wc, wtries, groups, per); gi < groups;
        gi = wave_next_part(st->work[WORK_SHADE], wc, wtries, groups, per)) {
-    const uint32_t i = gi * 64 + lane_id();
+    const uint32_t i = gi * 64u + lane_id();
     if (i >= nq) continue;
     const uint32_t slot = order[i];
     const Query qq = eb.q[slot];
@@ -2317,92 +2290,48 @@ __global__ __launch_bounds__(256) void k_shade(SceneView sc, const uint2* cells,
 template <int BV>
 static void launch_shade(hipStream_t s, uint32_t blocks, size_t shmem, const SceneView& v, const uint2* cells,
                          const PhotonRec* ph, PassState* st, const EyeBuf& eb, const uint32_t* order, int pf, int uc) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), shmem, s, v, cells, ph, st, eb, order, pf, uc);
+  };
   if (pf == FILTER_CONE)
-    hipLaunchKernelGGL((k_shade<BV, FILTER_CONE>), dim3(blocks), dim3(256), shmem, s, v, cells, ph, st, eb, order, pf,
-                       uc);
+    go(k_shade<BV, FILTER_CONE>);
   else if (pf == FILTER_GAUSS)
-    hipLaunchKernelGGL((k_shade<BV, FILTER_GAUSS>), dim3(blocks), dim3(256), shmem, s, v, cells, ph, st, eb, order,
-                       pf, uc);
+    go(k_shade<BV, FILTER_GAUSS>);
   else
-    hipLaunchKernelGGL((k_shade<BV, FILTER_NONE>), dim3(blocks), dim3(256), shmem, s, v, cells, ph, st, eb, order, pf,
-                       uc);
+    go(k_shade<BV, FILTER_NONE>);
 }
 
 // The same shading over a box-tree map (ppm_trace_eye on a PhotonMap, whose
-// radius comes with the call): a wave takes 64 consecutive sorted queries
-// and traverses the tree for the union of their balls; each overlapped leaf
-// is staged once into LDS with coalesced loads and every lane whose ball
-// overlaps the leaf box tests its photons from LDS (broadcast reads).
+// radius comes with the call): four lanes per query, walking the tree for its
+// ball (tree_query).
 template <int BV, bool BVH = (BV != 0)>
 __device__ __forceinline__ void k_shade_tree_body(SceneView sc, const Node* nodes, const PhotonRec* ph,
                                                const PassState* st, EyeBuf eb, const uint32_t* order, int pf,
                                                int uc, Blk blk) {
-  __shared__ LeafLds lds[4];
-  const uint32_t wib = threadIdx.x >> 6, lane = lane_id();
   const uint32_t n = st->n_stored, depth = st->depth;
   const float r2 = st->r2f, scale = st->scale, inv_r2 = 1.0f / r2;
   const uint32_t nq = st->n_qsort;
-  const uint32_t groups = (nq + 63) / 64;
-  const uint32_t waves = blk.n * 4;
-  const uint32_t first_leaf = (1u << depth) - 1u;
-  for (uint32_t g = blk.b * 4 + wib; g < groups; g += waves) {
-    const uint32_t i = g * 64 + lane;
-    const bool active = i < nq;
-    uint32_t slot = 0;
-    Query qq{};
-    if (active) {
-      slot = order[i];
-      qq = eb.q[slot];
-    }
+  if (blk.b * 64u >= nq) return;
+  scene_to_lds<BV>(sc);
+  const uint32_t step = blk.n * 64u;
+  for (uint32_t base = blk.b * 64u; base < nq; base += step) {
+    const uint32_t i = base + (threadIdx.x >> 2);
+    if (i >= nq) continue;
+    const uint32_t slot = order[i];
+    const Query qq = eb.q[slot];
     const float qx = qq.a.x, qy = qq.a.y, qz = qq.a.z;
     const float nx = qq.b.x, ny = qq.b.y, nz = qq.b.z;
     float ar = 0.0f, ag = 0.0f, ab = 0.0f;
-    uint32_t node = 0;
-    while (n > 0) {
-      node = __builtin_amdgcn_readfirstlane(node);
-      const Node nd = ldc(nodes, node);
-      const bool ov = active && box_dist2_nc(qx, qy, qz, nd.lo, nd.hi) <= r2;
-      if (__ballot(ov)) {
-        if (node < first_leaf) {
-          node = 2 * node + 1;
-          continue;
-        }
-        const uint32_t base = (node - first_leaf) * LEAF;
-        const uint32_t cnt = base < n ? min((uint32_t)LEAF, n - base) : 0u;
-        if (lane < cnt) {
-          const PhotonRec r = ph[base + lane];
-          lds[wib].pm[lane] = r.pm;
-          lds[wib].dm[lane] = r.dm;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (ov) {
-          for (uint32_t j = 0; j < cnt; ++j) {
-            const float4 pm = lds[wib].pm[j];
-            const float d2 = dist2_nc(qx, qy, qz, pm.x, pm.y, pm.z);
-            if (d2 <= r2) {
-              const float4 dm = lds[wib].dm[j];
-              const float c = nx * dm.x + ny * dm.y + nz * dm.z;  // optics.rs:225
-              const float v = c < 0.0f ? -c * filter_weight(pf, d2 * inv_r2) * dm.w : 0.0f;
-              const uint32_t wl = __float_as_uint(pm.w) & 3u;
-              ar += wl == 0 ? v : 0.0f;
-              ag += wl == 1 ? v : 0.0f;
-              ab += wl == 2 ? v : 0.0f;
-            }
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
-      while (node != 0 && (node & 1u) == 0) node = (node - 1) >> 1;
-      if (node == 0) break;
-      node += 1;
-    }
+    tree_query<true>(nodes, ph, n, depth, qx, qy, qz, r2, [&](uint32_t, float4 pm, float4 dm, bool valid) {
+      const float d2 = dist2_nc(qx, qy, qz, pm.x, pm.y, pm.z);
+      const float c = photon_cos(nx, ny, nz, dm);  // optics.rs:225
+      const float v = (valid && d2 <= r2 && c < 0.0f) ? -c * filter_weight(pf, d2 * inv_r2) * dm.w : 0.0f;
+      const uint32_t wl = __float_as_uint(pm.w) & 3u;
+      quad_photons(wl == 0 ? v : 0.0f, wl == 1 ? v : 0.0f, wl == 2 ? v : 0.0f, ar, ag, ab);
+    });
     C3 di = C3{ar * scale, ag * scale, ab * scale};
-    if (uc) di = di + direct_light<BV>(sc, mk(qq.a), mk(qq.b));
-    if (active) eb.res[slot] = make_float4(qq.w.x * di.r, qq.w.y * di.g, qq.w.z * di.b, 0.0f);
+    if (uc) di = di + direct_light_quad<BV>(sc, mk(qq.a), mk(qq.b));
+    if ((threadIdx.x & 3u) == 0u) eb.res[slot] = make_float4(qq.w.x * di.r, qq.w.y * di.g, qq.w.z * di.b, 0.0f);
   }
 }
 
@@ -2673,20 +2602,20 @@ hipError_t launch_gather(hipStream_t s, const SceneBuf& sc, const MapBuf& m, Pas
         launch_shade<0>(s, blocks, 0, v, m.cells, m.sorted, st, eb, qv[cur], pfilter, use_classic);
     }
   } else {
+    // four lanes per query; the blocks past the queries leave at once
+    const uint32_t tblocks = (uint32_t)n_cu * 16u;
     switch (bvh_kind(sc)) {
       case 2:
-        hipLaunchKernelGGL(k_shade_tree<2>, dim3(blocks), dim3(256), bvh_dyn_lds(sc), s, v, m.nodes, m.sorted, st,
-                         eb, qv[cur],
-                         pfilter, use_classic);
+        hipLaunchKernelGGL(k_shade_tree<2>, dim3(tblocks), dim3(256), bvh_dyn_lds(sc), s, v, m.nodes, m.sorted, st, eb,
+                           qv[cur], pfilter, use_classic);
         break;
       case 1:
-        hipLaunchKernelGGL(k_shade_tree<1>, dim3(blocks), dim3(256), 0, s, v, m.nodes, m.sorted, st,
-                         eb, qv[cur],
-                         pfilter, use_classic);
+        hipLaunchKernelGGL(k_shade_tree<1>, dim3(tblocks), dim3(256), 0, s, v, m.nodes, m.sorted, st, eb, qv[cur],
+                           pfilter, use_classic);
         break;
       default:
-        hipLaunchKernelGGL(k_shade_tree<0>, dim3(blocks), dim3(256), 0, s, v, m.nodes, m.sorted, st, eb, qv[cur],
-                         pfilter, use_classic);
+        hipLaunchKernelGGL(k_shade_tree<0>, dim3(tblocks), dim3(256), 0, s, v, m.nodes, m.sorted, st, eb, qv[cur],
+                           pfilter, use_classic);
     }
   }
   if (ev && (e = hipEventRecord(ev[1], s)) != hipSuccess) return e;
@@ -2787,27 +2716,23 @@ __device__ __forceinline__ bool in_ball(float d2f, float r2f, float band, bool r
   return s <= r2;
 }
 
+template <int MODE>
 __global__ __launch_bounds__(256) void k_query(const Node* nodes, const PhotonRec* ph, const double* ph64,
                                                const uint32_t* src_idx, const PassState* st, const float4* qf,
                                                const double* q64, const float4* qn, uint32_t nq, double r2,
-                                               int refine, int mode, int pf, uint32_t* counts,
+                                               int refine, int pf, uint32_t* counts,
                                                const uint64_t* offsets, uint32_t* idx_out, float4* rgb_out) {
-  __shared__ LeafLds lds[4];
-  const uint32_t w_in_b = threadIdx.x >> 6;
-  const uint32_t lane = lane_id();
   const uint32_t n = st->n_stored;
   const uint32_t depth = st->depth;
   const float r2f = (float)r2;
-  const uint32_t groups = (nq + 63) / 64;
-  const uint32_t waves = gridDim.x * 4;
-  for (uint32_t g = blockIdx.x * 4 + w_in_b; g < groups; g += waves) {
-    const uint32_t i = g * 64 + lane;
-    const bool active = i < nq;
-    const float4 qp = active ? qf[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 nn = (active && mode == 2) ? qn[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  // sums (mode 2): four lanes per query; counts and lists: one
+  constexpr uint32_t L = MODE == 2 ? 4u : 1u;
+  for (uint32_t i = (blockIdx.x * 256u + threadIdx.x) / L; i < nq; i += gridDim.x * (256u / L)) {
+    const float4 qp = qf[i];
+    const float4 nn = MODE == 2 ? qn[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     double qx = 0, qy = 0, qz = 0;
     float band = 0.0f;
-    if (active && refine) {
+    if (refine) {
       qx = q64[3 * (uint64_t)i];
       qy = q64[3 * (uint64_t)i + 1];
       qz = q64[3 * (uint64_t)i + 2];
@@ -2817,42 +2742,43 @@ __global__ __launch_bounds__(256) void k_query(const Node* nodes, const PhotonRe
     }
     const float r2box = refine ? r2f + band : r2f;
     uint32_t cnt = 0;
-    const uint64_t off = (mode == 1 && active) ? offsets[i] : 0;
+    const uint64_t off = MODE == 1 ? offsets[i] : 0;
     float ar = 0.f, ag = 0.f, ab = 0.f;
-    wave_query(nodes, ph, n, depth, active, qp.x, qp.y, qp.z, r2box, lds[w_in_b],
-               [&](uint32_t j, float4 pm, float4 dm) {
-                 const float d2 = dist2_nc(qp.x, qp.y, qp.z, pm.x, pm.y, pm.z);
-                 float t;
-                 if (in_ball(d2, r2f, band, refine != 0, ph64, j, qx, qy, qz, r2, &t)) {
-                   if (mode == 1) idx_out[off + cnt] = src_idx[j];
-                   ++cnt;
-                   if (mode == 2) {
-                     const float c = nn.x * dm.x + nn.y * dm.y + nn.z * dm.z;
-                     const float v = c < 0.0f ? -c * filter_weight(pf, t) * dm.w : 0.0f;
-                     const uint32_t wl = __float_as_uint(pm.w) & 3u;
-                     ar += wl == 0 ? v : 0.0f;
-                     ag += wl == 1 ? v : 0.0f;
-                     ab += wl == 2 ? v : 0.0f;
-                   }
-                 }
-               });
-    if (active) {
-      if (mode == 0) counts[i] = cnt;
-      if (mode == 2) rgb_out[i] = make_float4(ar, ag, ab, 0.0f);
-    }
+    tree_query<MODE == 2>(nodes, ph, n, depth, qp.x, qp.y, qp.z, r2box,
+                          [&](uint32_t j, float4 pm, float4 dm, bool valid) {
+      const float d2 = dist2_nc(qp.x, qp.y, qp.z, pm.x, pm.y, pm.z);
+      float t;
+      const bool in = valid && in_ball(d2, r2f, band, refine != 0, ph64, j, qx, qy, qz, r2, &t);
+      if constexpr (MODE == 2) {
+        const float c = photon_cos(nn.x, nn.y, nn.z, dm);
+        const float v = in && c < 0.0f ? -c * filter_weight(pf, t) * dm.w : 0.0f;
+        const uint32_t wl = __float_as_uint(pm.w) & 3u;
+        quad_photons(wl == 0 ? v : 0.0f, wl == 1 ? v : 0.0f, wl == 2 ? v : 0.0f, ar, ag, ab);
+      } else if (in) {
+        if (MODE == 1) idx_out[off + cnt] = src_idx[j];
+        ++cnt;
+      }
+    });
+    if (MODE == 0) counts[i] = cnt;
+    if (MODE == 2 && (threadIdx.x & 3u) == 0u) rgb_out[i] = make_float4(ar, ag, ab, 0.0f);
   }
 }
 
 hipError_t launch_query(hipStream_t s, const MapBuf& m, PassState* st, const float4* qf, const double* q64,
                         const float4* qn, uint32_t nq, double r2, int refine64, int mode, int pfilter,
                         uint32_t* counts, const uint64_t* offsets, uint32_t* idx_out, float4* rgb_out, int n_cu) {
-  uint32_t groups = (nq + 63) / 64;
-  uint32_t blocks = (groups + 3) / 4;
-  uint32_t maxb = (uint32_t)n_cu * 8u;
-  if (blocks > maxb) blocks = maxb;
-  if (blocks == 0) blocks = 1;
-  hipLaunchKernelGGL(k_query, dim3(blocks), dim3(256), 0, s, m.nodes, m.sorted, m.sorted64, m.src_idx, st, qf, q64,
-                     qn, nq, r2, refine64, mode, pfilter, counts, offsets, idx_out, rgb_out);
+  const uint32_t per = mode == 2 ? 64u : 256u;  // queries per block
+  const uint32_t blocks = std::max<uint32_t>(1u, std::min<uint32_t>((nq + per - 1u) / per, (uint32_t)n_cu * 32u));
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, m.nodes, m.sorted, m.sorted64, m.src_idx, st, qf, q64,
+                       qn, nq, r2, refine64, pfilter, counts, offsets, idx_out, rgb_out);
+  };
+  if (mode == 2)
+    go(k_query<2>);
+  else if (mode == 1)
+    go(k_query<1>);
+  else
+    go(k_query<0>);
   return hipGetLastError();
 }
 
