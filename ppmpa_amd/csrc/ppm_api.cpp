@@ -2231,7 +2231,7 @@ struct ppm_batch {
   BatchItem* items = nullptr;      // device, K x n (pipeline-major), each in `order`
   uint32_t* tab = nullptr;         // device, BK_KINDS x (n + 1)
   std::vector<uint32_t> htab;
-  bool bvh = false;
+  int bvh = 0;                     // the scenes' bvh_kind() bits: the kernels' BV
   uint32_t dyn = 0;                // dynamic LDS of the BVH kernels: the most any scene asks (bvh_dyn_lds)
   ppm_launch_cfg lc{};
   std::vector<hipGraphExec_t> exec;  // per pipeline j and number of running scenes a: j * n + a - 1
@@ -2437,7 +2437,7 @@ ppm_status ppm_batch_create(ppm_ctx* c, uint32_t n, const ppm_scene* const* scen
       return st;
     }
     b->sess.push_back(s);
-    if (scenes[i]->buf.bvh) b->bvh = true;
+    b->bvh |= bvh_kind(scenes[i]->buf);
     b->dyn = std::max(b->dyn, bvh_dyn_lds(scenes[i]->buf));
   }
   b->order.resize(n);

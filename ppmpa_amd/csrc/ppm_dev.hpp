@@ -235,7 +235,7 @@ __device__ __forceinline__ void scene_to_lds(SceneView& sc) {
   }
   if (mat) copy16((float4*)g_mat_lds, (const float4*)sc.mats, (sc.n_mats + 1u) * (uint32_t)(sizeof(DevMaterial) / 16));
   bool nodes = false, prims = false;
-  if (BV == 2 && sc.dyn_lds && sc.n_bprims > 0) {
+  if (BV >= 2 && sc.dyn_lds && sc.n_bprims > 0) {
     const uint32_t n_nodes = (2u << sc.bvh_depth) - 1u;
     nodes = n_nodes <= BVH_LDS_NODES;
     prims = sc.n_bprims <= BVH_LDS_PRIMS;
@@ -461,9 +461,9 @@ __device__ __forceinline__ Node bvh_node(const SceneView& sc, uint32_t i) {
 }
 // The nearest-hit test of primitive j: from its LDS compact sphere when
 // scene_to_lds put the primitives there, else from global memory.
-template <bool CACHED>
+template <bool NL>
 __device__ __forceinline__ void bprim_hit(const SceneView& sc, uint32_t j, V3 o, V3 d, Hit& h) {
-  if (CACHED && (sc.lds & 8u)) {
+  if (NL) {
     const float4 c = bvh_lds_sph()[j];
     if (c.w >= 0.0f) {
       sphere_hit(mk(c.x, c.y, c.z), c.w, bvh_lds_idx()[j], o, d, h);
@@ -518,29 +518,57 @@ __device__ __forceinline__ uint32_t trail_pop(uint32_t& trail, uint32_t node) {
 // Nearest hit over the BVH primitives: ordered depth-first traversal (the
 // nearer child first, the farther one deferred on the bit trail).  A node is
 // entered while its box starts no later than the best hit, so equal
-// distances still reach the lower shape index.
-template <bool CACHED, bool NL>
-__device__ __forceinline__ void bvh_nearest_walk(const SceneView& sc, V3 o, V3 d, Hit& h) {
+// distances still reach the lower shape index: the hit does not depend on the
+// order in which nodes are visited.
+struct BvhRay {
+  V3 inv, noi;
+};
+struct BvhWalk {
+  uint32_t node, trail;
+};
+__device__ __forceinline__ BvhRay bvh_ray(V3 o, V3 d) {
   const V3 inv = slab_inv(d);
-  const V3 noi = mk(-o.x * inv.x, -o.y * inv.y, -o.z * inv.z);
-  const uint32_t first_leaf = (1u << sc.bvh_depth) - 1u;
-  uint32_t node = 0, trail = 0;
+  return BvhRay{inv, mk(-o.x * inv.x, -o.y * inv.y, -o.z * inv.z)};
+}
+// A walk of the subtree at `node`; false: the ray does not enter it.
+template <bool NL>
+__device__ __forceinline__ bool bvh_walk_begin(const SceneView& sc, const BvhRay& r, float tmax, uint32_t node,
+                                               BvhWalk& w) {
+  w.node = node;
+  w.trail = 0;
   float tn;
-  if (!slab(bvh_node<NL>(sc, 0), inv, noi, h.t, tn)) return;
+  return slab(bvh_node<NL>(sc, node), r.inv, r.noi, tmax, tn);
+}
+// The calling lanes' walks from w on.  SOME: until no more than `left` of them
+// are going or they went `steps` steps; true for those whose walks go on from w.
+template <bool NL, bool SOME>
+__device__ __forceinline__ bool bvh_walk_on(const SceneView& sc, V3 o, V3 d, const BvhRay& r, Hit& h, BvhWalk& w,
+                                            uint32_t left, uint32_t steps) {
+  const uint32_t first_leaf = (1u << sc.bvh_depth) - 1u;
+  uint32_t node = w.node, trail = w.trail;
+  bool going = false;
   while (true) {
+    if (SOME) {
+      if (steps == 0u || (uint32_t)__popcll(__ballot(true)) <= left) {
+        going = true;
+        break;
+      }
+      --steps;
+    }
+    float tn;
     if (node >= first_leaf) {
       if (NL) {
         leaf_hit_lds(sc, node - first_leaf, o, d, h);
       } else {
         const uint32_t base = (node - first_leaf) * sc.bvh_leaf;
         const uint32_t end = min(base + sc.bvh_leaf, sc.n_bprims);
-        for (uint32_t j = base; j < end; ++j) bprim_hit<CACHED>(sc, j, o, d, h);
+        for (uint32_t j = base; j < end; ++j) bprim_hit<NL>(sc, j, o, d, h);
       }
     } else {
       const uint32_t l = 2u * node + 1u;
       float tl, tr;
-      const bool hl = slab(bvh_node<NL>(sc, l), inv, noi, h.t, tl);
-      const bool hr = slab(bvh_node<NL>(sc, l + 1u), inv, noi, h.t, tr);
+      const bool hl = slab(bvh_node<NL>(sc, l), r.inv, r.noi, h.t, tl);
+      const bool hr = slab(bvh_node<NL>(sc, l + 1u), r.inv, r.noi, h.t, tr);
       if (hl && hr) {
         const bool left_first = tl <= tr;
         node = left_first ? l : l + 1u;
@@ -555,27 +583,127 @@ __device__ __forceinline__ void bvh_nearest_walk(const SceneView& sc, V3 o, V3 d
     bool more = false;
     while (trail != 0u) {
       node = trail_pop(trail, node);
-      if (slab(bvh_node<NL>(sc, node), inv, noi, h.t, tn)) {
+      if (slab(bvh_node<NL>(sc, node), r.inv, r.noi, h.t, tn)) {
         more = true;
         break;
       }
     }
     if (!more) break;
   }
+  w.node = node;
+  w.trail = trail;
+  return going;
+}
+template <bool NL>
+__device__ __forceinline__ void bvh_nearest_walk(const SceneView& sc, V3 o, V3 d, Hit& h) {
+  const BvhRay r = bvh_ray(o, d);
+  BvhWalk w;
+  if (bvh_walk_begin<NL>(sc, r, h.t, 0u, w)) bvh_walk_on<NL, false>(sc, o, d, r, h, w, 0u, 0u);
 }
 template <bool CACHED>
 __device__ __forceinline__ void bvh_nearest(const SceneView& sc, V3 o, V3 d, Hit& h) {
   if (sc.n_bprims == 0) return;  // a scene without a BVH in a batch that has one
   if (CACHED && (sc.lds & 12u) == 12u)  // nodes and primitives in LDS
-    bvh_nearest_walk<CACHED, true>(sc, o, d, h);
+    bvh_nearest_walk<true>(sc, o, d, h);
   else
-    bvh_nearest_walk<CACHED, false>(sc, o, d, h);
+    bvh_nearest_walk<false>(sc, o, d, h);
 }
 
-// calc_intersection (tracer.rs:306-335): the nearest hit over every shape.
-// BVH = false: the scene has no BVH and `lin` holds all shapes.
-template <int BV, bool BVH = (BV != 0)>
-__device__ __forceinline__ Hit nearest(const SceneView& sc, V3 o, V3 d) {
+// --- the wave's walks together -------------------------------------------------
+// A step of a tracing wave lasts as long as its longest walk, while most rays
+// meet few nodes (327k-triangle mesh in a room: a tenth of the lanes of the
+// photon trace were at work).  So once WAVE_WALK_LEFT or fewer lanes walk, each
+// of them gives its shallowest deferred node (the largest subtree it has put
+// off) to an idle lane, which walks it for the same ray, again every
+// WAVE_WALK_STEPS steps; the lanes of a ray meet in its best hit so far, in LDS.
+// The nearest hit does not depend on who visits which node, so every hit is the
+// lone walk's.  Mesh pass 51.2 -> 33.3 ms; 20k triangles: trace alone 3.21 ->
+// 1.58 ms, eye 5.94 -> 3.40 (sharing every 4 steps 1.66 and 3.53, every 10 1.80
+// and 3.77; from 56 lanes on 1.76 and 3.66, from 16 on 2.07 and 4.18, both at 4
+// to 6 steps).
+constexpr uint32_t WAVE_WALK_LEFT = 48, WAVE_WALK_STEPS = 2;
+struct WalkLds {  // of one wave
+  unsigned long long best[64];  // per ray (its lane): distance bits, shape
+  uint2 mail[64];               // a given node and its ray's lane
+};
+__device__ __forceinline__ unsigned long long hit_key(const Hit& h) {
+  return ((unsigned long long)__float_as_uint(h.t) << 32) | (uint32_t)h.obj;
+}
+__device__ __forceinline__ Hit hit_of(unsigned long long k) {
+  return Hit{__uint_as_float((uint32_t)(k >> 32)), (int32_t)(uint32_t)k};
+}
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ uint64_t lanes_below() { return (1ull << __lane_id()) - 1ull; }
+__device__ __forceinline__ V3 shfl3(V3 a, uint32_t src) {
+  return mk(__shfl(a.x, (int)src), __shfl(a.y, (int)src), __shfl(a.z, (int)src));
+}
+// All lanes of the wave call it; act: the lane has a ray, and h its best hit
+// over the list.
+__device__ __forceinline__ void bvh_nearest_lanes(const SceneView& sc, WalkLds& wl, V3 o, V3 d, bool act, Hit& h) {
+  const uint32_t lane = __lane_id();
+  uint32_t own = lane;  // the ray that the lane walks for: its lane
+  V3 ro = o, rd = d;
+  BvhRay r = bvh_ray(o, d);
+  BvhWalk w{0u, 0u};
+  bool walking = false, split = false;
+  if (act) walking = bvh_walk_begin<false>(sc, r, h.t, 0u, w);
+  uint32_t left = WAVE_WALK_LEFT, steps = ~0u;
+  while (true) {
+    if (walking) walking = bvh_walk_on<false, true>(sc, ro, rd, r, h, w, left, steps);
+    const uint64_t going = __ballot(walking);
+    if (going == 0) break;
+    const uint64_t gives = __ballot(walking && w.trail != 0u);
+    const uint32_t n = min((uint32_t)__popcll(gives), 64u - (uint32_t)__popcll(going));
+    if (n != 0u) {
+      if (!split)
+        wl.best[lane] = hit_key(h);
+      else
+        atomicMin(&wl.best[own], hit_key(h));
+      split = true;
+      const uint64_t set = walking ? gives : ~going;
+      const uint32_t rank = (uint32_t)__popcll(set & lanes_below());
+      if (walking && w.trail != 0u && rank < n) {
+        const uint32_t k = (uint32_t)__builtin_ctz(w.trail);  // the shallowest level
+        w.trail &= w.trail - 1u;
+        const uint32_t a = ((w.node + 1u) >> (heap_level(w.node) - k)) - 1u;
+        wl.mail[rank] = make_uint2(((a - 1u) ^ 1u) + 1u, own);
+      }
+      wave_lds_fence();
+      uint32_t node = 0u;
+      const bool takes = !walking && rank < n;
+      if (takes) {
+        const uint2 m = wl.mail[rank];
+        node = m.x;
+        own = m.y;
+      }
+      h = hit_of(wl.best[own]);
+      const V3 no = shfl3(o, own), nd = shfl3(d, own);
+      if (takes) {
+        ro = no;
+        rd = nd;
+        r = bvh_ray(ro, rd);
+        walking = bvh_walk_begin<false>(sc, r, h.t, node, w);
+      }
+      wave_lds_fence();
+    }
+    const bool few = (uint32_t)__popcll(__ballot(walking)) <= WAVE_WALK_LEFT;
+    left = few ? 0u : WAVE_WALK_LEFT;
+    steps = few ? WAVE_WALK_STEPS : ~0u;
+  }
+  if (split) {
+    atomicMin(&wl.best[own], hit_key(h));
+    wave_lds_fence();
+    h = hit_of(wl.best[lane]);
+    wave_lds_fence();
+  }
+}
+
+// The nearest hit over the shapes of the list.
+__device__ __forceinline__ Hit nearest_listed(const SceneView& sc, V3 o, V3 d) {
   // the list is in scene order, so of equal distances the first one taken
   // stays; each record comes in scalar loads, the next one's in flight
   Hit h{INF_F, -1};
@@ -589,7 +717,32 @@ __device__ __forceinline__ Hit nearest(const SceneView& sc, V3 o, V3 d) {
     h.t = better ? t : h.t;
     h.obj = better ? (int32_t)__float_as_uint(r.b.w) : h.obj;
   }
-  if (BVH) bvh_nearest<BV == 2>(sc, o, d, h);
+  return h;
+}
+
+// calc_intersection (tracer.rs:306-335): the nearest hit over every shape.
+// BVH = false: the scene has no BVH and `lin` holds all shapes.
+template <int BV, bool BVH = (BV != 0)>
+__device__ __forceinline__ Hit nearest(const SceneView& sc, V3 o, V3 d) {
+  Hit h = nearest_listed(sc, o, d);
+  if (BVH) bvh_nearest<(BV >= 2)>(sc, o, d, h);
+  return h;
+}
+// The same for the rays of a wave (act: the lane has one; all lanes call it),
+// in kernels that walk large trees.  A tree in LDS is walked lane by lane:
+// its walks are short (300 spheres: sharing them took the trace from 0.71 to
+// 0.64 ms alone and the eye from 2.01 to 2.18, a batch of 24 rooms from 42.2
+// to 44.1 ms).
+template <int BV>
+__device__ __forceinline__ Hit nearest_wave(const SceneView& sc, WalkLds& wl, V3 o, V3 d, bool act) {
+  Hit h{INF_F, -1};
+  if (act) h = nearest_listed(sc, o, d);
+  if (sc.n_bprims == 0) return h;  // a scene without a BVH in a batch that has one
+  if (BV == 3 && (sc.lds & 12u) == 12u) {
+    if (act) bvh_nearest_walk<true>(sc, o, d, h);
+  } else {
+    bvh_nearest_lanes(sc, wl, o, d, act, h);
+  }
   return h;
 }
 
@@ -1154,7 +1307,7 @@ __device__ __forceinline__ bool sample_lit(const SceneView& sc, V3 p, V3 n, V3 l
   }
   for (uint32_t i = CAND_BITS; i < sc.n_lin; ++i)
     if (lin_occludes(sc, i, p, ld3, sq_l, any)) return false;
-  if (BVH && bvh_shadow<BV == 2>(sc, p, ld3, sq_l, any, occ)) return false;
+  if (BVH && bvh_shadow<(BV >= 2)>(sc, p, ld3, sq_l, any, occ)) return false;
   // no occluder; lit iff the ray meets something at all (calc_intersection
   // returns None otherwise, tracer.rs:284)
   for (uint32_t i = 0; i < min(sc.n_lin, CAND_BITS) && !any; ++i) {

@@ -194,16 +194,16 @@ __device__ __forceinline__ void emit_photon(const SceneView& sc, uint32_t pid, R
   p.d = d;
 }
 
-// One step of trace_photon.  Returns whether the photon lives on; `store`
-// reports a photon-map record (position, INCOMING direction, channel).
+// One step of trace_photon at the ray's nearest hit h.  Returns whether the
+// photon lives on; `store` reports a photon-map record (position, INCOMING
+// direction, channel).
 template <int BV, bool BVH = (BV != 0)>
-__device__ __forceinline__ bool photon_bounce(const SceneView& sc, int uc, int maxd, PhotonState& p, Rng& rng,
+__device__ __forceinline__ bool photon_bounce(const SceneView& sc, int uc, PhotonState& p, const Hit& h, Rng& rng,
                                               bool& store, V3& spos, int& ev_mat) {
   store = false;
   ev_mat = -1;
-  if ((int)p.depth >= maxd) return false;  // tracer.rs:32
   Isect is;
-  if (!intersect<BV>(sc, p.o, p.d, is)) return false;  // tracer.rs:36-39
+  if (!finish_hit<BV>(sc, p.o, p.d, h, is)) return false;  // tracer.rs:36-39
   const DevMaterial M = material(sc, is.mat);
   // tracer.rs:77-79
   store = (uc == 0 || p.depth > 0) && surf_store(M);
@@ -341,6 +341,8 @@ __device__ __forceinline__ void k_trace_photons_body(SceneView sc, PassState* st
   __shared__ float part[ADJ ? 3 * ADJ_LDS_MATS : 1];
   __shared__ uint16_t evl[ADJ ? ADJ_MAX_EV * 256 : 1];
   __shared__ EmitLds s_emit[4];
+  constexpr bool BIG = BV == 1 || BV == 3;  // large trees: the wave's walks together
+  __shared__ WalkLds s_walk[BIG ? 4 : 1];
   scene_to_lds<BV>(sc);
   const uint32_t w = blk.b * (blockDim.x / 64) + (threadIdx.x >> 6);
   if (ADJ) {
@@ -425,7 +427,13 @@ __device__ __forceinline__ void k_trace_photons_body(SceneView sc, PassState* st
     const uint32_t swl = p.wl;
     const uint32_t smeta = pack_meta(p.wl, p.depth, p.pid);
     int ev_mat = -1;
-    if (alive) alive = photon_bounce<BV>(sc, uc, maxd, p, rng, store, spos, ev_mat);
+    if constexpr (BIG) {
+      alive = alive && (int)p.depth < maxd;  // tracer.rs:32
+      const Hit h = nearest_wave<BV>(sc, s_walk[threadIdx.x >> 6], p.o, p.d, alive);
+      if (alive) alive = photon_bounce<BV>(sc, uc, p, h, rng, store, spos, ev_mat);
+    } else if (alive) {
+      alive = (int)p.depth < maxd && photon_bounce<BV>(sc, uc, p, nearest<BV>(sc, p.o, p.d), rng, store, spos, ev_mat);
+    }
     const uint64_t sm = __ballot(store);
     if (sm) {
       if (store) {
@@ -1779,6 +1787,8 @@ __device__ __forceinline__ void k_eye_body(SceneView sc, PassState* st, EyeBuf e
                                              int maxd, uint32_t n_waves, Blk blk) {
   __shared__ uint32_t s_nsec[4 * 64];  // per wave of the block and pixel of its tile
   __shared__ float s_acc[4 * 64 * 3];
+  constexpr bool BIG = BV == 1 || BV == 3;  // large trees: the wave's walks together
+  __shared__ WalkLds s_walk[BIG ? 4 : 1];
   scene_to_lds<BV>(sc);
   const uint32_t wb = threadIdx.x >> 6;
   const uint32_t w = blk.b * (blockDim.x / 64) + wb;
@@ -1847,11 +1857,18 @@ __device__ __forceinline__ void k_eye_body(SceneView sc, PassState* st, EyeBuf e
       C3 emit{0.0f, 0.0f, 0.0f};
       Query qq;
       const uint32_t depth = cur.meta & 31u;
+      Hit h{INF_F, -1};
+      if constexpr (BIG) h = nearest_wave<BV>(sc, s_walk[wb], cur.o, cur.d, alive && (int)depth < maxd);
       if (alive) {
         const uint32_t med = (cur.meta >> 5) & 2047u;
         const uint32_t path = cur.meta >> 16;
         Isect is;
-        if ((int)depth < maxd && intersect<BV>(sc, cur.o, cur.d, is)) {
+        bool met;
+        if constexpr (BIG)
+          met = finish_hit<BV>(sc, cur.o, cur.d, h, is);
+        else
+          met = (int)depth < maxd && intersect<BV>(sc, cur.o, cur.d, is);
+        if (met) {
           const DevMaterial M = material(sc, is.mat);
           const DevMaterial Mm = material(sc, med);
           emit = cur.w * (c3(M.em) * SR_HALF_F);
@@ -3073,14 +3090,17 @@ __global__ __launch_bounds__(256) void kb_accumulate(const BatchItem* items, con
 #undef BATCH_PROLOGUE
 
 hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
-                             uint32_t n_all, bool bvh, uint32_t dyn) {
+                             uint32_t n_all, int bvh, uint32_t dyn) {
   // blocks[k] = total blocks of kind k over the first n scenes.  One chain of
   // launches: the rounds of the other pipelines run beside it.
   const dim3 T256(256), T1024(1024), T64(64), TOS(OS_THREADS);
   hipError_t e;
   hipLaunchKernelGGL(kb_pass_begin, dim3(n), T64, 0, s, items, n);
   hipLaunchKernelGGL(kb_tile_order, dim3(blocks[BK_PIX]), T256, 0, s, items, tab, n, n_all);
-  switch ((bvh ? (dyn != 0u ? 2 : 1) : 0)) {
+  switch (bvh) {
+    case 3:
+      hipLaunchKernelGGL(kb_eye<3>, dim3(blocks[BK_EYE]), T256, dyn, s, items, tab, n, n_all);
+      break;
     case 2:
       hipLaunchKernelGGL(kb_eye<2>, dim3(blocks[BK_EYE]), T256, dyn, s, items, tab, n, n_all);
       break;
@@ -3097,7 +3117,10 @@ hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32
   for (uint32_t p = 0; p < QUERY_KEY_BITS / 8u; ++p)
     hipLaunchKernelGGL(kb_os_scatter<false>, dim3(blocks[BK_QOS]), TOS, 0, s, items, tab, n, n_all, 1, p);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  switch ((bvh ? (dyn != 0u ? 2 : 1) : 0)) {
+  switch (bvh) {
+    case 3:
+      hipLaunchKernelGGL(kb_trace<3>, dim3(blocks[BK_TRACE]), T256, dyn, s, items, tab, n, n_all);
+      break;
     case 2:
       hipLaunchKernelGGL(kb_trace<2>, dim3(blocks[BK_TRACE]), T256, dyn, s, items, tab, n, n_all);
       break;
@@ -3119,7 +3142,10 @@ hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32
   hipLaunchKernelGGL(kb_grid_clear, dim3(blocks[BK_CLEAR]), T256, 0, s, items, tab, n, n_all);
   hipLaunchKernelGGL(kb_grid_cells, dim3(blocks[BK_LEAVES]), T256, 0, s, items, tab, n, n_all);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  switch ((bvh ? (dyn != 0u ? 2 : 1) : 0)) {
+  switch (bvh) {
+    case 3:
+      hipLaunchKernelGGL(kb_shade<3>, dim3(blocks[BK_SHADE]), T256, dyn, s, items, tab, n, n_all);
+      break;
     case 2:
       hipLaunchKernelGGL(kb_shade<2>, dim3(blocks[BK_SHADE]), T256, dyn, s, items, tab, n, n_all);
       break;

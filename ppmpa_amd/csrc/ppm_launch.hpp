@@ -37,7 +37,8 @@ __host__ __device__ inline uint32_t bvh_dyn_lds(const SceneBuf& b) {
   return small ? BVH_DYN_LDS_BYTES : 0u;
 }
 // The instantiation of a BVH kernel for scene buffers b: 0 no BVH, 1 a large
-// tree (read from global memory only), 2 a small tree with its LDS copies.
+// tree (read from global memory only), 2 a small tree with its LDS copies.  A
+// batch takes the union of its scenes' bits: 3 serves trees of both kinds.
 inline int bvh_kind(const SceneBuf& b) { return b.bvh ? (bvh_dyn_lds(b) != 0u ? 2 : 1) : 0; }
 
 // Photons in regions: region r holds count[r] records starting at
@@ -361,7 +362,7 @@ hipError_t launch_adjoint(hipStream_t s, const SceneBuf& sc, const MapBuf& m, Pa
 // One pass of the first n scenes of a batch (scenes sorted by pass count,
 // so the scenes still running are a prefix); blocks[k] = tab[k*(n_all+1)+n].
 hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
-                             uint32_t n_all, bool bvh, uint32_t dyn);  // dyn: the BVH kernels' dynamic LDS
+                             uint32_t n_all, int bvh, uint32_t dyn);  // bvh: the kernels' BV; dyn: their dynamic LDS
 
 // Test hook: nearest hit of n rays (unit directions).
 hipError_t launch_intersect(hipStream_t s, const SceneBuf& sc, const float4* o, const float4* d, uint32_t n,
