@@ -12,6 +12,10 @@
 #include <cstring>
 #include <string>
 #include <vector>
+#include <atomic>
+#include <condition_variable>
+#include <mutex>
+#include <thread>
 
 #include "../../include/ppm.h"
 #include "ppm_launch.hpp"
@@ -31,6 +35,14 @@ using namespace ppm;
 // work is done), so its sessions and batches may share them.
 constexpr int AUX_PIPE = 0, AUX_CAPTURE = MAX_PIPES - 1, AUX_N = MAX_PIPES;
 
+// Pinned host memory a context keeps for the caller's arrays (stage_out,
+// stage_in), in slots: kernels write some while the host empties others.
+constexpr size_t STAGE_BYTES = 8u << 20;
+constexpr uint32_t STAGE_SLOTS = 8;
+constexpr size_t STAGE_SLOT = STAGE_BYTES / STAGE_SLOTS;
+constexpr size_t STAGE_PAYLOAD = STAGE_SLOT - 256;  // a slot's last 256 bytes hold flags
+constexpr uint32_t STAGE_THREADS = 4;
+
 struct ppm_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -39,15 +51,10 @@ struct ppm_ctx {
   std::string err;
   hipStream_t aux[AUX_N] = {};
   unsigned char* stage = nullptr;      // STAGE_BYTES of pinned host memory (ctx_stage)
-  hipEvent_t stage_ev[2] = {};         // one per half of it
+  hipEvent_t stage_ev[STAGE_SLOTS] = {};  // one per slot of it
   void* work = nullptr;                // the device block calls lay their buffers out in (Work)
   size_t work_bytes = 0;
 };
-
-// Pinned host memory a context keeps for bringing results to the caller's
-// arrays: kernels write one half of it while the host empties the other.
-constexpr size_t STAGE_BYTES = 8u << 20;
-constexpr size_t STAGE_HALF = STAGE_BYTES / 2 - 256;  // payload of a half; its last 256 bytes hold flags
 
 struct ppm_scene {
   ppm_ctx* ctx = nullptr;
@@ -166,6 +173,119 @@ hipError_t ctx_stage(ppm_ctx* c) {
       return e;
     }
   return hipSuccess;
+}
+
+// n results of `item` bytes each to the caller's arrays, a slot at a time:
+// launch(base, count, slot, flags) queues the kernel that writes results
+// [base, base + count) to the slot (and, where there are any, its flags), copy(base,
+// count, slot, flags) then brings them to the caller; false: to be stopped.
+// Slots are filled ahead while others are copied out, and from four slots on
+// by up to STAGE_THREADS threads (not in_order: in any order): one core writes
+// some 10 GB/s, a fifth of what the link brings.  At least one launch, also
+// with n = 0.
+template <typename Launch, typename Copy>
+hipError_t stage_out(ppm_ctx* c, uint64_t n, size_t item, bool in_order, Launch&& launch, Copy&& copy) {
+  hipError_t err = ctx_stage(c);
+  if (err != hipSuccess) return err;
+  const uint64_t per = STAGE_PAYLOAD / item, chunks = std::max<uint64_t>(1, (n + per - 1) / per);
+  auto slot = [&](uint64_t k) { return c->stage + (k % STAGE_SLOTS) * STAGE_SLOT; };
+  auto flags = [&](uint64_t k) { return reinterpret_cast<uint32_t*>(slot(k) + STAGE_PAYLOAD); };
+  auto count = [&](uint64_t k) { return std::min(per, n - k * per); };
+  auto queue = [&](uint64_t k) {
+    const hipError_t e = launch(k * per, count(k), slot(k), flags(k));
+    return e != hipSuccess ? e : hipEventRecord(c->stage_ev[k % STAGE_SLOTS], c->stream);
+  };
+  auto take = [&](uint64_t k) { return copy(k * per, count(k), (const unsigned char*)slot(k), (const uint32_t*)flags(k)); };
+  uint64_t queued = 0;
+  bool stop = false;
+  std::vector<std::thread> helpers;
+  std::mutex mx;
+  std::condition_variable cv;
+  uint64_t taken[STAGE_SLOTS] = {};  // per slot: chunks copied out of it
+  const uint64_t want = in_order ? 1 : std::min<uint64_t>(STAGE_THREADS, chunks / 2);
+  if (want > 1) {
+    auto work = [&](uint64_t t) {
+      (void)hipSetDevice(c->device);
+      for (uint64_t k = t; k < chunks; k += want) {
+        {
+          std::unique_lock<std::mutex> l(mx);
+          cv.wait(l, [&] { return stop || queued > k; });
+          if (stop) return;
+        }
+        const hipError_t e = hipEventSynchronize(c->stage_ev[k % STAGE_SLOTS]);
+        const bool ok = e == hipSuccess && take(k);
+        std::lock_guard<std::mutex> l(mx);
+        if (e != hipSuccess && err == hipSuccess) err = e;
+        if (!ok) stop = true;
+        ++taken[k % STAGE_SLOTS];
+        cv.notify_all();
+        if (!ok) return;
+      }
+    };
+    try {
+      helpers.reserve(want);
+      for (uint64_t t = 0; t < want; ++t) helpers.emplace_back(work, t);
+    } catch (...) {  // no threads to be had: this one copies
+      {
+        std::lock_guard<std::mutex> l(mx);
+        stop = true;
+      }
+      cv.notify_all();
+      for (std::thread& t : helpers) t.join();
+      helpers.clear();
+      stop = false;
+    }
+  }
+  if (!helpers.empty()) {
+    for (uint64_t k = 0; k < chunks; ++k) {
+      {
+        std::unique_lock<std::mutex> l(mx);
+        cv.wait(l, [&] { return stop || taken[k % STAGE_SLOTS] >= k / STAGE_SLOTS; });
+        if (stop) break;
+      }
+      const hipError_t e = queue(k);
+      std::lock_guard<std::mutex> l(mx);
+      if (e != hipSuccess) {
+        if (err == hipSuccess) err = e;
+        stop = true;
+      }
+      queued = k + 1;
+      cv.notify_all();
+      if (stop) break;
+    }
+    for (std::thread& t : helpers) t.join();
+  } else {
+    for (uint64_t k = 0; k < chunks && !stop && err == hipSuccess; ++k) {
+      for (; queued < std::min(chunks, k + STAGE_SLOTS) && err == hipSuccess; ++queued) err = queue(queued);
+      if (err == hipSuccess) err = hipEventSynchronize(c->stage_ev[k % STAGE_SLOTS]);
+      if (err == hipSuccess && !take(k)) stop = true;
+    }
+  }
+  if (stop || err != hipSuccess) {  // queued kernels may still write the staging memory
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (err == hipSuccess) err = e;
+  }
+  return err;
+}
+
+// n items of `item` bytes each to the device, a slot at a time: fill(base,
+// count, slot) writes items [base, base + count) to the slot (false: stop),
+// push(base, count, slot) queues their copies.  The slots are free again on
+// return.
+template <typename Fill, typename Push>
+hipError_t stage_in(ppm_ctx* c, uint64_t n, size_t item, Fill&& fill, Push&& push) {
+  hipError_t err = ctx_stage(c);
+  const uint64_t per = STAGE_PAYLOAD / item, chunks = (n + per - 1) / per;
+  for (uint64_t k = 0; k < chunks && err == hipSuccess; ++k) {
+    hipEvent_t ev = c->stage_ev[k % STAGE_SLOTS];
+    unsigned char* slot = c->stage + (k % STAGE_SLOTS) * STAGE_SLOT;
+    const uint64_t m = std::min(per, n - k * per);
+    if (k >= STAGE_SLOTS) err = hipEventSynchronize(ev);
+    if (err != hipSuccess || !fill(k * per, m, slot)) break;
+    if ((err = push(k * per, m, slot)) == hipSuccess) err = hipEventRecord(ev, c->stream);
+  }
+  const hipError_t e = hipStreamSynchronize(c->stream);
+  return err != hipSuccess ? err : e;
 }
 
 ppm_status fail(ppm_ctx* c, ppm_status s, const std::string& msg) {
@@ -1286,27 +1406,26 @@ ppm_status ppm_photons_download(ppm_ctx* c, const ppm_photons* p, uint64_t cap, 
   *n = cnt;
   if (cnt > cap) return fail(c, PPM_E_RANGE, "output capacity too small");
   if (cnt && (!pos || !dir || !wl)) return fail(c, PPM_E_INVALID, "null output array");
-  std::vector<PhotonRec> recs(cnt);
-  if (cnt) {
-    PhotonRec* dense = nullptr;
-    HIP_TRY(c, dalloc(&dense, cnt));
-    hipError_t e = launch_compact(c->stream, p->pb, p->st, dense);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = hipMemcpy(recs.data(), dense, sizeof(PhotonRec) * cnt, hipMemcpyDeviceToHost);
-    dfree(dense);
-    if (e != hipSuccess) return fail(c, PPM_E_HIP, hipGetErrorString(e));
-  }
-  for (uint64_t i = 0; i < cnt; ++i) {
-    uint32_t m = __builtin_bit_cast(uint32_t, recs[i].pm.w);
-    pos[3 * i] = recs[i].pm.x;
-    pos[3 * i + 1] = recs[i].pm.y;
-    pos[3 * i + 2] = recs[i].pm.z;
-    dir[3 * i] = recs[i].dm.x;
-    dir[3 * i + 1] = recs[i].dm.y;
-    dir[3 * i + 2] = recs[i].dm.z;
-    wl[i] = (uint8_t)(m & 3u);
-    if (meta) meta[i] = m;
-  }
+  if (cnt == 0) return PPM_OK;
+  // a slot holds its photons' positions, directions, meta words and channels,
+  // each as the caller's arrays do
+  HIP_TRY(c, stage_out(
+      c, cnt, 6 * sizeof(double) + sizeof(uint32_t) + 1, false,
+      [&](uint64_t base, uint64_t k, unsigned char* slot, uint32_t*) {
+        double* d = reinterpret_cast<double*>(slot);
+        uint32_t* m = reinterpret_cast<uint32_t*>(d + 6 * k);
+        return launch_photons_out(c->stream, p->pb, (uint32_t)base, (uint32_t)k, d, d + 3 * k, m,
+                                  reinterpret_cast<uint8_t*>(m + k));
+      },
+      [&](uint64_t base, uint64_t k, const unsigned char* slot, const uint32_t*) {
+        const double* d = reinterpret_cast<const double*>(slot);
+        const uint32_t* m = reinterpret_cast<const uint32_t*>(d + 6 * k);
+        std::memcpy(pos + 3 * base, d, 3 * k * sizeof(double));
+        std::memcpy(dir + 3 * base, d + 3 * k, 3 * k * sizeof(double));
+        if (meta) std::memcpy(meta + base, m, k * sizeof(uint32_t));
+        std::memcpy(wl + base, m + k, k);
+        return true;
+      }));
   return PPM_OK;
 }
 
@@ -1417,48 +1536,92 @@ ppm_status ppm_map_build_grid(ppm_ctx* c, const ppm_scene* sc, const ppm_photons
   return PPM_OK;
 }
 
+// n device RGB values to the caller's doubles, times *k in double where given; the
+// overflow flags of st (may be null) to *over, values only when there are none.
+static hipError_t rgb_to_host(ppm_ctx* c, const float4* rgb, uint64_t n, const double* k, const PassState* st,
+                              double* out, uint32_t* over) {
+  std::atomic<uint32_t> seen{0u};
+  const hipError_t e = stage_out(
+      c, n, 3 * sizeof(double), false,
+      [&](uint64_t base, uint64_t m, unsigned char* slot, uint32_t* flags) {
+        return launch_rgb_out(c->stream, rgb + base, (uint32_t)m, k ? *k : 1.0, st, reinterpret_cast<double*>(slot), flags);
+      },
+      [&](uint64_t base, uint64_t m, const unsigned char* slot, const uint32_t* flags) {
+        if (flags[0]) {
+          seen |= flags[0];
+          return false;
+        }
+        std::memcpy(out + 3 * base, slot, 3 * m * sizeof(double));
+        return true;
+      });
+  *over = seen;
+  return e;
+}
+
+// mode 0: the photons in each query's ball counted (counts); 1: their indices
+// (idx_out, from offsets[i] on); 2: their sums, times k (rgb_out).
 static ppm_status run_query(ppm_ctx* c, const ppm_map* m, const double* q_xyz, const double* q_nrm, uint64_t nq,
                             double r2, int refine64, int mode, int pfilter, std::vector<uint32_t>* counts,
-                            const std::vector<uint64_t>* offsets, uint32_t* idx_out, uint64_t idx_total,
-                            std::vector<float4>* rgb) {
-  std::vector<float4> qf(nq), qn;
-  for (uint64_t i = 0; i < nq; ++i) {
-    if (!finite3(q_xyz + 3 * i)) return fail(c, PPM_E_NONFINITE, "non-finite query point");
-    qf[i] = make_float4((float)q_xyz[3 * i], (float)q_xyz[3 * i + 1], (float)q_xyz[3 * i + 2], 0.0f);
-  }
-  if (q_nrm) {
-    qn.resize(nq);
-    for (uint64_t i = 0; i < nq; ++i)
-      qn[i] = make_float4((float)q_nrm[3 * i], (float)q_nrm[3 * i + 1], (float)q_nrm[3 * i + 2], 0.0f);
-  }
+                            const std::vector<uint64_t>* offsets, uint32_t* idx_out, uint64_t idx_total, double k,
+                            double* rgb_out) {
+  Work work;
   float4 *dqf = nullptr, *dqn = nullptr, *drgb = nullptr;
   double* dq64 = nullptr;
   uint32_t *dcnt = nullptr, *didx = nullptr, *dflag = nullptr, hflag = 0;
   uint64_t* doff = nullptr;
+  bool finite = true;
   hipError_t e = hipSuccess;
-  auto cleanup = [&]() {
-    dfree(dqf); dfree(dqn); dfree(drgb); dfree(dq64); dfree(dcnt); dfree(didx); dfree(doff); dfree(dflag);
-  };
   do {
-    if ((e = dalloc(&dqf, nq)) != hipSuccess) break;
-    if ((e = hipMemcpy(dqf, qf.data(), sizeof(float4) * nq, hipMemcpyHostToDevice)) != hipSuccess) break;
-    if (refine64) {
-      if ((e = dalloc(&dq64, 3 * nq)) != hipSuccess) break;
-      if ((e = hipMemcpy(dq64, q_xyz, sizeof(double) * 3 * nq, hipMemcpyHostToDevice)) != hipSuccess) break;
-    }
-    if (q_nrm) {
-      if ((e = dalloc(&dqn, nq)) != hipSuccess) break;
-      if ((e = hipMemcpy(dqn, qn.data(), sizeof(float4) * nq, hipMemcpyHostToDevice)) != hipSuccess) break;
-    }
-    if (mode == 0 && (e = dalloc(&dcnt, nq)) != hipSuccess) break;
-    if (mode == 1) {
-      if ((e = dalloc(&doff, nq)) != hipSuccess) break;
-      if ((e = hipMemcpy(doff, offsets->data(), sizeof(uint64_t) * nq, hipMemcpyHostToDevice)) != hipSuccess) break;
-      if ((e = dalloc(&didx, idx_total)) != hipSuccess) break;
-    }
-    if (mode == 2 && (e = dalloc(&drgb, nq)) != hipSuccess) break;
+    if ((e = work.get(c, [&](Arena& a) {
+           a.take(&dqf, nq);
+           if (refine64) a.take(&dq64, 3 * nq);
+           if (q_nrm) a.take(&dqn, nq);
+           if (mode == 0) a.take(&dcnt, nq);
+           if (mode == 1) {
+             a.take(&doff, nq);
+             a.take(&didx, idx_total);
+           }
+           if (mode == 2) a.take(&drgb, nq);
+           if (m->grid) a.take(&dflag, 1);
+         })) != hipSuccess)
+      break;
+    // a slot: the points in float, then in double and the normals, where used
+    e = stage_in(
+        c, nq, sizeof(float4) * (q_nrm ? 2 : 1) + (refine64 ? 3 * sizeof(double) : 0),
+        [&](uint64_t base, uint64_t n, unsigned char* slot) {
+          float4* f = reinterpret_cast<float4*>(slot);
+          const double* q = q_xyz + 3 * base;
+          for (uint64_t i = 0; i < n; ++i) {
+            if (!finite3(q + 3 * i)) return finite = false;
+            f[i] = make_float4((float)q[3 * i], (float)q[3 * i + 1], (float)q[3 * i + 2], 0.0f);
+          }
+          f += n;
+          if (q_nrm) {
+            const double* v = q_nrm + 3 * base;
+            for (uint64_t i = 0; i < n; ++i)
+              f[i] = make_float4((float)v[3 * i], (float)v[3 * i + 1], (float)v[3 * i + 2], 0.0f);
+            f += n;
+          }
+          if (refine64) std::memcpy(f, q, 3 * n * sizeof(double));
+          return true;
+        },
+        [&](uint64_t base, uint64_t n, const unsigned char* slot) {
+          const float4* f = reinterpret_cast<const float4*>(slot);
+          hipError_t e2 = hipMemcpyAsync(dqf + base, f, sizeof(float4) * n, hipMemcpyHostToDevice, c->stream);
+          f += n;
+          if (q_nrm) {
+            if (e2 == hipSuccess)
+              e2 = hipMemcpyAsync(dqn + base, f, sizeof(float4) * n, hipMemcpyHostToDevice, c->stream);
+            f += n;
+          }
+          if (refine64 && e2 == hipSuccess)
+            e2 = hipMemcpyAsync(dq64 + 3 * base, f, 3 * sizeof(double) * n, hipMemcpyHostToDevice, c->stream);
+          return e2;
+        });
+    if (e != hipSuccess || !finite) break;
+    if (mode == 1 && (e = hipMemcpy(doff, offsets->data(), sizeof(uint64_t) * nq, hipMemcpyHostToDevice)) != hipSuccess)
+      break;
     if (m->grid) {
-      if ((e = dalloc(&dflag, 1)) != hipSuccess) break;
       if ((e = hipMemsetAsync(dflag, 0, sizeof(uint32_t), c->stream)) != hipSuccess) break;
       if ((e = launch_grid_query(c->stream, grid_view_of(m), m->st, m->gbmin, dqf, dq64, (uint32_t)nq, r2, refine64,
                                  mode, dcnt, doff, didx, dflag)) != hipSuccess)
@@ -1468,19 +1631,21 @@ static ppm_status run_query(ppm_ctx* c, const ppm_map* m, const double* q_xyz, c
                                  pfilter, dcnt, doff, didx, drgb, c->n_cu)) != hipSuccess) {
       break;
     }
+    if (mode == 2) {
+      uint32_t over = 0;
+      e = rgb_to_host(c, drgb, nq, &k, nullptr, rgb_out, &over);
+      break;
+    }
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) break;
     if (mode == 0) {
       counts->resize(nq);
       e = hipMemcpy(counts->data(), dcnt, sizeof(uint32_t) * nq, hipMemcpyDeviceToHost);
-    } else if (mode == 1) {
-      if (idx_total) e = hipMemcpy(idx_out, didx, sizeof(uint32_t) * idx_total, hipMemcpyDeviceToHost);
-    } else {
-      rgb->resize(nq);
-      e = hipMemcpy(rgb->data(), drgb, sizeof(float4) * nq, hipMemcpyDeviceToHost);
+    } else if (idx_total) {
+      e = hipMemcpy(idx_out, didx, sizeof(uint32_t) * idx_total, hipMemcpyDeviceToHost);
     }
   } while (0);
-  cleanup();
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
+  if (!finite) return fail(c, PPM_E_NONFINITE, "non-finite query point");
   if (hflag) return fail(c, PPM_E_RANGE, "a query's cells exceed the grid's span");
   return PPM_OK;
 }
@@ -1561,7 +1726,8 @@ ppm_status ppm_radius_query(ppm_ctx* c, const ppm_map* m, const double* q_xyz, u
   offsets_out[0] = 0;
   if (nq == 0) return PPM_OK;
   std::vector<uint32_t> counts;
-  if (ppm_status s = run_query(c, m, q_xyz, nullptr, nq, r2, refine64, 0, 0, &counts, nullptr, nullptr, 0, nullptr))
+  if (ppm_status s = run_query(c, m, q_xyz, nullptr, nq, r2, refine64, 0, 0, &counts, nullptr, nullptr, 0, 1.0,
+                               nullptr))
     return s;
   std::vector<uint64_t> off(nq);
   uint64_t tot = 0;
@@ -1573,7 +1739,8 @@ ppm_status ppm_radius_query(ppm_ctx* c, const ppm_map* m, const double* q_xyz, u
   offsets_out[nq] = tot;
   if (tot > idx_cap) return fail(c, PPM_E_RANGE, "idx_cap too small: need " + std::to_string(tot));
   if (tot && !idx_out) return fail(c, PPM_E_INVALID, "null idx_out");
-  if (ppm_status s = run_query(c, m, q_xyz, nullptr, nq, r2, refine64, 1, 0, nullptr, &off, idx_out, tot, nullptr))
+  if (ppm_status s = run_query(c, m, q_xyz, nullptr, nq, r2, refine64, 1, 0, nullptr, &off, idx_out, tot, 1.0,
+                               nullptr))
     return s;
   for (uint64_t i = 0; i < nq; ++i) std::sort(idx_out + off[i], idx_out + off[i] + counts[i]);
   return PPM_OK;
@@ -1600,17 +1767,9 @@ ppm_status ppm_gather(ppm_ctx* c, const ppm_map* m, const double* q_xyz, const d
   if (ppm_status s = check_gather(c, m, q_xyz, q_nrm, nq, r2, pfilter, refine64, rgb_out)) return s;
   if (nq == 0) return PPM_OK;
   if (m->grid) return run_grid_gather(c, m, q_xyz, q_nrm, nq, r2, pfilter, rgb_out);
-  std::vector<float4> rgb;
-  if (ppm_status s = run_query(c, m, q_xyz, q_nrm, nq, r2, refine64, 2, pfilter, nullptr, nullptr, nullptr, 0, &rgb))
-    return s;
   // tracer.rs:191-193: Σ (wt * power) * max(0, -cos) then * (1/pi / r2)
   const double k = m->power * (1.0 / M_PI) / r2;
-  for (uint64_t i = 0; i < nq; ++i) {
-    rgb_out[3 * i] = (double)rgb[i].x * k;
-    rgb_out[3 * i + 1] = (double)rgb[i].y * k;
-    rgb_out[3 * i + 2] = (double)rgb[i].z * k;
-  }
-  return PPM_OK;
+  return run_query(c, m, q_xyz, q_nrm, nq, r2, refine64, 2, pfilter, nullptr, nullptr, nullptr, 0, k, rgb_out);
 }
 
 static_assert(PPM_NOALLOC_MAX_QUERIES == NOALLOC_MAX_QUERIES, "ppm.h and the kernels disagree on the bound");
@@ -1654,7 +1813,7 @@ ppm_status ppm_trace_eye(ppm_ctx* c, const ppm_scene* sc, const ppm_map* m, uint
   Work work;
   PassState* st = nullptr;
   hipError_t e = hipSuccess;
-  std::vector<float4> h;
+  uint32_t over = 0;
   PassState hs;
   do {
     if ((e = eye_work(c, work, eb, &st, sc->buf.cam, max_depth)) != hipSuccess) break;
@@ -1680,20 +1839,10 @@ ppm_status ppm_trace_eye(ppm_ctx* c, const ppm_scene* sc, const ppm_map* m, uint
     if ((e = launch_gather(c->stream, sb, map_view(m), st, eb, pfilter, use_classic, c->n_cu, nullptr, nullptr)) !=
         hipSuccess)
       break;
-    h.resize(eb.n_pix);
-    if ((e = hipMemcpyAsync(h.data(), eb.pix, sizeof(float4) * eb.n_pix, hipMemcpyDeviceToHost, c->stream)) !=
-        hipSuccess)
-      break;
-    if ((e = hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, c->stream)) != hipSuccess) break;
-    if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) break;
+    e = rgb_to_host(c, eb.pix, eb.n_pix, nullptr, st, rgb_out, &over);
   } while (0);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
-  if (hs.overflow) return fail(c, PPM_E_RANGE, "gather query buffer overflow");
-  for (size_t p = 0; p < h.size(); ++p) {
-    rgb_out[3 * p] = h[p].x;
-    rgb_out[3 * p + 1] = h[p].y;
-    rgb_out[3 * p + 2] = h[p].z;
-  }
+  if (over) return fail(c, PPM_E_RANGE, "gather query buffer overflow");
   return PPM_OK;
 }
 
@@ -1706,7 +1855,7 @@ ppm_status ppm_trace_classic(ppm_ctx* c, const ppm_scene* sc, uint64_t seed, uin
   Work work;
   PassState* st = nullptr;
   hipError_t e = hipSuccess;
-  std::vector<float4> h;
+  uint32_t over = 0;
   PassState hs = host_state();
   do {
     if ((e = eye_work(c, work, eb, &st, sc->buf.cam, CLASSIC_DEPTH)) != hipSuccess) break;
@@ -1714,20 +1863,10 @@ ppm_status ppm_trace_classic(ppm_ctx* c, const ppm_scene* sc, uint64_t seed, uin
     if ((e = hipMemcpy(st, &hs, sizeof(hs), hipMemcpyHostToDevice)) != hipSuccess) break;
     const float4 amb = make_float4((float)ambient[0], (float)ambient[1], (float)ambient[2], 0.0f);
     if ((e = launch_classic(c->stream, sc->buf, st, eb, seed, amb, c->n_cu)) != hipSuccess) break;
-    h.resize(eb.n_pix);
-    if ((e = hipMemcpyAsync(h.data(), eb.pix, sizeof(float4) * eb.n_pix, hipMemcpyDeviceToHost, c->stream)) !=
-        hipSuccess)
-      break;
-    if ((e = hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, c->stream)) != hipSuccess) break;
-    if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) break;
+    e = rgb_to_host(c, eb.pix, eb.n_pix, nullptr, st, rgb_out, &over);
   } while (0);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
-  if (hs.overflow) return fail(c, PPM_E_RANGE, "gather query buffer overflow");
-  for (size_t p = 0; p < h.size(); ++p) {
-    rgb_out[3 * p] = h[p].x;
-    rgb_out[3 * p + 1] = h[p].y;
-    rgb_out[3 * p + 2] = h[p].z;
-  }
+  if (over) return fail(c, PPM_E_RANGE, "gather query buffer overflow");
   return PPM_OK;
 }
 
@@ -1999,17 +2138,15 @@ static hipError_t pipe_states(ppm_session* s, std::vector<PassState>& h) {
   return e;
 }
 
-// Sum over all passes: the pipelines' FP64 sums added in pipeline order.
-static hipError_t merged_sum(ppm_session* s, std::vector<double>& sum) {
-  const uint64_t n3 = 3ull * s->pipes[0].eb.n_pix;
-  sum.assign(n3, 0.0);
-  std::vector<double> a(n3);
-  for (Pipe& p : s->pipes) {
-    const hipError_t e = hipMemcpy(a.data(), p.sum, sizeof(double) * n3, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return e;
-    for (uint64_t i = 0; i < n3; ++i) sum[i] += a[i];
+static ImageSrc image_src(const ppm_session* s) {
+  ImageSrc src;
+  src.n_pipes = (uint32_t)s->pipes.size();
+  for (uint32_t j = 0; j < src.n_pipes; ++j) {
+    src.sum[j] = s->pipes[j].sum;
+    src.sumsq[j] = s->pipes[j].sumsq;
+    src.st[j] = s->pipes[j].st;
   }
-  return hipSuccess;
+  return src;
 }
 
 ppm_status ppm_session_timings(ppm_session* s, ppm_timings* t) {
@@ -2096,15 +2233,24 @@ ppm_status ppm_session_backward(ppm_session* s, const double* grad_image, double
   const uint32_t n_pix = s->pipes[0].eb.n_pix;
   const uint32_t nm = s->sbuf.n_mats;
   // dL/d(pass image) = dL/d(mean image) / K
-  std::vector<float4> g(n_pix);
-  for (uint32_t p = 0; p < n_pix; ++p) {
-    const double* v = grad_image + 3ull * p;
-    if (!finite3(v)) return fail(c, PPM_E_NONFINITE, "non-finite image gradient");
-    g[p] = make_float4((float)(v[0] / K), (float)(v[1] / K), (float)(v[2] / K), 0.0f);
-  }
   if (!s->gimg) HIP_TRY(c, dalloc(&s->gimg, n_pix));
   if (!s->grad) HIP_TRY(c, dalloc(&s->grad, 3ull * nm));
-  HIP_TRY(c, hipMemcpy(s->gimg, g.data(), sizeof(float4) * n_pix, hipMemcpyHostToDevice));
+  bool finite = true;
+  HIP_TRY(c, stage_in(
+      c, n_pix, sizeof(float4),
+      [&](uint64_t base, uint64_t n, unsigned char* slot) {
+        float4* g = reinterpret_cast<float4*>(slot);
+        for (uint64_t i = 0; i < n; ++i) {
+          const double* v = grad_image + 3ull * (base + i);
+          if (!finite3(v)) return finite = false;
+          g[i] = make_float4((float)(v[0] / K), (float)(v[1] / K), (float)(v[2] / K), 0.0f);
+        }
+        return true;
+      },
+      [&](uint64_t base, uint64_t n, const unsigned char* slot) {
+        return hipMemcpyAsync(s->gimg + base, slot, sizeof(float4) * n, hipMemcpyHostToDevice, c->stream);
+      }));
+  if (!finite) return fail(c, PPM_E_NONFINITE, "non-finite image gradient");
   HIP_TRY(c, hipMemset(s->grad, 0, sizeof(double) * 3 * nm));
   const float4 bmin = make_float4((float)sc->bmin[0], (float)sc->bmin[1], (float)sc->bmin[2], 0.f);
   const float4 bmax = make_float4((float)sc->bmax[0], (float)sc->bmax[1], (float)sc->bmax[2], 0.f);
@@ -2150,10 +2296,18 @@ ppm_status ppm_session_backward(ppm_session* s, const double* grad_image, double
   for (size_t i = 0; i < hg.size(); ++i) grad_albedo[i] = hg[i];
   if (grad_light) {
     // the image is proportional to the light scale: dL/ds = sum g * mean / s
-    std::vector<double> sum;
-    HIP_TRY(c, merged_sum(s, sum));
+    const ImageSrc src = image_src(s);
     double acc = 0.0;
-    for (size_t i = 0; i < sum.size(); ++i) acc += grad_image[i] * (sum[i] / K);
+    HIP_TRY(c, stage_out(
+        c, 3ull * n_pix, sizeof(double), true,
+        [&](uint64_t base, uint64_t n, unsigned char* slot, uint32_t* flags) {
+          return launch_image(c->stream, src, base, (uint32_t)n, K, reinterpret_cast<double*>(slot), nullptr, flags);
+        },
+        [&](uint64_t base, uint64_t n, const unsigned char* slot, const uint32_t*) {
+          const double* mean = reinterpret_cast<const double*>(slot);
+          for (uint64_t i = 0; i < n; ++i) acc += grad_image[base + i] * mean[i];
+          return true;
+        }));
     *grad_light = sc->light_scale > 0.0 ? acc / sc->light_scale : 0.0;
   }
   return PPM_OK;
@@ -2174,46 +2328,30 @@ ppm_status ppm_session_image(ppm_session* s, double* mean_out, double* var_out, 
   if (!s) return PPM_E_INVALID;
   ppm_ctx* c = s->ctx;
   if (passes_done) *passes_done = s->passes_done;
-  HIP_TRY(c, ctx_stage(c));
-  ImageSrc src;
-  src.n_pipes = (uint32_t)s->pipes.size();
-  for (uint32_t j = 0; j < src.n_pipes; ++j) {
-    src.sum[j] = s->pipes[j].sum;
-    src.sumsq[j] = s->pipes[j].sumsq;
-    src.st[j] = s->pipes[j].st;
-  }
-  // chunks of the image alternate between the halves of the staging memory:
-  // k_image writes one while the other is copied out
+  const ImageSrc src = image_src(s);
   const uint64_t n3 = 3ull * s->pipes[0].eb.n_pix;
   const uint32_t outs = (mean_out ? 1u : 0u) + (var_out ? 1u : 0u);
-  const uint64_t per = outs ? STAGE_HALF / (sizeof(double) * outs) : n3;
-  const uint64_t chunks = outs ? (n3 + per - 1) / per : 1;
-  auto half = [&](uint64_t k) { return c->stage + (k & 1u) * (STAGE_BYTES / 2); };
-  auto flags = [&](uint64_t k) { return reinterpret_cast<uint32_t*>(half(k) + STAGE_HALF); };
-  auto queue = [&](uint64_t k) -> hipError_t {
-    double* d = reinterpret_cast<double*>(half(k));
-    const uint64_t n = outs ? std::min(per, n3 - k * per) : 0;
-    const hipError_t e = launch_image(c->stream, src, k * per, (uint32_t)n, s->passes_done, mean_out ? d : nullptr,
-                                      var_out ? d + (mean_out ? n : 0) : nullptr, flags(k));
-    return e != hipSuccess ? e : hipEventRecord(c->stage_ev[k & 1u], c->stream);
-  };
-  HIP_TRY(c, queue(0));
-  for (uint64_t k = 0; k < chunks; ++k) {
-    if (k + 1 < chunks) HIP_TRY(c, queue(k + 1));
-    hipError_t e = hipEventSynchronize(c->stage_ev[k & 1u]);
-    const uint32_t over = e == hipSuccess ? flags(k)[0] : 0u, bad = e == hipSuccess ? flags(k)[1] : 0u;
-    if (e != hipSuccess || over || bad) {
-      const hipError_t e2 = hipStreamSynchronize(c->stream);  // the queued chunk still writes the staging memory
-      if (e == hipSuccess) e = e2;
-      HIP_TRY(c, e);
-      if (over) return fail(c, PPM_E_RANGE, "capacity exceeded during a pass: " + overflow_text(over));
-      return fail(c, PPM_E_NONFINITE, "non-finite photon position (photonmap.rs:26)");
-    }
-    const double* d = reinterpret_cast<const double*>(half(k));
-    const uint64_t n = outs ? std::min(per, n3 - k * per) : 0;
-    if (mean_out) std::memcpy(mean_out + k * per, d, n * sizeof(double));
-    if (var_out) std::memcpy(var_out + k * per, d + (mean_out ? n : 0), n * sizeof(double));
-  }
+  std::atomic<uint32_t> over{0u}, bad{0u};
+  HIP_TRY(c, stage_out(
+      c, outs ? n3 : 0, sizeof(double) * std::max(1u, outs), false,
+      [&](uint64_t base, uint64_t n, unsigned char* slot, uint32_t* flags) {
+        double* d = reinterpret_cast<double*>(slot);
+        return launch_image(c->stream, src, base, (uint32_t)n, s->passes_done, mean_out ? d : nullptr,
+                            var_out ? d + (mean_out ? n : 0) : nullptr, flags);
+      },
+      [&](uint64_t base, uint64_t n, const unsigned char* slot, const uint32_t* flags) {
+        if (flags[0] || flags[1]) {
+          over |= flags[0];
+          bad |= flags[1];
+          return false;
+        }
+        const double* d = reinterpret_cast<const double*>(slot);
+        if (mean_out) std::memcpy(mean_out + base, d, n * sizeof(double));
+        if (var_out) std::memcpy(var_out + base, d + (mean_out ? n : 0), n * sizeof(double));
+        return true;
+      }));
+  if (over) return fail(c, PPM_E_RANGE, "capacity exceeded during a pass: " + overflow_text(over));
+  if (bad) return fail(c, PPM_E_NONFINITE, "non-finite photon position (photonmap.rs:26)");
   return PPM_OK;
 }
 

@@ -179,7 +179,8 @@ uint32_t trace_waves(uint64_t n_photon, int n_cu);
 
 hipError_t launch_trace_photons(hipStream_t s, const SceneBuf& sc, PassState* st, PhotonBuf& pb, uint64_t seed,
                                 int use_classic, int max_depth);
-hipError_t launch_compact(hipStream_t s, const PhotonBuf& pb, const PassState* st, PhotonRec* dense);
+hipError_t launch_photons_out(hipStream_t s, const PhotonBuf& pb, uint32_t base, uint32_t n, double* pos, double* dir,
+                              uint32_t* meta, uint8_t* wl);
 
 hipError_t launch_map_build(hipStream_t s, MapBuf& m, PassState* st, const PhotonBuf& in, float4 bmin, float4 bmax);
 
@@ -308,6 +309,8 @@ struct ImageSrc {
   const PassState* st[MAX_PIPES] = {};
   uint32_t n_pipes = 0;
 };
+hipError_t launch_rgb_out(hipStream_t s, const float4* rgb, uint32_t n, double k, const PassState* st, double* out,
+                          uint32_t* flags);
 hipError_t launch_image(hipStream_t s, const ImageSrc& src, uint64_t base, uint32_t n, uint32_t passes, double* mean,
                         double* var, uint32_t* flags);
 
