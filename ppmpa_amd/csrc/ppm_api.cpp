@@ -512,22 +512,46 @@ uint32_t cam_tiles_max(const DevCamera& cam) {
   return m;
 }
 
+// The parts (1 << the result) that the eye waves take a tile of 64 pixels in.  A
+// wave holds a tile until its deepest path is done, and behind glass a pixel's
+// tree has dozens of nodes: with few tiles the last waves set the eye's time,
+// and a part's trees are shared by all 64 lanes all the same.  Whole tiles issue
+// the fewest instructions, which is what counts once there are enough of them,
+// and where no path branches there is nothing to share.  Times of whole tiles /
+// halves / quarters, in ms:
+//   160x120, glass sphere: eye alone 0.122 / 0.067 / 0.062
+//   256x256, rough glass: eye 0.157 / 0.101 / 0.071, eight passes 1.62 / 1.49 / 1.46
+//   512x512, 40 shapes: eye 0.558 / 0.341 / 0.428
+//   640x400, 300 spheres: eye 2.08 / 1.32 / 1.05, eight passes 15.4 / 14.4 / 14.7
+//   640x400, 20k triangles: eye 3.35 / 1.83 / 1.13, eight passes 27.4 / 24.0 / 22.6
+//   1024x768, glass sphere: 64 passes 41.1 / 42.3 / 47.3
+//   1920x1080, 327k triangles: four passes 132.6 / 129.9 / 131.8
+//   256x256, a mirror sphere: 16 passes 2.06 / 2.13 / 2.16
+//   24 rooms of 128^2-512^2 in one batch: four rounds 41.4 / 41.7 / 43.9
+uint32_t eye_part_shift(const SceneBuf& sc, uint32_t tiles) {
+  if (!sc.branches) return 0;
+  const bool few = tiles <= 8192u;
+  // by the shapes, not the tree: with and without a tree an image is the same
+  return sc.n_shapes > BVH_SMALL_PRIMS ? (few ? 2 : 1) : (few ? 1 : 0);
+}
+
 // The eye buffers at tile shape `shift` (sized for any shape by eye_alloc);
 // the tiles' query counts of earlier passes, which only order the eye's
 // work, start again from zero.
-bool eye_tiles(EyeBuf& eb, DevCamera& cam, uint32_t shift) {
+bool eye_tiles(EyeBuf& eb, const SceneBuf& sc, DevCamera& cam, uint32_t shift) {
   uint32_t tx = 0;
   const uint32_t tiles = cam_tiles(cam, shift, &tx);
   if (tiles > eb.tiles_cap) return false;
   cam.tile_shift = (int32_t)shift;
   cam.tiles_x = (int32_t)tx;
   eb.n_tiles = tiles;
+  eb.part_shift = eye_part_shift(sc, tiles);
   eb.q_primary = tiles * 64u;
   eb.q_fine = eb.q_primary >= QUERY_FINE_PIXELS ? 1u : 0u;
   return true;
 }
-hipError_t eye_set_tiles(EyeBuf& eb, DevCamera& cam, uint32_t shift) {
-  if (!eye_tiles(eb, cam, shift)) return hipErrorInvalidValue;
+hipError_t eye_set_tiles(EyeBuf& eb, const SceneBuf& sc, DevCamera& cam, uint32_t shift) {
+  if (!eye_tiles(eb, sc, cam, shift)) return hipErrorInvalidValue;
   return hipMemset(eb.tile_count, 0, sizeof(uint32_t) * eb.tiles_cap);
 }
 
@@ -548,7 +572,7 @@ void eye_layout(Arena& a, EyeBuf& eb, const DevCamera& cam, int max_depth, int n
   eb.n_pix = (uint32_t)cam.xreso * (uint32_t)cam.yreso;
   eb.ovf_cap = 2u * eb.n_pix + 1024u;
   const uint64_t slots = (uint64_t)eb.q_primary * (1u + eb.sec_max) + eb.ovf_cap;
-  eb.estack_lanes = 64u * std::max<uint32_t>(1, std::min<uint32_t>(tiles, (uint32_t)n_cu * EYE_WAVES_PER_CU_MAX));
+  eb.estack_lanes = 64u * std::max<uint32_t>(1, std::min<uint32_t>(4u * tiles, (uint32_t)n_cu * EYE_WAVES_PER_CU_MAX));
   eb.estack_depth = (uint32_t)std::max(1, std::min(max_depth, MAX_DEPTH_LIMIT));
   a.take(&eb.q, slots);
   a.take(&eb.sec_count, eb.q_primary);
@@ -578,14 +602,14 @@ void eye_layout(Arena& a, EyeBuf& eb, const DevCamera& cam, int max_depth, int n
 }
 
 // The eye's buffers alone and a pass state (one pass outside a session).
-hipError_t eye_work(ppm_ctx* c, Work& w, EyeBuf& eb, PassState** st, const DevCamera& cam, int max_depth) {
+hipError_t eye_work(ppm_ctx* c, Work& w, EyeBuf& eb, PassState** st, const SceneBuf& sc, int max_depth) {
   const hipError_t e = w.get(c, [&](Arena& a) {
     a.take(st, 1);
-    eye_layout(a, eb, cam, max_depth, c->n_cu, nullptr, 0, 0);
+    eye_layout(a, eb, sc.cam, max_depth, c->n_cu, nullptr, 0, 0);
   });
   if (e != hipSuccess) return e;
-  DevCamera cm = cam;
-  return eye_set_tiles(eb, cm, (uint32_t)cam.tile_shift);
+  DevCamera cm = sc.cam;
+  return eye_set_tiles(eb, sc, cm, (uint32_t)cm.tile_shift);
 }
 
 // What the overflow flags of a pass state say (device-side bits 1 photon
@@ -1093,6 +1117,13 @@ ppm_status ppm_scene_create(ppm_ctx* c, const ppm_scene_desc* d, ppm_scene** out
   b.n_shapes = (uint32_t)d->n_shapes;
   b.n_mats = (uint32_t)d->n_materials;
   b.n_lights = (uint32_t)d->n_lights;
+  for (const DevShape& x : shapes) {
+    const DevMaterial& m = mats[x.mat];
+    const bool clear = m.c2.x == 1.0f && m.c2.y == 1.0f && m.c2.z == 1.0f;
+    if (m.diff != 1.0f && m.metal != 1.0f && m.ior_avg != 0.0f && !clear &&
+        (m.surface == SURF_SIMPLE || m.surface == SURF_TS))
+      b.branches = 1;
+  }
   const ppm_camera_desc& cd = d->camera;
   DevCamera& cam = b.cam;
   std::memset(&cam, 0, sizeof(cam));
@@ -1816,7 +1847,7 @@ ppm_status ppm_trace_eye(ppm_ctx* c, const ppm_scene* sc, const ppm_map* m, uint
   uint32_t over = 0;
   PassState hs;
   do {
-    if ((e = eye_work(c, work, eb, &st, sc->buf.cam, max_depth)) != hipSuccess) break;
+    if ((e = eye_work(c, work, eb, &st, sc->buf, max_depth)) != hipSuccess) break;
     if ((e = hipMemcpyAsync(&hs, m->st, sizeof(PassState), hipMemcpyDeviceToHost, c->stream)) != hipSuccess) break;
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) break;
     hs.pass = pass;
@@ -1858,7 +1889,7 @@ ppm_status ppm_trace_classic(ppm_ctx* c, const ppm_scene* sc, uint64_t seed, uin
   uint32_t over = 0;
   PassState hs = host_state();
   do {
-    if ((e = eye_work(c, work, eb, &st, sc->buf.cam, CLASSIC_DEPTH)) != hipSuccess) break;
+    if ((e = eye_work(c, work, eb, &st, sc->buf, CLASSIC_DEPTH)) != hipSuccess) break;
     hs.pass = pass;
     if ((e = hipMemcpy(st, &hs, sizeof(hs), hipMemcpyHostToDevice)) != hipSuccess) break;
     const float4 amb = make_float4((float)ambient[0], (float)ambient[1], (float)ambient[2], 0.0f);
@@ -1995,7 +2026,7 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
     s->lights_host = L;
     for (size_t j = 0; j < s->pipes.size(); ++j) {
       Pipe& p = s->pipes[j];
-      eye_tiles(p.eb, s->sbuf.cam, (uint32_t)sc->buf.cam.tile_shift);
+      eye_tiles(p.eb, s->sbuf, s->sbuf.cam, (uint32_t)sc->buf.cam.tile_shift);
       p.stream = j == 0 || !own_streams ? c->stream : c->aux[AUX_PIPE + j - 1];
       if (own_streams && (e = hipEventCreateWithFlags(&p.done, hipEventDisableTiming)) != hipSuccess) break;
     }
@@ -2208,7 +2239,7 @@ static hipError_t session_set_tiles(ppm_session* s, uint32_t shift) {
     if (p.stream && (e = hipStreamSynchronize(p.stream)) != hipSuccess) return e;
   }
   for (Pipe& p : s->pipes) {
-    const hipError_t e = eye_set_tiles(p.eb, s->sbuf.cam, shift);
+    const hipError_t e = eye_set_tiles(p.eb, s->sbuf, s->sbuf.cam, shift);
     if (e != hipSuccess) return e;
     pipe_drop_graph(p);
   }
@@ -2427,7 +2458,7 @@ hipError_t batch_layout(ppm_batch* b) {
     it.maxd = s->cfg.max_depth;
     it.pfilter = s->cfg.pfilter;
     it.trace_per_wave = (uint32_t)(((uint64_t)s->sbuf.n_emit_total + it.pb.n_regions - 1) / it.pb.n_regions);
-    it.eye_waves = std::max(1u, std::min(std::min(it.eb.n_tiles, n_cu * ew), it.eb.estack_lanes / 64u));
+    it.eye_waves = std::max(1u, std::min(std::min(it.eb.n_tiles << it.eb.part_shift, n_cu * ew), it.eb.estack_lanes / 64u));
     // the sorts' blocks from the expected key counts (about 2 stored photons
     // per emitted one, 1.5 queries per pixel): the histogram blocks stride
     // and the digit passes' persistent blocks take tiles until none is left,

@@ -1782,9 +1782,10 @@ __device__ __forceinline__ uint64_t peer_mask(uint32_t key, bool pred) {
   return m;
 }
 
-// Persistent eye kernel.  A wave takes tiles in the order of tile_order from
-// the pass's work counters and walks the eye trees of a tile's 64 pixels (one per
-// lane to start with) together: each loop step processes one node per busy
+// Persistent eye kernel.  A wave takes tiles (or parts of them, eb.part_shift:
+// eye_part_shift on the host) in the order of tile_order from the pass's work
+// counters and walks the eye trees of their pixels (one per lane to start with;
+// a tile has 64) together: each loop step processes one node per busy
 // lane; a node with both a reflection and a refraction child continues with
 // the reflection and puts the refraction child on the wave's pending pool
 // (LIFO, in global memory), and idle lanes take the newest pool entries, so
@@ -1825,13 +1826,16 @@ __device__ __forceinline__ void k_eye_body(SceneView sc, PassState* st, EyeBuf e
   const uint32_t tx = (uint32_t)sc.cam.tiles_x;
   const uint32_t ts = (uint32_t)sc.cam.tile_shift, tm = (1u << ts) - 1u;  // tile width 1 << ts
   uint32_t wc = w & 7u, wtries = 0;
-  for (uint32_t k = wave_next8(st->work[WORK_EYE], wc, wtries, eb.n_tiles); k < eb.n_tiles;
-       k = wave_next8(st->work[WORK_EYE], wc, wtries, eb.n_tiles)) {
-    const uint32_t tile = eb.tile_order[k];
+  const uint32_t items = eb.n_tiles << eb.part_shift, part_lanes = 64u >> eb.part_shift;
+  for (uint32_t k = wave_next8(st->work[WORK_EYE], wc, wtries, items); k < items;
+       k = wave_next8(st->work[WORK_EYE], wc, wtries, items)) {
+    const uint32_t tile = eb.tile_order[k >> eb.part_shift];
+    const uint32_t part = k & ((1u << eb.part_shift) - 1u);
     const uint32_t x0 = (tile % tx) << ts, y0 = (tile / tx) << (6u - ts);
     const uint32_t t = tile * 64u + lane;
     const int x = (int)(x0 + (lane & tm)), y = (int)(y0 + (lane >> ts));
-    const bool inside = x < sc.cam.xreso && y < sc.cam.yreso;
+    const bool mine = lane / part_lanes == part;  // the lane's pixel is of the wave's part of the tile
+    const bool inside = mine && x < sc.cam.xreso && y < sc.cam.yreso;
     const uint32_t my_pixel = inside ? (uint32_t)y * (uint32_t)sc.cam.xreso + (uint32_t)x : 0u;
     nsec[lane] = 0u;
     acc3[3u * lane] = 0.0f;
@@ -2030,7 +2034,7 @@ __device__ __forceinline__ void k_eye_body(SceneView sc, PassState* st, EyeBuf e
     // the tile is done: each lane writes its pixel's emitted radiance and
     // in-place query count
     if (inside) eb.pix[my_pixel] = make_float4(acc3[3u * lane], acc3[3u * lane + 1u], acc3[3u * lane + 2u], 0.0f);
-    eb.sec_count[t] = inside ? nsec[lane] | (prim ? SEC_PRIMARY : 0u) : 0u;
+    if (mine) eb.sec_count[t] = inside ? nsec[lane] | (prim ? SEC_PRIMARY : 0u) : 0u;
   }
 }
 
@@ -2071,7 +2075,7 @@ hipError_t launch_eye(hipStream_t s, const SceneBuf& sc, PassState* st, const Ey
   // and the other pipeline's kernels (16 per CU filled every slot: caustic
   // 0.855 -> 0.816 ms per pass, mesh 95.6 -> 87.8 ms; 4 and 8: 0.815-0.834
   // and 90.6-94.5 ms)
-  uint32_t n_waves = std::min<uint32_t>(std::min<uint32_t>(eb.n_tiles, (uint32_t)n_cu * EYE_WAVES_PER_CU), eb.estack_lanes / 64u);
+  uint32_t n_waves = std::min<uint32_t>(std::min<uint32_t>(eb.n_tiles << eb.part_shift, (uint32_t)n_cu * EYE_WAVES_PER_CU), eb.estack_lanes / 64u);
   if (n_waves < 1) n_waves = 1;
   const uint32_t blocks = (n_waves + 3) / 4;
   switch (bvh_kind(sc)) {
@@ -2702,7 +2706,7 @@ __global__ __launch_bounds__(256) void k_shade_classic(SceneView sc, const PassS
 hipError_t launch_classic(hipStream_t s, const SceneBuf& sc, PassState* st, const EyeBuf& eb, uint64_t seed,
                           float4 ambient, int n_cu) {
   hipLaunchKernelGGL(k_tile_order, dim3((eb.n_tiles + 255) / 256), dim3(256), 0, s, eb, st);
-  uint32_t n_waves = std::min<uint32_t>(std::min<uint32_t>(eb.n_tiles, (uint32_t)n_cu * EYE_WAVES_PER_CU), eb.estack_lanes / 64u);
+  uint32_t n_waves = std::min<uint32_t>(std::min<uint32_t>(eb.n_tiles << eb.part_shift, (uint32_t)n_cu * EYE_WAVES_PER_CU), eb.estack_lanes / 64u);
   if (n_waves < 1) n_waves = 1;
   const uint32_t blocks = (n_waves + 3) / 4;
   const SceneView v = make_view(sc);

@@ -22,6 +22,7 @@ struct SceneBuf {
   uint32_t n_lin = 0, n_bprims = 0, bvh_depth = 0;
   uint32_t bvh_leaf = 1;        // primitives per BVH leaf
   uint32_t n_shapes = 0, n_mats = 0, n_lights = 0;
+  uint32_t branches = 0;        // 1: some shape both reflects and transmits (eye paths branch)
   uint32_t n_emit_total = 0;  // photons per pass over all lights
   DevCamera cam{};
   float4 bmin{}, bmax{};
@@ -122,6 +123,7 @@ struct EyeBuf {
   float4* pix = nullptr;  // per-pixel float radiance of the pass (row-major)
   uint32_t n_pix = 0;
   uint32_t n_tiles = 0;
+  uint32_t part_shift = 0; // the eye waves take a tile in 1 << part_shift parts
   uint32_t tiles_cap = 0;  // the buffers hold the tiles of any tile shape
   uint32_t* tile_count = nullptr;   // queries per tile (of the last pass until k_tile_count)
   uint32_t* tile_off = nullptr;
