@@ -2062,24 +2062,24 @@ static hipError_t enqueue_pass(ppm_session* s, uint32_t j, hipStream_t st, hipEv
   const int n_cu = s->ctx->n_cu;
   const uint32_t K = (uint32_t)s->pipes.size();
   auto mark = [&](int k) { return ev ? hipEventRecord(ev[k], st) : hipSuccess; };
+  const PassBegin begin{cfg.first_pass + j, K, cfg.radius0 * cfg.radius0, cfg.alpha};
   auto eye = [&] {
-    return launch_eye(st, s->sbuf, p.st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, n_cu);
+    return launch_eye(st, s->sbuf, p.st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, n_cu, ev ? PassBegin{} : begin);
   };
   auto order = [&] { return launch_query_prep(st, s->sbuf, p.map, p.st, p.eb); };
   if ((e = mark(0)) != hipSuccess) return e;
-  if ((e = launch_pass_begin(st, p.st, cfg.first_pass + j, cfg.radius0 * cfg.radius0, cfg.alpha, K)) != hipSuccess)
-    return e;
+  if (ev && (e = launch_pass_begin(st, p.st, begin.first_pass, begin.r2_first, begin.alpha, K)) != hipSuccess) return e;
   if (!ev && ((e = eye()) != hipSuccess || (e = order()) != hipSuccess)) return e;
-  if ((e = launch_trace_photons(st, s->sbuf, p.st, p.pb, cfg.seed, cfg.use_classic, cfg.max_depth)) != hipSuccess)
+  if ((e = launch_trace_photons(st, s->sbuf, p.st, p.pb, cfg.seed, cfg.use_classic, cfg.max_depth, false)) != hipSuccess)
     return e;
   if ((e = mark(1)) != hipSuccess) return e;
-  if ((e = launch_grid_build(st, p.map, p.st, p.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total)) != hipSuccess) return e;
+  if ((e = launch_grid_build(st, p.map, p.st, p.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total, true)) != hipSuccess)
+    return e;
   if ((e = mark(2)) != hipSuccess) return e;
   if (ev && ((e = eye()) != hipSuccess || (e = mark(3)) != hipSuccess || (e = order()) != hipSuccess)) return e;
   if ((e = launch_gather(st, s->sbuf, p.map, p.st, p.eb, cfg.pfilter, cfg.use_classic, n_cu, p.sum, p.sumsq,
-                         ev ? ev + 4 : nullptr, true)) != hipSuccess)
+                         ev ? ev + 4 : nullptr, true, true)) != hipSuccess)
     return e;
-  if ((e = launch_pass_end(st, p.st)) != hipSuccess) return e;
   return mark(6);
 }
 
@@ -2304,18 +2304,19 @@ ppm_status ppm_session_backward(ppm_session* s, const double* grad_image, double
     // the adjoint's scratch: the photon sort's keys, done with by then
     float* adj_sorted = reinterpret_cast<float*>(p.map.keys[0]);
     float* adj_slot = reinterpret_cast<float*>(p.map.keys[1]);
-    if ((e = launch_pass_begin(q, st, cfg.first_pass + j, cfg.radius0 * cfg.radius0, cfg.alpha, NP)) != hipSuccess) break;
-    if ((e = launch_eye(q, s->sbuf, st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, c->n_cu)) != hipSuccess) break;
+    if ((e = launch_eye(q, s->sbuf, st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, c->n_cu,
+                        PassBegin{cfg.first_pass + j, NP, cfg.radius0 * cfg.radius0, cfg.alpha})) != hipSuccess)
+      break;
     if ((e = launch_query_prep(q, s->sbuf, p.map, st, p.eb)) != hipSuccess) break;
-    if ((e = launch_trace_photons(q, s->sbuf, st, p.pb, cfg.seed, cfg.use_classic, cfg.max_depth)) != hipSuccess) break;
-    if ((e = launch_grid_build(q, p.map, st, p.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total)) != hipSuccess) break;
+    if ((e = launch_trace_photons(q, s->sbuf, st, p.pb, cfg.seed, cfg.use_classic, cfg.max_depth, false)) != hipSuccess)
+      break;
+    if ((e = launch_grid_build(q, p.map, st, p.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total, true)) != hipSuccess)
+      break;
     if ((e = launch_gather(q, s->sbuf, p.map, st, p.eb, cfg.pfilter, cfg.use_classic, c->n_cu, nullptr, nullptr,
-                           nullptr, true)) != hipSuccess)
+                           nullptr, true, true)) != hipSuccess)
       break;
-    if ((e = launch_adjoint(q, s->sbuf, p.map, st, p.pb, p.eb, cfg.pfilter, c->n_cu, cfg.seed, cfg.use_classic,
-                            cfg.max_depth, s->gimg, adj_sorted, adj_slot, s->grad)) != hipSuccess)
-      break;
-    e = launch_pass_end(q, st);
+    e = launch_adjoint(q, s->sbuf, p.map, st, p.pb, p.eb, cfg.pfilter, c->n_cu, cfg.seed, cfg.use_classic,
+                            cfg.max_depth, s->gimg, adj_sorted, adj_slot, s->grad);
   }
   for (uint32_t j = 0; j < NP; ++j) {  // also after an error: nothing keeps running on the buffers
     const hipError_t e2 = hipStreamSynchronize(s->pipes[j].stream);

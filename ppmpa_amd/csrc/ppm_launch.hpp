@@ -174,13 +174,18 @@ hipError_t launch_pipes_init(hipStream_t s, const PipesInit& in);
 // The photon power is in the state already.
 hipError_t launch_pass_begin(hipStream_t s, PassState* st, uint32_t first_pass, double r2_first, double alpha,
                              uint32_t stride);
-hipError_t launch_pass_end(hipStream_t s, PassState* st);
+// The same, with another launch (launch_eye); stride 0: nothing to begin.
+struct PassBegin {
+  uint32_t first_pass = 0, stride = 0;
+  double r2_first = 0.0, alpha = 0.0;
+};
 
 // Number of tracing waves (= photon regions) used for n photons.
 uint32_t trace_waves(uint64_t n_photon, int n_cu);
 
+// scan: also the offsets of the regions' records (else launch_grid_build's)
 hipError_t launch_trace_photons(hipStream_t s, const SceneBuf& sc, PassState* st, PhotonBuf& pb, uint64_t seed,
-                                int use_classic, int max_depth);
+                                int use_classic, int max_depth, bool scan = true);
 hipError_t launch_photons_out(hipStream_t s, const PhotonBuf& pb, uint32_t base, uint32_t n, double* pos, double* dir,
                               uint32_t* meta, uint8_t* wl);
 
@@ -231,10 +236,10 @@ inline uint64_t next_pow2_u64(uint64_t v) {
 // expect: the photons the pass is expected to store, which sizes the grid
 // kernels (0: the set's capacity).
 hipError_t launch_grid_build(hipStream_t s, MapBuf& m, PassState* st, const PhotonBuf& in, float4 bmin, float4 bmax,
-                             uint64_t expect = 0);
+                             uint64_t expect = 0, bool scan = false);
 
 hipError_t launch_eye(hipStream_t s, const SceneBuf& sc, PassState* st, const EyeBuf& eb, uint64_t seed,
-                      int use_classic, int max_depth, int n_cu);
+                      int use_classic, int max_depth, int n_cu, const PassBegin& begin = PassBegin{});
 // One pass of the classic ray tracer (trace_ray_classic) into eb.pix:
 // k_eye_classic, the query sort, k_shade_classic (direct light + ambient),
 // the overflow queries and the per-pixel sum.
@@ -252,7 +257,7 @@ hipError_t launch_query_prep(hipStream_t s, const SceneBuf& sc, const MapBuf& m,
 // pix.  ev (optional, 2 events) brackets the k_shade launch alone.
 hipError_t launch_gather(hipStream_t s, const SceneBuf& sc, const MapBuf& m, PassState* st, const EyeBuf& eb,
                          int pfilter, int use_classic, int n_cu, double* sum, double* sumsq,
-                         hipEvent_t* ev = nullptr, bool prepared = false);
+                         hipEvent_t* ev = nullptr, bool prepared = false, bool end = false);  // end: of the pass
 
 // Test hooks (radius query / gather on host-provided query points).
 // mode 0: count, 1: list, 2: gather rgb
