@@ -2124,6 +2124,14 @@ __device__ __forceinline__ void quad_photons(float vr, float vg, float vb, float
   quad_photon<2>(vr, vg, vb, ar, ag, ab);
   quad_photon<3>(vr, vg, vb, ar, ag, ab);
 }
+// The sums of the quad's four lanes, in their order, where each lane has summed
+// its own photons: the shading's way, whose pixels are floats.  There the ordered
+// sum took 12 of some 35 instructions per photon (eye pass over 0.43M photons:
+// the shade alone 0.92 -> 0.81 ms).  Radiance estimates, which callers get as
+// doubles, keep the photons' order.
+__device__ __forceinline__ float quad_sum(float v) {
+  return ((quad_get<0>(v) + quad_get<1>(v)) + quad_get<2>(v)) + quad_get<3>(v);
+}
 
 // ===========================================================================
 // Radius query over the heap-ordered tree, one query per lane: the photons of
@@ -2381,9 +2389,11 @@ __device__ __forceinline__ void k_shade_tree_body(SceneView sc, const Node* node
       const float c = photon_cos(nx, ny, nz, dm);  // optics.rs:225
       const float v = (valid && d2 <= r2 && c < 0.0f) ? -c * filter_weight(pf, d2 * inv_r2) * dm.w : 0.0f;
       const uint32_t wl = __float_as_uint(pm.w) & 3u;
-      quad_photons(wl == 0 ? v : 0.0f, wl == 1 ? v : 0.0f, wl == 2 ? v : 0.0f, ar, ag, ab);
+      ar += wl == 0u ? v : 0.0f;
+      ag += wl == 1u ? v : 0.0f;
+      ab += wl == 2u ? v : 0.0f;
     });
-    C3 di = C3{ar * scale, ag * scale, ab * scale};
+    C3 di = C3{quad_sum(ar) * scale, quad_sum(ag) * scale, quad_sum(ab) * scale};
     if (uc) di = di + direct_light_quad<BV>(sc, mk(qq.a), mk(qq.b));
     if ((threadIdx.x & 3u) == 0u) eb.res[slot] = make_float4(qq.w.x * di.r, qq.w.y * di.g, qq.w.z * di.b, 0.0f);
   }
