@@ -160,9 +160,11 @@ typedef struct {
   uint32_t first_pass;   /* 1-based index of the first pass to run */
   uint32_t pipelines;    /* passes in flight at once, each with its own buffers
                             (util/iterator.rb:18 NPARA = 4 parallel pm | rt
-                            runs); 0 = automatic: 4, or fewer when the
-                            device's free memory does not hold their buffers
-                            twice */
+                            runs); 0 = automatic: 4, which share two sets of
+                            buffers or one when the device's free memory does
+                            not hold four sets twice (images are the same).
+                            The image's double sums are formed per pipeline,
+                            then added: their last bits depend on this count */
   double   radius0;      /* r_1, the radius of pass 1 (not squared) */
   double   alpha;        /* iterator.rb:17 ALPHA */
   int32_t  use_classic;  /* ppmpa.rs:16 DEF_USECLASSIC; "-nc" clears it */

@@ -104,7 +104,7 @@ struct ppm_map {
 // pass graph.  Passes of different pipelines run at once, as the reference's
 // iterator runs NPARA pm | rt processes at once (util/iterator.rb:18,90-117).
 struct Pipe {
-  void* mem = nullptr;  // all of the pipeline's buffers (pipe_alloc)
+  void* mem = nullptr;  // what pipe_alloc allocated for it
   PhotonBuf pb;
   MapBuf map;
   EyeBuf eb;
@@ -1929,19 +1929,49 @@ void ppm_session_destroy(ppm_session* s) {
   delete s;
 }
 
-// All buffers of one pass pipeline, in one allocation.
+// What a pass pipeline keeps from pass to pass: its states and sums.
+static void pipe_own_layout(Arena& a, Pipe& p, const DevCamera& cam) {
+  const uint64_t n3 = 3ull * (uint32_t)cam.xreso * (uint32_t)cam.yreso;
+  a.take(&p.st, 1);
+  a.take(&p.st_adj, 1);
+  a.take(&p.sum, 2 * n3);
+  p.sumsq = p.sum ? p.sum + n3 : nullptr;
+}
+
+// A pass pipeline's buffers, in one allocation: what it keeps and the photons,
+// map and eye buffers of one pass.
+static void pipe_layout(Arena& a, Pipe& p, const DevCamera& cam, uint64_t n_emit, int max_depth, int n_cu) {
+  const uint64_t cap = photons_needed(n_emit, max_depth, n_cu);
+  pipe_own_layout(a, p, cam);
+  eye_layout(a, p.eb, cam, max_depth, n_cu, &p.pb, cap, trace_waves(n_emit, n_cu));
+  map_layout(a, p.map, cap, n_cu, true);
+}
+
+// lender: a pipeline whose passes run on the same stream, and whose photons,
+// map and eye buffers this one then uses too.
 static hipError_t pipe_alloc(ppm_ctx* c, Pipe& p, const DevCamera& cam, uint64_t n_emit, int max_depth,
-                             size_t* bytes) {
-  const uint64_t cap = photons_needed(n_emit, max_depth, c->n_cu);
-  return arena_alloc(c, &p.mem, [&](Arena& a) {
-    a.take(&p.st, 1);
-    a.take(&p.st_adj, 1);
-    eye_layout(a, p.eb, cam, max_depth, c->n_cu, &p.pb, cap, trace_waves(n_emit, c->n_cu));
-    map_layout(a, p.map, cap, c->n_cu, true);
-    const uint64_t n3 = 3ull * p.eb.n_pix;
-    a.take(&p.sum, 2 * n3);
-    p.sumsq = p.sum ? p.sum + n3 : nullptr;
-  }, bytes);
+                             const Pipe* lender) {
+  if (!lender)
+    return arena_alloc(c, &p.mem, [&](Arena& a) { pipe_layout(a, p, cam, n_emit, max_depth, c->n_cu); });
+  p.pb = lender->pb;
+  p.map = lender->map;
+  p.eb = lender->eb;
+  return arena_alloc(c, &p.mem, [&](Arena& a) { pipe_own_layout(a, p, cam); });
+}
+
+// The sets of pass buffers of an automatic session of MAX_PIPES pipelines: one
+// each, or two or one where that many take more than half of the memory that is
+// free or that the context's idle block would give back.
+static uint32_t session_sets(ppm_ctx* c, size_t set_bytes) {
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return MAX_PIPES;
+  }
+  avail += c->work_bytes;
+  uint32_t n = MAX_PIPES;
+  while (n > 1 && n * set_bytes > avail / 2) n /= 2;
+  return n;
 }
 
 // Before the first pass: sums cleared, pass states as new with the photon
@@ -1992,27 +2022,35 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
   s->sbuf = sc->buf;
   s->sbuf.n_emit_total = (uint32_t)total;
   // Automatic: MAX_PIPES pipelines, one per hardware queue.  A pass is a chain
-  // of kernels that rarely fill the GPU alone, and four passes in flight, each
-  // a plain chain on a queue of its own, beat one or two whose eye branch was
-  // forked beside the photon branch (ms per pass: 160x120 and 20k photons
-  // 0.35 -> 0.20, 256x256 and 200k 0.335 -> 0.154, caustic box 0.665 ->
-  // 0.637, 327k-triangle mesh 56 -> 53; three: 0.28, 0.18, 0.67, 69).  Fewer
-  // when the GPU's memory does not hold that many: at most half of what is
-  // free, except the first.
+  // of kernels that rarely fill the GPU alone: with one, two, three and four
+  // passes in flight 16 passes of 160x120 pixels and 20k photons took 6.6, 3.5,
+  // 2.6 and 1.9 ms, of 256x256 and 200k 7.8, 4.4, 3.4 and 2.6, of the caustic
+  // box (1024x768, 2M) 20.4, 14.4, 12.3 and 11.7, four of the 327k-triangle
+  // mesh (1920x1080, 8M) 212, 158, 159 and 149.
+  // Where memory is short, pipelines j and j + sets take turns on one set of
+  // buffers and one stream.  The passes and the order of the sums are the same
+  // then, so images do not depend on the memory that was free; with fewer
+  // pipelines instead the FP64 sums were grouped by other passes.
   const bool automatic = cfg->pipelines == 0;
-  uint32_t want = automatic ? MAX_PIPES : cfg->pipelines;
+  const uint32_t want = automatic ? MAX_PIPES : cfg->pipelines;
+  uint32_t sets = want;
+  if (automatic) {
+    Arena a;
+    Pipe p;
+    pipe_layout(a, p, sc->buf.cam, total, cfg->max_depth, c->n_cu);
+    sets = session_sets(c, a.used);
+  }
   hipError_t e = hipSuccess;
   s->pipes.reserve(want);
-  size_t free0 = 0, total_mem = 0, per = 0;
-  if (automatic) (void)hipMemGetInfo(&free0, &total_mem);
   for (uint32_t j = 0; j < want; ++j) {
-    if (automatic && j > 0 && (j + 1) * per > free0 / 2) break;
     Pipe p;
-    e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, &per);
-    if (e == hipErrorOutOfMemory && automatic && j > 0) {
+    e = hipErrorOutOfMemory;
+    if (j < sets) e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, nullptr);
+    if (automatic && j > 0 && e == hipErrorOutOfMemory) {
       (void)hipGetLastError();
-      e = hipSuccess;
-      break;
+      sets = std::min(sets, j);
+      p = Pipe{};
+      e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, &s->pipes[j % sets]);
     }
     if (e != hipSuccess) break;
     photons_layout(p.pb, total, cfg->max_depth, c->n_cu);
@@ -2027,7 +2065,7 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
     for (size_t j = 0; j < s->pipes.size(); ++j) {
       Pipe& p = s->pipes[j];
       eye_tiles(p.eb, s->sbuf, s->sbuf.cam, (uint32_t)sc->buf.cam.tile_shift);
-      p.stream = j == 0 || !own_streams ? c->stream : c->aux[AUX_PIPE + j - 1];
+      p.stream = j % sets == 0 || !own_streams ? c->stream : c->aux[AUX_PIPE + j % sets - 1];
       if (own_streams && (e = hipEventCreateWithFlags(&p.done, hipEventDisableTiming)) != hipSuccess) break;
     }
     if (e != hipSuccess) break;

@@ -1,0 +1,74 @@
+"""Calls while little device memory is free: photon sets of another context
+hold the rest, as a framework beside the library would."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_common import ctx, say
+
+import ppmpa_amd as P
+
+pytestmark = pytest.mark.gpu
+
+GIB = 1 << 30
+
+
+def _free():
+    """The device's free memory, from the HIP runtime that the library uses."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL(path).hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+class _Rest:
+    """All of the device's free memory but `leave` bytes."""
+
+    def __init__(self, leave):
+        self.leave = leave
+
+    def __enter__(self):
+        self.c, self.mem = P.Context(0), []
+        for step in (16 * GIB, GIB, GIB // 16):
+            while _free() >= self.leave + step:
+                self.mem.append(P.PhotonSet(self.c, (step - (1 << 20)) // 32))  # 32 B per photon
+        say("memory left: %.2f GiB" % (_free() / GIB))
+
+    def __exit__(self, *exc):
+        self.c.close()
+
+
+def _session(c, ds, n_pass=7, backward=False):
+    free = _free()
+    s = P.Session(c, ds, P.pass_cfg(seed=5, n_photon=250_000, radius0=0.01, alpha=2 / 3, max_depth=16))
+    took = free - _free()
+    s.run(n_pass - 4)
+    s.run(4)
+    out = s.image()[:2]
+    if backward:
+        out += s.backward(np.ones_like(out[0]))
+    s.close()
+    return took, out
+
+
+def test_automatic_session_gives_the_same_image():
+    """A set of buffers takes 1.3 GiB here: four of them where memory is
+    plenty, two where 8 GiB are free, one where 2.5 GiB are, whatever the
+    context's idle block (up to 2 GiB) adds.  Image and variance are the same
+    to the last bit; the adjoint adds floats by atomics in any order, up to
+    some 160 of them to a photon: 160 * 2^-24."""
+    say("memory short: automatic session")
+    c = ctx()
+    ds = P.DeviceScene(c, P.two_spheres_scene(512, 512))
+    many, plenty = _session(c, ds, backward=True)
+    again, same = _session(c, ds)
+    assert np.array_equal(plenty[0], same[0]) and np.array_equal(plenty[1], same[1])
+    for leave, most in ((8 * GIB, 0.6), (5 * GIB // 2, 0.35)):
+        with _Rest(leave):
+            few, short = _session(c, ds, backward=True)
+        assert np.array_equal(plenty[0], short[0]) and np.array_equal(plenty[1], short[1])
+        assert np.allclose(plenty[2], short[2], rtol=1e-5, atol=1e-9 * np.abs(plenty[2]).max())
+        assert abs(plenty[3] - short[3]) <= 1e-12 * abs(plenty[3])
+        assert few < most * many, (few, many)
