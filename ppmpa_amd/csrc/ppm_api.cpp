@@ -54,6 +54,7 @@ struct ppm_ctx {
   hipEvent_t stage_ev[STAGE_SLOTS] = {};  // one per slot of it
   void* work = nullptr;                // the device block calls lay their buffers out in (Work)
   size_t work_bytes = 0;
+  bool work_busy = false;  // a call's buffers lie in work
 };
 
 struct ppm_scene {
@@ -302,13 +303,6 @@ ppm_status fail(ppm_ctx* c, ppm_status s, const std::string& msg) {
   } while (0)
 
 template <typename T>
-hipError_t dalloc(T** p, uint64_t count) {
-  *p = nullptr;
-  if (count == 0) count = 1;
-  return hipMalloc((void**)p, count * sizeof(T));
-}
-
-template <typename T>
 void dfree(T*& p) {
   if (p) (void)hipFree((void*)p);
   p = nullptr;
@@ -326,11 +320,12 @@ struct Arena {
     used += ((count ? count : 1) * sizeof(T) + 255) & ~(size_t)255;
   }
 };
-// A device block of the context's; when memory runs out, once more without
-// the block it keeps for its calls.
+// Device memory; when it runs out, once more without the block that the context
+// keeps for its calls, unless the call at hand has laid its buffers out there.
+// Every allocation of a context's objects and calls comes through here.
 hipError_t block_alloc(ppm_ctx* c, void** mem, size_t bytes) {
   hipError_t e = hipMalloc(mem, bytes ? bytes : 1);
-  if (e == hipErrorOutOfMemory && c->work) {
+  if (e == hipErrorOutOfMemory && c->work && !c->work_busy) {
     (void)hipGetLastError();
     dfree(c->work);
     c->work_bytes = 0;
@@ -340,12 +335,19 @@ hipError_t block_alloc(ppm_ctx* c, void** mem, size_t bytes) {
   return e;
 }
 
+template <typename T>
+hipError_t dalloc(ppm_ctx* c, T** p, uint64_t count) {
+  void* m = nullptr;
+  const hipError_t e = block_alloc(c, &m, count * sizeof(T));
+  *p = static_cast<T*>(m);
+  return e;
+}
+
 // layout(arena) twice around one allocation; *mem is to be freed with dfree.
 template <typename F>
-hipError_t arena_alloc(ppm_ctx* c, void** mem, F&& layout, size_t* bytes = nullptr) {
+hipError_t arena_alloc(ppm_ctx* c, void** mem, F&& layout) {
   Arena a;
   layout(a);
-  if (bytes) *bytes = a.used;
   const hipError_t e = block_alloc(c, mem, a.used);
   if (e != hipSuccess) return e;
   a.base = static_cast<unsigned char*>(*mem);
@@ -362,6 +364,7 @@ hipError_t arena_alloc(ppm_ctx* c, void** mem, F&& layout, size_t* bytes = nullp
 // pass of 640x480 over 500k photons 22.1 -> 2.1 ms.
 constexpr size_t WORK_KEEP = 2ull << 30;
 struct Work {
+  ppm_ctx* held = nullptr;  // whose block it is
   void* own = nullptr;
   template <typename F>
   hipError_t get(ppm_ctx* c, F&& layout) {
@@ -380,6 +383,10 @@ struct Work {
       c->work_bytes = a.used;
       m = c->work;
     }
+    if (!own) {
+      held = c;
+      c->work_busy = true;
+    }
     a.base = static_cast<unsigned char*>(m);
     a.used = 0;
     layout(a);
@@ -388,7 +395,10 @@ struct Work {
   Work() = default;
   Work(const Work&) = delete;
   Work& operator=(const Work&) = delete;
-  ~Work() { dfree(own); }
+  ~Work() {
+    if (held) held->work_busy = false;
+    dfree(own);
+  }
 };
 
 // One-sweep sort state for up to cap keys (the look-back words count keys + 1
@@ -787,7 +797,7 @@ static ppm_status scene_layout_bvh(ppm_ctx* c, ppm_scene* sc, const std::vector<
 
 // Padded float boxes of the shapes tested one by one, for the shadow test's
 // candidate culling: a plane is marked by lo.w = 1, a point gets an empty box.
-static hipError_t upload_lin_boxes(SceneBuf& b, const std::vector<DevShape>& lin) {
+static hipError_t upload_lin_boxes(ppm_ctx* c, SceneBuf& b, const std::vector<DevShape>& lin) {
   std::vector<Node> boxes(std::max<size_t>(lin.size(), 1));
   for (size_t i = 0; i < lin.size(); ++i) {
     const DevShape& s = lin[i];
@@ -812,7 +822,7 @@ static hipError_t upload_lin_boxes(SceneBuf& b, const std::vector<DevShape>& lin
     nd.hi = make_float4(std::nextafter((float)(hi[0] + pad), INFINITY), std::nextafter((float)(hi[1] + pad), INFINITY),
                         std::nextafter((float)(hi[2] + pad), INFINITY), 0.f);
   }
-  hipError_t e = dalloc(&b.lin_box, boxes.size());
+  hipError_t e = dalloc(c, &b.lin_box, boxes.size());
   if (e == hipSuccess) e = hipMemcpy(b.lin_box, boxes.data(), boxes.size() * sizeof(Node), hipMemcpyHostToDevice);
   return e;
 }
@@ -852,11 +862,11 @@ static LinRec lin_rec(const DevShape& s) {
   r.b.w = s.p.w;
   return r;
 }
-static hipError_t upload_lin_recs(SceneBuf& b, const std::vector<DevShape>& lin) {
+static hipError_t upload_lin_recs(ppm_ctx* c, SceneBuf& b, const std::vector<DevShape>& lin) {
   std::vector<LinRec> recs(std::max<size_t>(lin.size(), 1));
   std::memset(recs.data(), 0, recs.size() * sizeof(LinRec));
   for (size_t i = 0; i < lin.size(); ++i) recs[i] = lin_rec(lin[i]);
-  hipError_t e = dalloc(&b.lin_rec, recs.size());
+  hipError_t e = dalloc(c, &b.lin_rec, recs.size());
   if (e == hipSuccess) e = hipMemcpy(b.lin_rec, recs.data(), recs.size() * sizeof(LinRec), hipMemcpyHostToDevice);
   return e;
 }
@@ -869,8 +879,8 @@ static hipError_t upload_lin_recs(SceneBuf& b, const std::vector<DevShape>& lin)
 static ppm_status scene_layout(ppm_ctx* c, ppm_scene* sc, const std::vector<DevShape>& shapes, int flags) {
   const ppm_status r = scene_layout_bvh(c, sc, shapes, flags);
   if (r != PPM_OK) return r;
-  hipError_t e = upload_lin_boxes(sc->buf, sc->lin_host);
-  if (e == hipSuccess) e = upload_lin_recs(sc->buf, sc->lin_host);
+  hipError_t e = upload_lin_boxes(c, sc->buf, sc->lin_host);
+  if (e == hipSuccess) e = upload_lin_recs(c, sc->buf, sc->lin_host);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
   return PPM_OK;
 }
@@ -984,13 +994,13 @@ static ppm_status scene_layout_bvh(ppm_ctx* c, ppm_scene* sc, const std::vector<
   Node* pbox = nullptr;
   const uint32_t n32 = (uint32_t)n;
   hipError_t e;
-  if ((e = dalloc(&ids, n)) == hipSuccess && (e = dalloc(&keys[0], n)) == hipSuccess &&
-      (e = dalloc(&keys[1], n)) == hipSuccess && (e = dalloc(&vals[0], n)) == hipSuccess &&
-      (e = dalloc(&vals[1], n)) == hipSuccess && (e = dalloc(&np, 1)) == hipSuccess &&
-      (e = dalloc(&ghist, 256ull * sort_blocks)) == hipSuccess && (e = dalloc(&totals, 256)) == hipSuccess &&
-      (e = dalloc(&pbox, n)) == hipSuccess && (e = dalloc(&b.bprims, n)) == hipSuccess &&
-      (e = dalloc(&b.bvh, (2ull << depth) - 1)) == hipSuccess &&
-      (e = dalloc(&b.lin, lin.size())) == hipSuccess &&
+  if ((e = dalloc(c, &ids, n)) == hipSuccess && (e = dalloc(c, &keys[0], n)) == hipSuccess &&
+      (e = dalloc(c, &keys[1], n)) == hipSuccess && (e = dalloc(c, &vals[0], n)) == hipSuccess &&
+      (e = dalloc(c, &vals[1], n)) == hipSuccess && (e = dalloc(c, &np, 1)) == hipSuccess &&
+      (e = dalloc(c, &ghist, 256ull * sort_blocks)) == hipSuccess && (e = dalloc(c, &totals, 256)) == hipSuccess &&
+      (e = dalloc(c, &pbox, n)) == hipSuccess && (e = dalloc(c, &b.bprims, n)) == hipSuccess &&
+      (e = dalloc(c, &b.bvh, (2ull << depth) - 1)) == hipSuccess &&
+      (e = dalloc(c, &b.lin, lin.size())) == hipSuccess &&
       (e = hipMemcpy(ids, in_bvh.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice)) == hipSuccess &&
       (e = hipMemcpy(np, &n32, sizeof(n32), hipMemcpyHostToDevice)) == hipSuccess &&
       (lin.empty() ||
@@ -1152,8 +1162,8 @@ ppm_status ppm_scene_create(ppm_ctx* c, const ppm_scene_desc* d, ppm_scene** out
   b.bmin = f4(sc->bmin);
   b.bmax = f4(sc->bmax);
   hipError_t e = hipSuccess;
-  if ((e = dalloc(&b.shapes, shapes.size())) == hipSuccess && (e = dalloc(&b.mats, mats.size())) == hipSuccess &&
-      (e = dalloc(&b.lights, sc->lights.size())) == hipSuccess) {
+  if ((e = dalloc(c, &b.shapes, shapes.size())) == hipSuccess && (e = dalloc(c, &b.mats, mats.size())) == hipSuccess &&
+      (e = dalloc(c, &b.lights, sc->lights.size())) == hipSuccess) {
     if (!shapes.empty()) e = hipMemcpy(b.shapes, shapes.data(), sizeof(DevShape) * shapes.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b.mats, mats.data(), sizeof(DevMaterial) * mats.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess && !sc->lights.empty())
@@ -1277,8 +1287,8 @@ ppm_status ppm_intersect(ppm_ctx* c, const ppm_scene* sc, const double* origins,
   int32_t* dobj = nullptr;
   std::vector<float> ht(n);
   hipError_t e;
-  if ((e = dalloc(&d_o, n)) == hipSuccess && (e = dalloc(&dD, n)) == hipSuccess && (e = dalloc(&dt, n)) == hipSuccess &&
-      (e = dalloc(&dobj, n)) == hipSuccess &&
+  if ((e = dalloc(c, &d_o, n)) == hipSuccess && (e = dalloc(c, &dD, n)) == hipSuccess && (e = dalloc(c, &dt, n)) == hipSuccess &&
+      (e = dalloc(c, &dobj, n)) == hipSuccess &&
       (e = hipMemcpyAsync(d_o, ho.data(), n * sizeof(float4), hipMemcpyHostToDevice, c->stream)) == hipSuccess &&
       (e = hipMemcpyAsync(dD, hd.data(), n * sizeof(float4), hipMemcpyHostToDevice, c->stream)) == hipSuccess &&
       (e = launch_intersect(c->stream, sc->buf, d_o, dD, (uint32_t)n, dt, dobj)) == hipSuccess &&
@@ -1401,7 +1411,7 @@ ppm_status ppm_photons_upload(ppm_ctx* c, ppm_photons* p, uint64_t n, const doub
       hi[k] = std::max(hi[k], pp[k]);
     }
   }
-  if (!p->pb.rec64) HIP_TRY(c, dalloc(&p->pb.rec64, 3 * p->cap));
+  if (!p->pb.rec64) HIP_TRY(c, dalloc(c, &p->pb.rec64, 3 * p->cap));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   if (n) {
     HIP_TRY(c, hipMemcpy(p->pb.rec, recs.data(), sizeof(PhotonRec) * n, hipMemcpyHostToDevice));
@@ -1497,7 +1507,7 @@ ppm_status ppm_map_build(ppm_ctx* c, const ppm_scene* sc, const ppm_photons* ph,
   const double* lo = sc ? sc->bmin : ph->bmin;
   const double* hi = sc ? sc->bmax : ph->bmax;
   if (!sc && !ph->has_bounds) return fail(c, PPM_E_INVALID, "no bounds for the Morton keys");
-  if (ph->has64 && !m->m.sorted64) HIP_TRY(c, dalloc(&m->m.sorted64, 3 * m->m.cap));
+  if (ph->has64 && !m->m.sorted64) HIP_TRY(c, dalloc(c, &m->m.sorted64, 3 * m->m.cap));
   HIP_TRY(c, hipMemcpyAsync(m->st, ph->st, sizeof(PassState), hipMemcpyDeviceToDevice, c->stream));
   PhotonBuf in = ph->pb;
   if (!ph->has64) in.rec64 = nullptr;
@@ -1535,10 +1545,10 @@ ppm_status ppm_map_build_grid(ppm_ctx* c, const ppm_scene* sc, const ppm_photons
   if (!m->hook_mat) {
     DevMaterial air;
     std::memset(&air, 0, sizeof(air));
-    HIP_TRY(c, dalloc(&m->hook_mat, 1));
+    HIP_TRY(c, dalloc(c, &m->hook_mat, 1));
     HIP_TRY(c, hipMemcpy(m->hook_mat, &air, sizeof(air), hipMemcpyHostToDevice));
   }
-  if (ph->has64 && !m->m.sorted64) HIP_TRY(c, dalloc(&m->m.sorted64, 3 * m->m.cap));
+  if (ph->has64 && !m->m.sorted64) HIP_TRY(c, dalloc(c, &m->m.sorted64, 3 * m->m.cap));
   // the pass state of a pass with this radius (k_grid_setup sizes the cells from r2f)
   PassState hs;
   HIP_TRY(c, hipMemcpyAsync(&hs, ph->st, sizeof(hs), hipMemcpyDeviceToHost, c->stream));
@@ -1712,10 +1722,10 @@ static ppm_status run_grid_gather(ppm_ctx* c, const ppm_map* m, const double* q_
   std::vector<float4> res(nq);
   hipError_t e = hipSuccess;
   do {
-    if ((e = dalloc(&st, 1)) != hipSuccess) break;
-    if ((e = dalloc(&eb.q, nq)) != hipSuccess) break;
-    if ((e = dalloc(&eb.res, nq)) != hipSuccess) break;
-    if ((e = dalloc(&dorder, nq)) != hipSuccess) break;
+    if ((e = dalloc(c, &st, 1)) != hipSuccess) break;
+    if ((e = dalloc(c, &eb.q, nq)) != hipSuccess) break;
+    if ((e = dalloc(c, &eb.res, nq)) != hipSuccess) break;
+    if ((e = dalloc(c, &dorder, nq)) != hipSuccess) break;
     if ((e = hipMemcpy(st, &hs, sizeof(hs), hipMemcpyHostToDevice)) != hipSuccess) break;
     if ((e = hipMemcpy(eb.q, hq.data(), sizeof(Query) * nq, hipMemcpyHostToDevice)) != hipSuccess) break;
     if ((e = hipMemcpy(dorder, order.data(), sizeof(uint32_t) * nq, hipMemcpyHostToDevice)) != hipSuccess) break;
@@ -2058,7 +2068,7 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
   }
   s->cfg.pipelines = (uint32_t)s->pipes.size();
   if (e == hipSuccess) do {
-    if ((e = dalloc(&s->lights, L.size())) != hipSuccess) break;
+    if ((e = dalloc(c, &s->lights, L.size())) != hipSuccess) break;
     if ((e = hipMemcpy(s->lights, L.data(), sizeof(DevLight) * L.size(), hipMemcpyHostToDevice)) != hipSuccess) break;
     s->sbuf.lights = s->lights;
     s->lights_host = L;
@@ -2302,8 +2312,8 @@ ppm_status ppm_session_backward(ppm_session* s, const double* grad_image, double
   const uint32_t n_pix = s->pipes[0].eb.n_pix;
   const uint32_t nm = s->sbuf.n_mats;
   // dL/d(pass image) = dL/d(mean image) / K
-  if (!s->gimg) HIP_TRY(c, dalloc(&s->gimg, n_pix));
-  if (!s->grad) HIP_TRY(c, dalloc(&s->grad, 3ull * nm));
+  if (!s->gimg) HIP_TRY(c, dalloc(c, &s->gimg, n_pix));
+  if (!s->grad) HIP_TRY(c, dalloc(c, &s->grad, 3ull * nm));
   bool finite = true;
   HIP_TRY(c, stage_in(
       c, n_pix, sizeof(float4),
@@ -2661,8 +2671,8 @@ ppm_status ppm_batch_create(ppm_ctx* c, uint32_t n, const ppm_scene* const* scen
     b->ps[q] = c->aux[AUX_PIPE + (int)q - 1];
     e = hipEventCreateWithFlags(&b->pdone[q], hipEventDisableTiming);
   }
-  if (e != hipSuccess || (e = dalloc(&b->items, (uint64_t)b->K * n)) != hipSuccess ||
-      (e = dalloc(&b->tab, (uint64_t)BK_KINDS * (n + 1))) != hipSuccess ||
+  if (e != hipSuccess || (e = dalloc(c, &b->items, (uint64_t)b->K * n)) != hipSuccess ||
+      (e = dalloc(c, &b->tab, (uint64_t)BK_KINDS * (n + 1))) != hipSuccess ||
       (e = hipEventCreate(&b->ev[0])) != hipSuccess || (e = hipEventCreate(&b->ev[1])) != hipSuccess ||
       (e = batch_layout(b)) != hipSuccess) {
     ppm_batch_destroy(b);

@@ -24,15 +24,15 @@ def _free():
 
 
 class _Rest:
-    """All of the device's free memory but `leave` bytes."""
-
-    def __init__(self, leave):
-        self.leave = leave
+    """The device's free memory, taken but for what leave() says."""
 
     def __enter__(self):
         self.c, self.mem = P.Context(0), []
+        return self
+
+    def leave(self, n):
         for step in (16 * GIB, GIB, GIB // 16):
-            while _free() >= self.leave + step:
+            while _free() >= n + step:
                 self.mem.append(P.PhotonSet(self.c, (step - (1 << 20)) // 32))  # 32 B per photon
         say("memory left: %.2f GiB" % (_free() / GIB))
 
@@ -65,10 +65,36 @@ def test_automatic_session_gives_the_same_image():
     many, plenty = _session(c, ds, backward=True)
     again, same = _session(c, ds)
     assert np.array_equal(plenty[0], same[0]) and np.array_equal(plenty[1], same[1])
-    for leave, most in ((8 * GIB, 0.6), (5 * GIB // 2, 0.35)):
-        with _Rest(leave):
+    with _Rest() as rest:
+        for n, most in ((8 * GIB, 0.6), (5 * GIB // 2, 0.35)):
+            rest.leave(n)
             few, short = _session(c, ds, backward=True)
-        assert np.array_equal(plenty[0], short[0]) and np.array_equal(plenty[1], short[1])
-        assert np.allclose(plenty[2], short[2], rtol=1e-5, atol=1e-9 * np.abs(plenty[2]).max())
-        assert abs(plenty[3] - short[3]) <= 1e-12 * abs(plenty[3])
-        assert few < most * many, (few, many)
+            assert np.array_equal(plenty[0], short[0]) and np.array_equal(plenty[1], short[1])
+            assert np.allclose(plenty[2], short[2], rtol=1e-5, atol=1e-9 * np.abs(plenty[2]).max())
+            assert abs(plenty[3] - short[3]) <= 1e-12 * abs(plenty[3])
+            assert few < most * many, (few, many)
+
+
+def test_idle_block_is_given_back():
+    """The block that a context keeps from an image of the classic tracer (over
+    1 GiB) makes room for double positions (0.9 GiB) that the rest of the
+    memory does not hold; the next image allocates it again."""
+    say("memory short: idle block")
+    c = P.Context(0)
+    ds = P.DeviceScene(c, P.two_spheres_scene(1280, 720))
+    ph = P.PhotonSet(c, 40_000_000)
+    free = _free()
+    img = P.trace_classic(c, ds, 3, 1)
+    assert GIB < free - _free() <= 2 * GIB + GIB // 64, (free - _free()) / GIB
+    rng = np.random.default_rng(1)
+    pos, d = rng.random((500, 3)), rng.standard_normal((500, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    with _Rest() as rest:
+        rest.leave(GIB // 2)
+        ph.upload(pos, d, np.zeros(500, np.uint8))
+    m = P.build_photonmap(c, ph, 1e-3)
+    got = m.within(pos[:20], 0.2 ** 2, refine64=True)
+    for q, i in zip(pos[:20], got):
+        assert np.array_equal(i, np.nonzero(((pos - q) ** 2).sum(1) <= 0.2 ** 2)[0])
+    assert np.array_equal(P.trace_classic(c, ds, 3, 1), img)
+    c.close()
