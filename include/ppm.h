@@ -193,7 +193,8 @@ typedef struct {
 /* ---- context ------------------------------------------------------------ */
 
 /* Open a context on HIP device `device`; hip_stream may be NULL (the context
- * then creates its own default-priority stream). */
+ * then creates its own default-priority stream).  A stream of the caller's has
+ * to outlive the context's objects; ppm_destroy does not touch it. */
 ppm_status  ppm_create(ppm_ctx** out, int device, void* hip_stream);
 void        ppm_destroy(ppm_ctx* ctx);
 const char* ppm_last_error(const ppm_ctx* ctx);

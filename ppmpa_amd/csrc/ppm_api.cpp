@@ -720,7 +720,8 @@ void ppm_destroy(ppm_ctx* c) {
       (void)hipStreamDestroy(a);
       a = nullptr;
     }
-  if (c->stage || c->work) (void)hipStreamSynchronize(c->stream);
+  // calls return with their work done, and the frees wait for what a failed one
+  // may have left queued: a stream that is the caller's is not touched
   if (c->stage) (void)hipHostFree(c->stage);
   dfree(c->work);
   for (hipEvent_t v : c->stage_ev)
