@@ -659,8 +659,6 @@ static MapBuf grid_view_of(const ppm_map* m) {
 }
 static MapBuf map_view(const ppm_map* m) { return m->grid ? grid_view_of(m) : tree_view(m); }
 
-namespace {}  // namespace
-
 extern "C" {
 
 const char* ppm_status_string(ppm_status s) {

@@ -387,7 +387,6 @@ __device__ __forceinline__ bool rect_meet(V3 p, float a, float b, V3 o, V3 d, fl
 
 // Record r (list position i, wave-uniform) met by the ray at t: what
 // shape_hit would offer take(), when true.
-__device__ __forceinline__ DevShape lin_shape(const SceneView& sc, uint32_t i);
 __device__ __forceinline__ bool lin_meet(const SceneView& sc, const LinRec& r, uint32_t i, V3 o, V3 d, float& t) {
 #pragma clang fp contract(off)
   const V3 a = mk(r.a);

@@ -1497,9 +1497,8 @@ hipError_t launch_grid_build(hipStream_t s, MapBuf& m, PassState* st, const Phot
 // are marked not valid.  The next step's records are loaded before the
 // current ones are tested (256x256 box, whose waves each shade one group:
 // shade 0.085 -> 0.078 ms alone; caustic 0.340 -> 0.330).
-// ALL: on_photon(j, pm, dm, d2, inside, valid) for every slot, inside only when
-// valid; otherwise on_photon(j, pm, dm, d2) for the valid photons inside the
-// ball.
+// on_photon(j, pm, dm, d2, inside, valid) is called for every slot, inside only
+// when valid, so that its work can be a select instead of a branch per photon.
 struct RangeWalk {
   uint32_t k, j, e;
   __device__ __forceinline__ explicit RangeWalk(const uint2 (&se)[8]) : k(0), j(se[0].x), e(se[0].y) {}
@@ -1517,7 +1516,7 @@ struct RangeWalk {
     return true;
   }
 };
-template <bool ALL, typename OnPhoton>
+template <typename OnPhoton>
 __device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se)[8], float qx, float qy, float qz,
                                            float r2, OnPhoton& on_photon) {
   RangeWalk w(se);
@@ -1535,17 +1534,10 @@ __device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se
     const float d1 = dist2_nc(qx, qy, qz, p1.pm.x, p1.pm.y, p1.pm.z);
     const float d2 = dist2_nc(qx, qy, qz, p2.pm.x, p2.pm.y, p2.pm.z);
     const float d3 = dist2_nc(qx, qy, qz, p3.pm.x, p3.pm.y, p3.pm.z);
-    if constexpr (ALL) {
-      on_photon(j0, p0.pm, p0.dm, d0, d0 <= r2, true);
-      on_photon(i1, p1.pm, p1.dm, d1, v1 && d1 <= r2, v1);
-      on_photon(i2, p2.pm, p2.dm, d2, v2 && d2 <= r2, v2);
-      on_photon(i3, p3.pm, p3.dm, d3, v3 && d3 <= r2, v3);
-    } else {
-      if (d0 <= r2) on_photon(j0, p0.pm, p0.dm, d0);
-      if (v1 && d1 <= r2) on_photon(i1, p1.pm, p1.dm, d1);
-      if (v2 && d2 <= r2) on_photon(i2, p2.pm, p2.dm, d2);
-      if (v3 && d3 <= r2) on_photon(i3, p3.pm, p3.dm, d3);
-    }
+    on_photon(j0, p0.pm, p0.dm, d0, d0 <= r2, true);
+    on_photon(i1, p1.pm, p1.dm, d1, v1 && d1 <= r2, v1);
+    on_photon(i2, p2.pm, p2.dm, d2, v2 && d2 <= r2, v2);
+    on_photon(i3, p3.pm, p3.dm, d3, v3 && d3 <= r2, v3);
     if (!more) break;
     p0 = q0;
     p1 = q1;
@@ -1614,12 +1606,12 @@ __device__ __forceinline__ bool grid_ranges(const GridView& g, const uint2* cell
   return ok;
 }
 
-// on_photon for the photons of the query's cells (grid_walk8).
-template <bool ALL = false, typename OnPhoton>
+// on_photon for the slots of the query's cells (grid_walk8).
+template <typename OnPhoton>
 __device__ __forceinline__ bool grid_query(const GridView& g, const uint2* cells, const PhotonRec* ph, float qx,
                                            float qy, float qz, float r2, OnPhoton&& on_photon) {
   return grid_ranges(g, cells, qx, qy, qz,
-                     [&](const uint2 (&se)[8]) { grid_walk8<ALL>(ph, se, qx, qy, qz, r2, on_photon); });
+                     [&](const uint2 (&se)[8]) { grid_walk8(ph, se, qx, qy, qz, r2, on_photon); });
 }
 
 // ===========================================================================
@@ -2298,8 +2290,8 @@ __device__ __forceinline__ bool shade_gather(const GridView& g, const uint2* cel
   // grid records (grid_rec): the direction carries the weight, pm.w and dm.w
   // flag channels 0 and 1; v * 1 and v * 0 are exact, so each channel's sum
   // is formed as with a select
-  return grid_query<true>(g, cells, ph, qq.a.x, qq.a.y, qq.a.z, r2,
-                          [&](uint32_t, float4 pm, float4 dm, float d2, bool in, bool) {
+  return grid_query(g, cells, ph, qq.a.x, qq.a.y, qq.a.z, r2,
+                    [&](uint32_t, float4 pm, float4 dm, float d2, bool in, bool) {
     const float c = photon_cos(nx, ny, nz, dm);  // optics.rs:225
     const float v = (in && c < 0.0f) ? -c * filter_weight(f, d2 * inv_r2) : 0.0f;
     ar = fmaf(v, pm.w, ar);
@@ -2452,16 +2444,16 @@ __global__ __launch_bounds__(256) void k_adj_gather(SceneView sc, const uint2* c
     const bool want = active && (fr != 0.0f || fg != 0.0f || fb != 0.0f);
     if (want) {
       const float nx = qq.b.x, ny = qq.b.y, nz = qq.b.z;
-      complete &= grid_query<true>(g, cells, ph, qq.a.x, qq.a.y, qq.a.z, r2,
-                                   // the channel factors by value: a conditional over referenced
-                                   // floats selects an address, which puts the closure in scratch
-                                   [=](uint32_t j, float4 pm, float4 dm, float d2, bool in, bool) {
-                                     // grid records (grid_rec): weighted direction, channel flags
-                                     const float c = photon_cos(nx, ny, nz, dm);
-                                     const float f = pm.w != 0.0f ? fr : (dm.w != 0.0f ? fg : fb);
-                                     const float a = in && c < 0.0f ? f * (-c * filter_weight(pf, d2 * inv_r2)) : 0.0f;
-                                     if (a != 0.0f) atomicAdd(&adj[j], a);
-                                   });
+      complete &= grid_query(g, cells, ph, qq.a.x, qq.a.y, qq.a.z, r2,
+                             // the channel factors by value: a conditional over referenced
+                             // floats selects an address, which puts the closure in scratch
+                             [=](uint32_t j, float4 pm, float4 dm, float d2, bool in, bool) {
+                               // grid records (grid_rec): weighted direction, channel flags
+                               const float c = photon_cos(nx, ny, nz, dm);
+                               const float f = pm.w != 0.0f ? fr : (dm.w != 0.0f ? fg : fb);
+                               const float a = in && c < 0.0f ? f * (-c * filter_weight(pf, d2 * inv_r2)) : 0.0f;
+                               if (a != 0.0f) atomicAdd(&adj[j], a);
+                             });
     }
   }
   if (!complete) atomicOr(&st->overflow, 4u);
@@ -2896,17 +2888,17 @@ __global__ __launch_bounds__(256) void k_grid_query(const uint2* cells, const Ph
   }
   uint32_t cnt = 0;
   const uint64_t off = mode == 1 ? offsets[i] : 0;
-  const bool ok = grid_query<true>(g, cells, ph, qp.x, qp.y, qp.z, r2f,
-                                   [&](uint32_t j, float4, float4, float d2, bool in, bool valid) {
-                                     float t;
-                                     const bool keep =
-                                         refine ? valid && in_ball(d2, r2f, band, true, ph64, j, qx, qy, qz, r2, &t)
-                                                : in;
-                                     if (keep) {
-                                       if (mode == 1) idx_out[off + cnt] = src_idx[j];
-                                       ++cnt;
-                                     }
-                                   });
+  const bool ok = grid_query(g, cells, ph, qp.x, qp.y, qp.z, r2f,
+                             [&](uint32_t j, float4, float4, float d2, bool in, bool valid) {
+                               float t;
+                               const bool keep =
+                                   refine ? valid && in_ball(d2, r2f, band, true, ph64, j, qx, qy, qz, r2, &t)
+                                          : in;
+                               if (keep) {
+                                 if (mode == 1) idx_out[off + cnt] = src_idx[j];
+                                 ++cnt;
+                               }
+                             });
   if (!ok) atomicOr(flags, 1u);
   if (mode == 0) counts[i] = cnt;
 }
