@@ -5,7 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from gpu_common import ctx, say
+from gpu_common import ctx, random_photons, say
 
 import ppmpa_amd as P
 
@@ -97,4 +97,34 @@ def test_idle_block_is_given_back():
     for q, i in zip(pos[:20], got):
         assert np.array_equal(i, np.nonzero(((pos - q) ** 2).sum(1) <= 0.2 ** 2)[0])
     assert np.array_equal(P.trace_classic(c, ds, 3, 1), img)
+    c.close()
+
+
+@pytest.mark.parametrize("kind", ["eye", "classic"])
+def test_call_larger_than_the_kept_block(kind):
+    """At 1920x1080 the buffers of an eye pass take more than the 2 GiB that a
+    context keeps: the call allocates its own and gives them back.  Its rows
+    are those of a picture a third as high, whose buffers fit; a pixel's terms
+    may be added in another order (80 of one sign: 2 * 80 * 2^-24 < 1e-5)."""
+    say("memory: a call larger than the kept block", kind)
+    c = P.Context(0)
+    ph = P.PhotonSet(c, 5000)
+    ph.upload(*random_photons(5000, 1))
+    m = P.build_photonmap(c, ph, 1e-3)
+
+    def image(rows):
+        sc = P.two_spheres_scene(1920, 360)
+        at = sc.camera.screen()  # the first rows keep their rays and random streams
+        sc.camera.screen, sc.camera.yreso = lambda: at, rows
+        ds = P.DeviceScene(c, sc)
+        if kind == "classic":
+            return P.trace_classic(c, ds, 3, 1)
+        return P.trace_eye(c, ds, m, 3, 1, 0.02 ** 2, max_depth=10)
+
+    small = image(360)
+    free = _free()
+    large = image(1080)
+    assert abs(free - _free()) <= GIB // 64
+    assert np.allclose(large[:360], small, rtol=1e-5, atol=0.0) and (large[360:] > 0).any()
+    assert np.array_equal(image(360), small)
     c.close()
