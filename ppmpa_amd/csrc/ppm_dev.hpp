@@ -202,6 +202,9 @@ constexpr uint32_t MAT_LDS = 48;  // materials (M_AIR included)
 __shared__ DevShape g_lin_lds[LIN_LDS];
 __shared__ Node g_linbox_lds[LIN_LDS];
 __shared__ DevMaterial g_mat_lds[MAT_LDS];
+constexpr uint32_t SCENE_LDS_BYTES =
+    LIN_LDS * (uint32_t)(sizeof(DevShape) + sizeof(Node)) + MAT_LDS * (uint32_t)sizeof(DevMaterial);
+constexpr uint32_t CU_LDS_BYTES = 160u * 1024u;
 
 __device__ __forceinline__ void copy16(float4* dst, const float4* src, uint32_t n) {
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];

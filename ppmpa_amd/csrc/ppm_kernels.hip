@@ -301,6 +301,10 @@ __device__ __forceinline__ bool photon_bounce(const SceneView& sc, int uc, Photo
 // blocks and a direction) in every step of the wave: caustic workload, 2M
 // photons, together with the bounce's one block per step (Rng::peek4): the
 // trace alone 0.289 -> 0.253 ms, the pass 0.697 -> 0.665 ms.
+// Kernels that copy small trees to LDS emit on demand: with the slots, 12 KB of
+// a block, beside the 18 KB of the copies four blocks fit on a CU instead of
+// five, and the walks wait on their LDS loads (64 rooms in a batch: a round
+// 18.45 ms with the slots, 17.75 without; 24 rooms, eight rounds: 71.4, 68.6).
 struct EmitLds {
   float4 o[64];    // origin, channel
   float4 d[64];    // direction, draws consumed
@@ -335,9 +339,14 @@ __device__ __forceinline__ void k_trace_photons_body(SceneView sc, PassState* st
                                                        AdjTrace at = AdjTrace{nullptr, nullptr}) {
   __shared__ float part[ADJ ? 3 * ADJ_LDS_MATS : 1];
   __shared__ uint16_t evl[ADJ ? ADJ_MAX_EV * 256 : 1];
-  __shared__ EmitLds s_emit[4];
+  constexpr bool AHEAD = BV < 2;  // emission ahead
+  __shared__ EmitLds s_emit[AHEAD ? 4 : 1];
   constexpr bool BIG = BV == 1 || BV == 3;  // large trees: the wave's walks together
   __shared__ WalkLds s_walk[BIG ? 4 : 1];
+  static_assert(BV < 2 || ADJ ||
+                    5u * (BVH_DYN_LDS_BYTES + SCENE_LDS_BYTES + (AHEAD ? sizeof(EmitLds) * 4 : 0) +
+                          (BIG ? sizeof(WalkLds) * 4 : 0)) <= CU_LDS_BYTES,
+                "five blocks of a small-tree trace on a CU");
   scene_to_lds<BV>(sc);
   const uint32_t w = blk.b * (blockDim.x / 64) + (threadIdx.x >> 6);
   if (ADJ) {
@@ -354,7 +363,7 @@ __device__ __forceinline__ void k_trace_photons_body(SceneView sc, PassState* st
   const uint32_t p_begin = (uint32_t)min<uint64_t>(lo, sc.n_emit);
   const uint32_t p_end = (uint32_t)min<uint64_t>(lo + per_wave, sc.n_emit);
   PhotonRec* region = rec + (uint64_t)w * region_cap;
-  EmitLds& em = s_emit[threadIdx.x >> 6];
+  EmitLds& em = s_emit[AHEAD ? threadIdx.x >> 6 : 0u];
   uint32_t next = p_begin;   // wave-uniform: the next photon to hand out
   uint32_t ready = p_begin;  // wave-uniform: photons [next, ready) are emitted, photon i in em's slot (i - p_begin) % 64
   uint32_t cnt = 0;          // wave-uniform
@@ -363,56 +372,74 @@ __device__ __forceinline__ void k_trace_photons_body(SceneView sc, PassState* st
   Rng rng;
   p.pid = 0;
   uint32_t n_ev = 0;
+  auto start = [&] {  // p has its origin, direction, channel and index
+    p.med = sc.n_mats;  // M_AIR
+    p.depth = 0;
+    p.w = 1.0f;
+    n_ev = 0;
+    alive = true;
+  };
   while (true) {
     bool need = !alive && !done;
-    for (uint64_t m = __ballot(need); m != 0u; m = __ballot(need)) {
-      if (next == ready && ready < p_end) {
-        const uint32_t pid = ready + lane;
-        if (pid < p_end) {
-          PhotonState q;
-          Rng r;
-          r.init(seed, pid, pass, TAG_PHOTON);
-          emit_photon(sc, pid, r, q);
-          em.o[lane] = make_float4(q.o.x, q.o.y, q.o.z, __uint_as_float(q.wl));
-          em.d[lane] = make_float4(q.d.x, q.d.y, q.d.z, __uint_as_float(r.n));
-          em.b[0][lane] = r.blk.x;
-          em.b[1][lane] = r.blk.y;
-          em.b[2][lane] = r.blk.z;
-          em.b[3][lane] = r.blk.w;
+    if constexpr (AHEAD) {
+      for (uint64_t m = __ballot(need); m != 0u; m = __ballot(need)) {
+        if (next == ready && ready < p_end) {
+          const uint32_t pid = ready + lane;
+          if (pid < p_end) {
+            PhotonState q;
+            Rng r;
+            r.init(seed, pid, pass, TAG_PHOTON);
+            emit_photon(sc, pid, r, q);
+            em.o[lane] = make_float4(q.o.x, q.o.y, q.o.z, __uint_as_float(q.wl));
+            em.d[lane] = make_float4(q.d.x, q.d.y, q.d.z, __uint_as_float(r.n));
+            em.b[0][lane] = r.blk.x;
+            em.b[1][lane] = r.blk.y;
+            em.b[2][lane] = r.blk.z;
+            em.b[3][lane] = r.blk.w;
+          }
+          ready = min(ready + 64u, p_end);
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        ready = min(ready + 64u, p_end);
+        const uint32_t have = ready - next, want = (uint32_t)__popcll(m);
+        if (need) {
+          const uint32_t k = (uint32_t)__popcll(m & lanemask_lt());
+          if (k < have) {
+            const uint32_t pid = next + k, e = (pid - p_begin) & 63u;
+            const float4 o = em.o[e], d = em.d[e];
+            rng.init(seed, pid, pass, TAG_PHOTON);
+            rng.n = __float_as_uint(d.w);
+            rng.blk = make_uint4(em.b[0][e], em.b[1][e], em.b[2][e], em.b[3][e]);
+            p.o = mk(o);
+            p.d = mk(d);
+            p.wl = __float_as_uint(o.w);
+            p.pid = pid;
+            start();
+            need = false;
+          } else if (ready == p_end) {
+            done = true;
+            need = false;
+          }
+        }
+        next += min(have, want);
+        // the slots read above are written again by the next emission
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
-      const uint32_t have = ready - next, want = (uint32_t)__popcll(m);
+    } else if (const uint64_t m = __ballot(need)) {
       if (need) {
-        const uint32_t k = (uint32_t)__popcll(m & lanemask_lt());
-        if (k < have) {
-          const uint32_t pid = next + k, e = (pid - p_begin) & 63u;
-          const float4 o = em.o[e], d = em.d[e];
+        const uint32_t pid = next + (uint32_t)__popcll(m & lanemask_lt());
+        if (pid < p_end) {
           rng.init(seed, pid, pass, TAG_PHOTON);
-          rng.n = __float_as_uint(d.w);
-          rng.blk = make_uint4(em.b[0][e], em.b[1][e], em.b[2][e], em.b[3][e]);
-          p.o = mk(o);
-          p.d = mk(d);
-          p.wl = __float_as_uint(o.w);
-          p.med = sc.n_mats;  // M_AIR
-          p.depth = 0;
+          emit_photon(sc, pid, rng, p);
           p.pid = pid;
-          p.w = 1.0f;
-          n_ev = 0;
-          alive = true;
-          need = false;
-        } else if (ready == p_end) {
+          start();
+        } else {
           done = true;
-          need = false;
         }
       }
-      next += min(have, want);
-      // the slots read above are written again by the next emission
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      next += (uint32_t)__popcll(m);
     }
     if (!__any(alive)) break;
     bool store = false;
