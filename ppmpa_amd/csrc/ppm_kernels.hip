@@ -1521,9 +1521,15 @@ hipError_t launch_grid_build(hipStream_t s, MapBuf& m, PassState* st, const Phot
 // before.  Four consecutive records per step, loaded together from one
 // address; the slots of a step that runs past its range's end (into the
 // next bucket's records, or the GRID_READ_SLACK zeroed ones after the last)
-// are marked not valid.  The next step's records are loaded before the
-// current ones are tested (256x256 box, whose waves each shade one group:
-// shade 0.085 -> 0.078 ms alone; caustic 0.340 -> 0.330).
+// are marked not valid.
+// AHEAD: the next step's records are loaded before the current ones are tested
+// (256x256 box, whose waves each shade one group: shade 0.085 -> 0.078 ms alone;
+// caustic 0.340 -> 0.330).  They pay only beside a callback of few registers:
+// with a photon filter the shade took 107 to 112 instead of 76 to 94 and kept
+// four waves on a SIMD instead of five or six (16 caustic passes with the cone
+// filter 11.48 ms with the loads ahead, 10.70 without; no filter 10.58, 11.00;
+// 64 rooms in a batch, whose kernel serves any filter, 17.75 and 17.22 ms a
+// round).
 // on_photon(j, pm, dm, d2, inside, valid) is called for every slot, inside only
 // when valid, so that its work can be a select instead of a branch per photon.
 struct RangeWalk {
@@ -1543,20 +1549,28 @@ struct RangeWalk {
     return true;
   }
 };
-template <typename OnPhoton>
+template <bool AHEAD, typename OnPhoton>
 __device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se)[8], float qx, float qy, float qz,
                                            float r2, OnPhoton& on_photon) {
   RangeWalk w(se);
   if (!w.advance(se)) return;
   const PhotonRec* p = ph + w.j;
-  PhotonRec p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+  PhotonRec p0, p1, p2, p3;
+  if constexpr (AHEAD) p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
   while (true) {
+    if constexpr (!AHEAD) {
+      p = ph + w.j;
+      p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+    }
     const uint32_t j0 = w.j, i1 = j0 + 1u, i2 = j0 + 2u, i3 = j0 + 3u;
     const bool v1 = i1 < w.e, v2 = i2 < w.e, v3 = i3 < w.e;
     w.j += 4u;
     const bool more = w.advance(se);
-    const PhotonRec* q = ph + (more ? w.j : j0);
-    const PhotonRec q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+    PhotonRec q0, q1, q2, q3;
+    if constexpr (AHEAD) {
+      const PhotonRec* q = ph + (more ? w.j : j0);
+      q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+    }
     const float d0 = dist2_nc(qx, qy, qz, p0.pm.x, p0.pm.y, p0.pm.z);
     const float d1 = dist2_nc(qx, qy, qz, p1.pm.x, p1.pm.y, p1.pm.z);
     const float d2 = dist2_nc(qx, qy, qz, p2.pm.x, p2.pm.y, p2.pm.z);
@@ -1566,10 +1580,7 @@ __device__ __forceinline__ void grid_walk8(const PhotonRec* ph, const uint2 (&se
     on_photon(i2, p2.pm, p2.dm, d2, v2 && d2 <= r2, v2);
     on_photon(i3, p3.pm, p3.dm, d3, v3 && d3 <= r2, v3);
     if (!more) break;
-    p0 = q0;
-    p1 = q1;
-    p2 = q2;
-    p3 = q3;
+    if constexpr (AHEAD) p0 = q0, p1 = q1, p2 = q2, p3 = q3;
   }
 }
 
@@ -1634,11 +1645,11 @@ __device__ __forceinline__ bool grid_ranges(const GridView& g, const uint2* cell
 }
 
 // on_photon for the slots of the query's cells (grid_walk8).
-template <typename OnPhoton>
+template <bool AHEAD = true, typename OnPhoton>
 __device__ __forceinline__ bool grid_query(const GridView& g, const uint2* cells, const PhotonRec* ph, float qx,
                                            float qy, float qz, float r2, OnPhoton&& on_photon) {
   return grid_ranges(g, cells, qx, qy, qz,
-                     [&](const uint2 (&se)[8]) { grid_walk8(ph, se, qx, qy, qz, r2, on_photon); });
+                     [&](const uint2 (&se)[8]) { grid_walk8<AHEAD>(ph, se, qx, qy, qz, r2, on_photon); });
 }
 
 // ===========================================================================
@@ -2299,16 +2310,16 @@ __global__ __launch_bounds__(256) void k_query_keys(EyeBuf eb, const PassState* 
 // BSDF factor and path throughput.  Gather and shadow rays share the kernel
 // so that the waves of one hide the memory latency of the other.  A query
 // whose cells exceed the grid's span rule raises flag 4 of the pass state.
-// The gather of one query: the summed -n.dir * filter * weight per channel
-// into ar, ag, ab.  PF >= 0 fixes the photon filter at compile time (no test
-// of it in the per-photon loop, and only that filter's registers); PF = -1
-// takes it from pf (batches, whose scenes may differ).
 // n . dir with its fused multiply-adds written out: the kernels that share the
 // gather (sessions, batches) must round alike, and left to the compiler the
 // choice of which products to fuse differed between them.
 __device__ __forceinline__ float photon_cos(float nx, float ny, float nz, float4 dm) {
   return fmaf(nz, dm.z, fmaf(nx, dm.x, ny * dm.y));
 }
+// The gather of one query: the summed -n.dir * filter * weight per channel
+// into ar, ag, ab.  PF >= 0 fixes the photon filter at compile time (no test
+// of it in the per-photon loop, and only that filter's registers); PF = -1
+// takes it from pf (batches, whose scenes may differ).
 template <int PF>
 __device__ __forceinline__ bool shade_gather(const GridView& g, const uint2* cells, const PhotonRec* ph, const Query& qq,
                                              float r2, float inv_r2, int pf, float& ar, float& ag, float& ab) {
@@ -2317,8 +2328,8 @@ __device__ __forceinline__ bool shade_gather(const GridView& g, const uint2* cel
   // grid records (grid_rec): the direction carries the weight, pm.w and dm.w
   // flag channels 0 and 1; v * 1 and v * 0 are exact, so each channel's sum
   // is formed as with a select
-  return grid_query(g, cells, ph, qq.a.x, qq.a.y, qq.a.z, r2,
-                    [&](uint32_t, float4 pm, float4 dm, float d2, bool in, bool) {
+  return grid_query<PF == FILTER_NONE>(g, cells, ph, qq.a.x, qq.a.y, qq.a.z, r2,
+                                       [&](uint32_t, float4 pm, float4 dm, float d2, bool in, bool) {
     const float c = photon_cos(nx, ny, nz, dm);  // optics.rs:225
     const float v = (in && c < 0.0f) ? -c * filter_weight(f, d2 * inv_r2) : 0.0f;
     ar = fmaf(v, pm.w, ar);
