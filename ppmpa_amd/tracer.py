@@ -56,6 +56,7 @@ class Context:
         self.lib = A.load()
         self.h = None
         self._objs = weakref.WeakSet()  # everything made on this context
+        self._live = {}                 # and its handles still to be destroyed: (destroy call, address) -> handle
         h = C.c_void_p()
         s = self.lib.ppm_create(C.byref(h), int(device), None)
         if s != 0:
@@ -63,9 +64,22 @@ class Context:
         self.h = h
         _CONTEXTS.add(self)
 
+    # the order in which a context's objects are destroyed
+    _DESTROY = ("ppm_batch_destroy", "ppm_session_destroy", "ppm_map_destroy", "ppm_photons_destroy",
+                "ppm_scene_destroy")
+
     def _own(self, obj):
-        """Record an object made on this context (closed before it)."""
+        """Record an object made on this context (destroyed before it).  Its
+        handle is kept, not only a weak reference to it: the garbage collector
+        clears those of a cycle that holds both before it calls anything."""
         self._objs.add(obj)
+        self._live[obj._destroy, obj.h.value] = obj.h
+
+    def _drop(self, obj):
+        """Destroy an object made on this context, unless it has been."""
+        h, obj.h = obj.h, None
+        if h and self._live.pop((obj._destroy, h.value), None):
+            getattr(self.lib, obj._destroy)(h)
 
     def check(self, s):
         if s != 0:
@@ -79,9 +93,11 @@ class Context:
         """ppm_destroy, after closing every object still open on the context
         (batches and sessions first, scenes last)."""
         if self.h:
-            rank = {Batch: 0, Session: 1, PhotonMap: 2, PhotonSet: 3, DeviceScene: 4}
-            for o in sorted(list(self._objs), key=lambda o: rank.get(type(o), 0)):
-                o.close()
+            for o in list(self._objs):
+                o.h = None
+            for k in sorted(self._live, key=lambda k: self._DESTROY.index(k[0])):
+                getattr(self.lib, k[0])(self._live[k])
+            self._live.clear()
             self.lib.ppm_destroy(self.h)
             self.h = None
 
@@ -94,6 +110,8 @@ class Context:
 
 class DeviceScene:
     """read_scene + read_camera uploaded (ppm_scene_create)."""
+
+    _destroy = "ppm_scene_destroy"
 
     def __init__(self, ctx, scene):
         self.ctx, self.scene = ctx, scene
@@ -140,9 +158,7 @@ class DeviceScene:
         return t, obj
 
     def close(self):
-        if self.h:
-            self.ctx.lib.ppm_scene_destroy(self.h)
-            self.h = None
+        self.ctx._drop(self)
 
     def __del__(self):
         try:
@@ -153,6 +169,8 @@ class DeviceScene:
 
 class PhotonSet:
     """A device-resident photon set (ppm_photons_*)."""
+
+    _destroy = "ppm_photons_destroy"
 
     def __init__(self, ctx, capacity):
         self.ctx = ctx
@@ -193,9 +211,7 @@ class PhotonSet:
         return pos[:n], dir[:n], wl[:n], meta[:n]
 
     def close(self):
-        if self.h:
-            self.ctx.lib.ppm_photons_destroy(self.h)
-            self.h = None
+        self.ctx._drop(self)
 
     def __del__(self):
         try:
@@ -223,6 +239,8 @@ def trace_photons(ctx, dscene, seed, pass_, n_photon, use_classic=True, max_dept
 
 class PhotonMap:
     """build_photonmap's PhotonMap (photonmap.rs:16-29) on the device."""
+
+    _destroy = "ppm_map_destroy"
 
     def __init__(self, ctx, capacity):
         self.ctx = ctx
@@ -277,9 +295,7 @@ class PhotonMap:
         return out
 
     def close(self):
-        if self.h:
-            self.ctx.lib.ppm_map_destroy(self.h)
-            self.h = None
+        self.ctx._drop(self)
 
     def __del__(self):
         try:
@@ -339,6 +355,8 @@ def pass_cfg(seed, n_photon, radius0, alpha, max_depth, use_classic=True, pfilte
 class Session:
     """PPM-PA pass loop (util/iterator.rb + util/averager2.rb) on the device."""
 
+    _destroy = "ppm_session_destroy"
+
     def __init__(self, ctx, dscene, cfg):
         self.ctx, self.dscene, self.cfg = ctx, dscene, cfg
         h = C.c_void_p()
@@ -390,9 +408,7 @@ class Session:
         return {k: getattr(t, k) for k, _ in A.Timings._fields_ if k != "reserved"}
 
     def close(self):
-        if self.h:
-            self.ctx.lib.ppm_session_destroy(self.h)
-            self.h = None
+        self.ctx._drop(self)
 
     def __del__(self):
         try:
@@ -415,6 +431,8 @@ class Batch:
     """Many scenes, each with its own pass schedule, run together: one launch
     per pass stage over every scene still running (ppm_batch_*).  Each
     scene's image equals what its own Session would produce."""
+
+    _destroy = "ppm_batch_destroy"
 
     def __init__(self, ctx, dscenes, cfgs, n_passes):
         self.ctx, self.dscenes = ctx, list(dscenes)
@@ -472,9 +490,7 @@ class Batch:
         return {k: getattr(t, k) for k, _ in A.Timings._fields_ if k != "reserved"}
 
     def close(self):
-        if self.h:
-            self.ctx.lib.ppm_batch_destroy(self.h)
-            self.h = None
+        self.ctx._drop(self)
 
     def __del__(self):
         try:

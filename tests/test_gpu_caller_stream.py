@@ -16,15 +16,9 @@ pytestmark = pytest.mark.gpu
 NON_BLOCKING, RELAXED = 1, 2  # hipStreamNonBlocking, hipStreamCaptureModeRelaxed
 
 
-def _hip():
-    A.load()
-    with open("/proc/self/maps") as f:
-        return C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
-
-
 def _context_on(stream):
     c = P.Context.__new__(P.Context)
-    c.lib, c.h, c._objs = A.load(), C.c_void_p(), weakref.WeakSet()
+    c.lib, c.h, c._objs, c._live = A.load(), C.c_void_p(), weakref.WeakSet(), {}
     assert c.lib.ppm_create(C.byref(c.h), 0, stream) == 0
     return c
 
@@ -34,7 +28,7 @@ def test_destroy_leaves_the_stream_alone():
     staged results and keeps a block, is destroyed: waiting for the stream
     would end the capture with an error."""
     say("caller stream: destroy during a capture")
-    hip = _hip()
+    hip = A.load()  # its symbols include those of the HIP runtime that it is linked to
     stream, graph = C.c_void_p(), C.c_void_p()
     assert hip.hipStreamCreateWithFlags(C.byref(stream), NON_BLOCKING) == 0
     want = P.trace_classic(ctx(), P.DeviceScene(ctx(), small_scene("caustic", 64, 48)), 3, 1)

@@ -8,6 +8,7 @@ import pytest
 from gpu_common import ctx, random_photons, say
 
 import ppmpa_amd as P
+from ppmpa_amd import _abi as A
 
 pytestmark = pytest.mark.gpu
 
@@ -15,11 +16,10 @@ GIB = 1 << 30
 
 
 def _free():
-    """The device's free memory, from the HIP runtime that the library uses."""
-    with open("/proc/self/maps") as f:
-        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    """The device's free memory, from the HIP runtime that the library is
+    linked to (torch, once imported, brings another)."""
     free, total = C.c_size_t(), C.c_size_t()
-    assert C.CDLL(path).hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    assert A.load().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
     return free.value
 
 
