@@ -26,14 +26,14 @@ using namespace ppm;
 // Streams of a context beside its own, kept until ppm_destroy, so that
 // creating and destroying sessions creates and destroys no streams: AUX_PIPE
 // + j - 1 runs pass pipeline j >= 1 (pipeline 0 runs on the context's
-// stream), AUX_CAPTURE is the stream pass graphs are captured on (made on
-// first use).  The pipelines' streams are made with the context, right after
+// stream), AUX_CAPTURE and AUX_CAPTURE2 are the streams pass graphs are captured
+// on (made on first use).  The pipelines' streams are made with the context, right after
 // its own: HIP spreads a process's streams over four hardware queues in the
 // order they are made, and two pipelines on one queue run one after the
 // other (four pipelines whose streams were made after a capture stream: as
 // slow as two).  Calls on a context never overlap (each returns once its
 // work is done), so its sessions and batches may share them.
-constexpr int AUX_PIPE = 0, AUX_CAPTURE = MAX_PIPES - 1, AUX_N = MAX_PIPES;
+constexpr int AUX_PIPE = 0, AUX_CAPTURE = MAX_PIPES - 1, AUX_CAPTURE2 = MAX_PIPES, AUX_N = MAX_PIPES + 1;
 
 // Pinned host memory a context keeps for the caller's arrays (stage_out,
 // stage_in), in slots: kernels write some while the host empties others.
@@ -128,6 +128,7 @@ struct ppm_session {
   double power = 0.0;
   uint32_t passes_done = 0;
   std::vector<Pipe> pipes;  // pass p (from cfg.first_pass) runs on pipes[p % K]
+  bool fork = false;        // the pass graphs' eye branch runs beside the photon branch
   std::vector<DevLight> lights_host;  // what `lights` holds
   float4* gimg = nullptr;   // ppm_session_backward: the image gradient and the
   double* grad = nullptr;   // material gradients (made on first use)
@@ -158,6 +159,38 @@ void ctx_stream_renew(ppm_ctx* c, int i) {
     (void)hipStreamDestroy(c->aux[i]);
   }
   c->aux[i] = nullptr;
+}
+
+// A pass's launches, enqueue(stream, fork), captured into *graph and made into
+// *exec, on the context's capture streams; fork: with a second one for the eye
+// branch, whose events live only while the graph is captured.  A capture that
+// fails part-way leaves no graph behind, and fresh streams replace these.
+template <typename F>
+hipError_t capture_pass(ppm_ctx* c, bool fork, hipGraph_t* graph, hipGraphExec_t* exec, F&& enqueue) {
+  hipStream_t cap = nullptr;
+  PassFork f;
+  hipError_t e = ctx_stream(c, AUX_CAPTURE, &cap);
+  if (e == hipSuccess && fork) e = ctx_stream(c, AUX_CAPTURE2, &f.side);
+  if (e == hipSuccess && fork) e = hipEventCreateWithFlags(&f.split, hipEventDisableTiming);
+  if (e == hipSuccess && fork) e = hipEventCreateWithFlags(&f.join, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
+  if (e == hipSuccess) {
+    const hipError_t e2 = enqueue(cap, f);
+    const hipError_t e3 = hipStreamEndCapture(cap, graph);
+    e = e2 != hipSuccess ? e2 : e3;
+  }
+  if (e == hipSuccess) e = hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
+  if (f.join) (void)hipEventDestroy(f.join);
+  if (f.split) (void)hipEventDestroy(f.split);
+  if (e != hipSuccess) {
+    if (*exec) (void)hipGraphExecDestroy(*exec);
+    if (*graph) (void)hipGraphDestroy(*graph);
+    *exec = nullptr;
+    *graph = nullptr;
+    ctx_stream_renew(c, AUX_CAPTURE);
+    ctx_stream_renew(c, AUX_CAPTURE2);
+  }
+  return e;
 }
 
 // The context's pinned staging memory and its events (made on first use,
@@ -1949,19 +1982,22 @@ static void pipe_own_layout(Arena& a, Pipe& p, const DevCamera& cam) {
 
 // A pass pipeline's buffers, in one allocation: what it keeps and the photons,
 // map and eye buffers of one pass.
-static void pipe_layout(Arena& a, Pipe& p, const DevCamera& cam, uint64_t n_emit, int max_depth, int n_cu) {
+// fork: its photons are traced beside its eye rays, so the two share no memory.
+static void pipe_layout(Arena& a, Pipe& p, const DevCamera& cam, uint64_t n_emit, int max_depth, int n_cu, bool fork) {
   const uint64_t cap = photons_needed(n_emit, max_depth, n_cu);
+  const uint32_t regions = trace_waves(n_emit, n_cu);
   pipe_own_layout(a, p, cam);
-  eye_layout(a, p.eb, cam, max_depth, n_cu, &p.pb, cap, trace_waves(n_emit, n_cu));
+  eye_layout(a, p.eb, cam, max_depth, n_cu, fork ? nullptr : &p.pb, cap, regions);
+  if (fork) photons_layout_mem(a, p.pb, cap, regions);
   map_layout(a, p.map, cap, n_cu, true);
 }
 
 // lender: a pipeline whose passes run on the same stream, and whose photons,
 // map and eye buffers this one then uses too.
-static hipError_t pipe_alloc(ppm_ctx* c, Pipe& p, const DevCamera& cam, uint64_t n_emit, int max_depth,
+static hipError_t pipe_alloc(ppm_ctx* c, Pipe& p, const DevCamera& cam, uint64_t n_emit, int max_depth, bool fork,
                              const Pipe* lender) {
   if (!lender)
-    return arena_alloc(c, &p.mem, [&](Arena& a) { pipe_layout(a, p, cam, n_emit, max_depth, c->n_cu); });
+    return arena_alloc(c, &p.mem, [&](Arena& a) { pipe_layout(a, p, cam, n_emit, max_depth, c->n_cu, fork); });
   p.pb = lender->pb;
   p.map = lender->map;
   p.eb = lender->eb;
@@ -2043,10 +2079,15 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
   const bool automatic = cfg->pipelines == 0;
   const uint32_t want = automatic ? MAX_PIPES : cfg->pipelines;
   uint32_t sets = want;
+  // One pipeline alone has no other pass to run beside: its eye branch runs beside
+  // its photon branch (ms per pass as a chain / forked: 160x120 and 20k photons
+  // 0.334 / 0.238, 256x256 and 100k 0.372 / 0.262, 1024x768 and 2M 1.24 / 0.95; a
+  // batch of 24 rooms, a round: 10.1 / 9.0).
+  s->fork = want == 1;
   if (automatic) {
     Arena a;
     Pipe p;
-    pipe_layout(a, p, sc->buf.cam, total, cfg->max_depth, c->n_cu);
+    pipe_layout(a, p, sc->buf.cam, total, cfg->max_depth, c->n_cu, false);
     sets = session_sets(c, a.used);
   }
   hipError_t e = hipSuccess;
@@ -2054,12 +2095,12 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
   for (uint32_t j = 0; j < want; ++j) {
     Pipe p;
     e = hipErrorOutOfMemory;
-    if (j < sets) e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, nullptr);
+    if (j < sets) e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, s->fork, nullptr);
     if (automatic && j > 0 && e == hipErrorOutOfMemory) {
       (void)hipGetLastError();
       sets = std::min(sets, j);
       p = Pipe{};
-      e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, &s->pipes[j % sets]);
+      e = pipe_alloc(c, p, sc->buf.cam, total, cfg->max_depth, false, &s->pipes[j % sets]);
     }
     if (e != hipSuccess) break;
     photons_layout(p.pb, total, cfg->max_depth, c->n_cu);
@@ -2098,8 +2139,10 @@ ppm_status ppm_session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass_cf
 // Enqueue the kernels of one pass of pipeline j on stream st, one after the
 // other: the eye rays and the order of their queries, then the photons, their
 // grid, the gather and the sums.  ev != nullptr (stage timing) records its
-// events between the stages, the photons first.
-static hipError_t enqueue_pass(ppm_session* s, uint32_t j, hipStream_t st, hipEvent_t* ev) {
+// events between the stages, the photons first.  f: the eye rays and their order
+// beside the photons and their grid.
+static hipError_t enqueue_pass(ppm_session* s, uint32_t j, hipStream_t st, hipEvent_t* ev,
+                               const PassFork& f = PassFork{}) {
   const ppm_pass_cfg& cfg = s->cfg;
   const ppm_scene* sc = s->scene;
   Pipe& p = s->pipes[j];
@@ -2110,18 +2153,23 @@ static hipError_t enqueue_pass(ppm_session* s, uint32_t j, hipStream_t st, hipEv
   const uint32_t K = (uint32_t)s->pipes.size();
   auto mark = [&](int k) { return ev ? hipEventRecord(ev[k], st) : hipSuccess; };
   const PassBegin begin{cfg.first_pass + j, K, cfg.radius0 * cfg.radius0, cfg.alpha};
+  const bool apart = ev || f.side;  // the pass begins in a launch of its own
+  hipStream_t es = f.side ? f.side : st;
   auto eye = [&] {
-    return launch_eye(st, s->sbuf, p.st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, n_cu, ev ? PassBegin{} : begin);
+    return launch_eye(es, s->sbuf, p.st, p.eb, cfg.seed, cfg.use_classic, cfg.max_depth, n_cu,
+                      apart ? PassBegin{} : begin);
   };
-  auto order = [&] { return launch_query_prep(st, s->sbuf, p.map, p.st, p.eb); };
+  auto order = [&] { return launch_query_prep(es, s->sbuf, p.map, p.st, p.eb); };
   if ((e = mark(0)) != hipSuccess) return e;
-  if (ev && (e = launch_pass_begin(st, p.st, begin.first_pass, begin.r2_first, begin.alpha, K)) != hipSuccess) return e;
+  if (apart && (e = launch_pass_begin(st, p.st, begin.first_pass, begin.r2_first, begin.alpha, K)) != hipSuccess) return e;
+  if ((e = f.split_from(st)) != hipSuccess) return e;
   if (!ev && ((e = eye()) != hipSuccess || (e = order()) != hipSuccess)) return e;
   if ((e = launch_trace_photons(st, s->sbuf, p.st, p.pb, cfg.seed, cfg.use_classic, cfg.max_depth, false)) != hipSuccess)
     return e;
   if ((e = mark(1)) != hipSuccess) return e;
   if ((e = launch_grid_build(st, p.map, p.st, p.pb, bmin, bmax, 2ull * s->sbuf.n_emit_total, true)) != hipSuccess)
     return e;
+  if ((e = f.join_to(st)) != hipSuccess) return e;
   if ((e = mark(2)) != hipSuccess) return e;
   if (ev && ((e = eye()) != hipSuccess || (e = mark(3)) != hipSuccess || (e = order()) != hipSuccess)) return e;
   if ((e = launch_gather(st, s->sbuf, p.map, p.st, p.eb, cfg.pfilter, cfg.use_classic, n_cu, p.sum, p.sumsq,
@@ -2130,28 +2178,12 @@ static hipError_t enqueue_pass(ppm_session* s, uint32_t j, hipStream_t st, hipEv
   return mark(6);
 }
 
-// The pass graph of pipeline j, captured once.  A capture that fails
-// part-way leaves no graph behind, and the capture stream is replaced by a
-// fresh one.
+// The pass graph of pipeline j, captured once.
 static hipError_t pipe_graph(ppm_session* s, uint32_t j) {
   Pipe& p = s->pipes[j];
   if (p.exec) return hipSuccess;
-  ppm_ctx* c = s->ctx;
-  hipStream_t cap;
-  hipError_t e = ctx_stream(c, AUX_CAPTURE, &cap);
-  if (e != hipSuccess) return e;
-  e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) {
-    const hipError_t e2 = enqueue_pass(s, j, cap, nullptr);
-    const hipError_t e3 = hipStreamEndCapture(cap, &p.graph);
-    e = e2 != hipSuccess ? e2 : e3;
-  }
-  if (e == hipSuccess) e = hipGraphInstantiate(&p.exec, p.graph, nullptr, nullptr, 0);
-  if (e != hipSuccess) {
-    pipe_drop_graph(p);
-    ctx_stream_renew(c, AUX_CAPTURE);
-  }
-  return e;
+  return capture_pass(s->ctx, s->fork, &p.graph, &p.exec,
+                      [&](hipStream_t cap, const PassFork& f) { return enqueue_pass(s, j, cap, nullptr, f); });
 }
 
 ppm_status ppm_session_run(ppm_session* s, uint32_t n_pass) {
@@ -2569,26 +2601,11 @@ hipError_t batch_round(ppm_batch* b, uint32_t act, uint32_t q) {
   if (!b->exec[gi]) {
     uint32_t blocks[BK_KINDS];
     for (int k = 0; k < BK_KINDS; ++k) blocks[k] = b->htab[(size_t)k * (n + 1) + act];
-    // captured on the context's capture stream.  A capture that fails
-    // part-way leaves no graph behind and replaces that stream.
-    hipStream_t cap = nullptr;
-    hipError_t e = ctx_stream(b->ctx, AUX_CAPTURE, &cap);
-    if (e == hipSuccess) e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess) {
-      const hipError_t e2 =
-          launch_batch_pass(cap, b->items + (size_t)q * n, b->tab, blocks, act, n, b->bvh, b->dyn);
-      const hipError_t e3 = hipStreamEndCapture(cap, &b->graph[gi]);
-      e = e2 != hipSuccess ? e2 : e3;
-    }
-    if (e == hipSuccess) e = hipGraphInstantiate(&b->exec[gi], b->graph[gi], nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-      if (b->exec[gi]) (void)hipGraphExecDestroy(b->exec[gi]);
-      if (b->graph[gi]) (void)hipGraphDestroy(b->graph[gi]);
-      b->exec[gi] = nullptr;
-      b->graph[gi] = nullptr;
-      ctx_stream_renew(b->ctx, AUX_CAPTURE);
-      return e;
-    }
+    const hipError_t e =
+        capture_pass(b->ctx, b->K == 1, &b->graph[gi], &b->exec[gi], [&](hipStream_t cap, const PassFork& f) {
+          return launch_batch_pass(cap, b->items + (size_t)q * n, b->tab, blocks, act, n, b->bvh, b->dyn, f);
+        });
+    if (e != hipSuccess) return e;
   }
   return hipGraphLaunch(b->exec[gi], b->ps[q]);
 }

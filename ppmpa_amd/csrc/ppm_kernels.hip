@@ -3188,32 +3188,35 @@ __global__ __launch_bounds__(256) void kb_accumulate(const BatchItem* items, con
 #undef BATCH_PROLOGUE
 
 hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
-                             uint32_t n_all, int bvh, uint32_t dyn) {
+                             uint32_t n_all, int bvh, uint32_t dyn, const PassFork& f) {
   // blocks[k] = total blocks of kind k over the first n scenes.  One chain of
-  // launches: the rounds of the other pipelines run beside it.
+  // launches, beside which the rounds of the other pipelines run; where there
+  // are none (f), the eye branch runs beside the photon branch.
   const dim3 T256(256), T1024(1024), T64(64), TOS(OS_THREADS);
   hipError_t e;
   hipLaunchKernelGGL(kb_pass_begin, dim3(n), T64, 0, s, items, n);
-  hipLaunchKernelGGL(kb_tile_order, dim3(blocks[BK_PIX]), T256, 0, s, items, tab, n, n_all);
+  if ((e = f.split_from(s)) != hipSuccess) return e;
+  hipStream_t es = f.side ? f.side : s;
+  hipLaunchKernelGGL(kb_tile_order, dim3(blocks[BK_PIX]), T256, 0, es, items, tab, n, n_all);
   switch (bvh) {
     case 3:
-      hipLaunchKernelGGL(kb_eye<3>, dim3(blocks[BK_EYE]), T256, dyn, s, items, tab, n, n_all);
+      hipLaunchKernelGGL(kb_eye<3>, dim3(blocks[BK_EYE]), T256, dyn, es, items, tab, n, n_all);
       break;
     case 2:
-      hipLaunchKernelGGL(kb_eye<2>, dim3(blocks[BK_EYE]), T256, dyn, s, items, tab, n, n_all);
+      hipLaunchKernelGGL(kb_eye<2>, dim3(blocks[BK_EYE]), T256, dyn, es, items, tab, n, n_all);
       break;
     case 1:
-      hipLaunchKernelGGL(kb_eye<1>, dim3(blocks[BK_EYE]), T256, 0, s, items, tab, n, n_all);
+      hipLaunchKernelGGL(kb_eye<1>, dim3(blocks[BK_EYE]), T256, 0, es, items, tab, n, n_all);
       break;
     default:
-      hipLaunchKernelGGL(kb_eye<0>, dim3(blocks[BK_EYE]), T256, 0, s, items, tab, n, n_all);
+      hipLaunchKernelGGL(kb_eye<0>, dim3(blocks[BK_EYE]), T256, 0, es, items, tab, n, n_all);
   }
-  hipLaunchKernelGGL(kb_tile_count, dim3(blocks[BK_PIX]), T256, 0, s, items, tab, n, n_all);
-  hipLaunchKernelGGL(kb_scan_tiles, dim3(n), T1024, 0, s, items, n);
-  hipLaunchKernelGGL(kb_query_keys, dim3(blocks[BK_QKEYS]), T256, 0, s, items, tab, n, n_all);
-  hipLaunchKernelGGL(kb_os_hist, dim3(blocks[BK_QHIST]), T1024, 0, s, items, tab, n, n_all, 1);
+  hipLaunchKernelGGL(kb_tile_count, dim3(blocks[BK_PIX]), T256, 0, es, items, tab, n, n_all);
+  hipLaunchKernelGGL(kb_scan_tiles, dim3(n), T1024, 0, es, items, n);
+  hipLaunchKernelGGL(kb_query_keys, dim3(blocks[BK_QKEYS]), T256, 0, es, items, tab, n, n_all);
+  hipLaunchKernelGGL(kb_os_hist, dim3(blocks[BK_QHIST]), T1024, 0, es, items, tab, n, n_all, 1);
   for (uint32_t p = 0; p < QUERY_KEY_BITS / 8u; ++p)
-    hipLaunchKernelGGL(kb_os_scatter<false>, dim3(blocks[BK_QOS]), TOS, 0, s, items, tab, n, n_all, 1, p);
+    hipLaunchKernelGGL(kb_os_scatter<false>, dim3(blocks[BK_QOS]), TOS, 0, es, items, tab, n, n_all, 1, p);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   switch (bvh) {
     case 3:
@@ -3240,6 +3243,7 @@ hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32
   hipLaunchKernelGGL(kb_grid_clear, dim3(blocks[BK_CLEAR]), T256, 0, s, items, tab, n, n_all);
   hipLaunchKernelGGL(kb_grid_cells, dim3(blocks[BK_LEAVES]), T256, 0, s, items, tab, n, n_all);
   if ((e = hipGetLastError()) != hipSuccess) return e;
+  if ((e = f.join_to(s)) != hipSuccess) return e;
   switch (bvh) {
     case 3:
       hipLaunchKernelGGL(kb_shade<3>, dim3(blocks[BK_SHADE]), T256, dyn, s, items, tab, n, n_all);

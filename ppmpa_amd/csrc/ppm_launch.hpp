@@ -180,6 +180,23 @@ struct PassBegin {
   double r2_first = 0.0, alpha = 0.0;
 };
 
+// A second stream for the eye branch of a pass and the events that split it off
+// and join it again (side null: the pass is one chain).
+struct PassFork {
+  hipStream_t side = nullptr;
+  hipEvent_t split = nullptr, join = nullptr;
+  hipError_t split_from(hipStream_t s) const {
+    if (!side) return hipSuccess;
+    const hipError_t e = hipEventRecord(split, s);
+    return e != hipSuccess ? e : hipStreamWaitEvent(side, split, 0);
+  }
+  hipError_t join_to(hipStream_t s) const {
+    if (!side) return hipSuccess;
+    const hipError_t e = hipEventRecord(join, side);
+    return e != hipSuccess ? e : hipStreamWaitEvent(s, join, 0);
+  }
+};
+
 // Number of tracing waves (= photon regions) used for n photons.
 uint32_t trace_waves(uint64_t n_photon, int n_cu);
 
@@ -372,7 +389,7 @@ hipError_t launch_adjoint(hipStream_t s, const SceneBuf& sc, const MapBuf& m, Pa
 // One pass of the first n scenes of a batch (scenes sorted by pass count,
 // so the scenes still running are a prefix); blocks[k] = tab[k*(n_all+1)+n].
 hipError_t launch_batch_pass(hipStream_t s, const BatchItem* items, const uint32_t* tab, const uint32_t* blocks, uint32_t n,
-                             uint32_t n_all, int bvh, uint32_t dyn);  // bvh: the kernels' BV; dyn: their dynamic LDS
+                             uint32_t n_all, int bvh, uint32_t dyn, const PassFork& f);  // bvh: the kernels' BV; dyn: their dynamic LDS
 
 // Test hook: nearest hit of n rays (unit directions).
 hipError_t launch_intersect(hipStream_t s, const SceneBuf& sc, const float4* o, const float4* d, uint32_t n,
