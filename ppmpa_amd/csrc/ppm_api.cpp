@@ -829,8 +829,7 @@ static ppm_status scene_layout_bvh(ppm_ctx* c, ppm_scene* sc, const std::vector<
 
 // Padded float boxes of the shapes tested one by one, for the shadow test's
 // candidate culling: a plane is marked by lo.w = 1, a point gets an empty box.
-static hipError_t upload_lin_boxes(ppm_ctx* c, SceneBuf& b, const std::vector<DevShape>& lin) {
-  std::vector<Node> boxes(std::max<size_t>(lin.size(), 1));
+static void lin_boxes(const std::vector<DevShape>& lin, Node* boxes) {
   for (size_t i = 0; i < lin.size(); ++i) {
     const DevShape& s = lin[i];
     Node& nd = boxes[i];
@@ -854,9 +853,6 @@ static hipError_t upload_lin_boxes(ppm_ctx* c, SceneBuf& b, const std::vector<De
     nd.hi = make_float4(std::nextafter((float)(hi[0] + pad), INFINITY), std::nextafter((float)(hi[1] + pad), INFINITY),
                         std::nextafter((float)(hi[2] + pad), INFINITY), 0.f);
   }
-  hipError_t e = dalloc(c, &b.lin_box, boxes.size());
-  if (e == hipSuccess) e = hipMemcpy(b.lin_box, boxes.data(), boxes.size() * sizeof(Node), hipMemcpyHostToDevice);
-  return e;
 }
 
 // The list as rays test it (LinRec).
@@ -894,13 +890,22 @@ static LinRec lin_rec(const DevShape& s) {
   r.b.w = s.p.w;
   return r;
 }
-static hipError_t upload_lin_recs(ppm_ctx* c, SceneBuf& b, const std::vector<DevShape>& lin) {
-  std::vector<LinRec> recs(std::max<size_t>(lin.size(), 1));
-  std::memset(recs.data(), 0, recs.size() * sizeof(LinRec));
-  for (size_t i = 0; i < lin.size(); ++i) recs[i] = lin_rec(lin[i]);
-  hipError_t e = dalloc(c, &b.lin_rec, recs.size());
-  if (e == hipSuccess) e = hipMemcpy(b.lin_rec, recs.data(), recs.size() * sizeof(LinRec), hipMemcpyHostToDevice);
-  return e;
+// The boxes and then the records of the list, in one allocation (lin_box's) and
+// one copy.
+static hipError_t upload_lin(ppm_ctx* c, SceneBuf& b, const std::vector<DevShape>& lin) {
+  static_assert(sizeof(LinRec) == sizeof(Node), "records after boxes in one array");
+  const size_t n = std::max<size_t>(lin.size(), 1);
+  std::vector<Node> both(2 * n);
+  std::memset(both.data(), 0, both.size() * sizeof(Node));
+  lin_boxes(lin, both.data());
+  for (size_t i = 0; i < lin.size(); ++i) {
+    const LinRec r = lin_rec(lin[i]);
+    std::memcpy(&both[n + i], &r, sizeof(r));
+  }
+  hipError_t e = dalloc(c, &b.lin_box, both.size());
+  if (e != hipSuccess) return e;
+  b.lin_rec = reinterpret_cast<LinRec*>(b.lin_box + n);
+  return hipMemcpy(b.lin_box, both.data(), both.size() * sizeof(Node), hipMemcpyHostToDevice);
 }
 
 // Shapes tested one by one and, when the scene asks for one (or has at least
@@ -911,8 +916,7 @@ static hipError_t upload_lin_recs(ppm_ctx* c, SceneBuf& b, const std::vector<Dev
 static ppm_status scene_layout(ppm_ctx* c, ppm_scene* sc, const std::vector<DevShape>& shapes, int flags) {
   const ppm_status r = scene_layout_bvh(c, sc, shapes, flags);
   if (r != PPM_OK) return r;
-  hipError_t e = upload_lin_boxes(c, sc->buf, sc->lin_host);
-  if (e == hipSuccess) e = upload_lin_recs(c, sc->buf, sc->lin_host);
+  const hipError_t e = upload_lin(c, sc->buf, sc->lin_host);
   if (e != hipSuccess) return fail(c, e == hipErrorOutOfMemory ? PPM_E_OOM : PPM_E_HIP, hipGetErrorString(e));
   return PPM_OK;
 }
@@ -1252,7 +1256,6 @@ void ppm_scene_destroy(ppm_scene* sc) {
   dfree(sc->buf.bvh);
   dfree(sc->buf.bprims);
   dfree(sc->buf.lin_box);
-  dfree(sc->buf.lin_rec);
   delete sc;
 }
 

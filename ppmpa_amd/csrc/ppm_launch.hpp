@@ -15,7 +15,7 @@ struct SceneBuf {
   DevMaterial* mats = nullptr;  // n_mats + 1 (M_AIR last)
   DevLight* lights = nullptr;
   DevShape* lin = nullptr;      // shapes tested one by one (== shapes when there is no BVH)
-  LinRec* lin_rec = nullptr;    // the lin shapes as rays test them
+  LinRec* lin_rec = nullptr;    // the lin shapes as rays test them (behind lin_box)
   Node* lin_box = nullptr;      // padded box of each lin shape; lo.w = 1 marks a plane
   Node* bvh = nullptr;          // 2^(bvh_depth+1) - 1 nodes, or null
   DevShape* bprims = nullptr;   // n_bprims shapes in leaf order
