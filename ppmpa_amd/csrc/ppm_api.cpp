@@ -2242,12 +2242,19 @@ ppm_status ppm_session_run(ppm_session* s, uint32_t n_pass) {
   return PPM_OK;
 }
 
-// The pass states of all pipelines (after the context stream's work).
+// The pass states of all pipelines (after the context stream's work), through the
+// staging memory: one wait for all of them.
 static hipError_t pipe_states(ppm_session* s, std::vector<PassState>& h) {
-  h.resize(s->pipes.size());
-  hipError_t e = hipStreamSynchronize(s->ctx->stream);
+  static_assert(MAX_PIPES * sizeof(PassState) <= STAGE_BYTES, "the states fit the staging memory");
+  ppm_ctx* c = s->ctx;
+  hipError_t e = ctx_stage(c);
   for (size_t j = 0; j < s->pipes.size() && e == hipSuccess; ++j)
-    e = hipMemcpy(&h[j], s->pipes[j].st, sizeof(PassState), hipMemcpyDeviceToHost);
+    e = hipMemcpyAsync(c->stage + j * sizeof(PassState), s->pipes[j].st, sizeof(PassState), hipMemcpyDeviceToHost,
+                       c->stream);
+  const hipError_t e2 = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = e2;
+  h.resize(s->pipes.size());
+  if (e == hipSuccess) std::memcpy(h.data(), c->stage, h.size() * sizeof(PassState));
   return e;
 }
 
