@@ -363,7 +363,7 @@ ppm_status  ppm_trace_classic(ppm_ctx* ctx, const ppm_scene* scene,
 ppm_status  ppm_session_create(ppm_ctx* ctx, const ppm_scene* scene,
                                const ppm_pass_cfg* cfg, ppm_session** out);
 void        ppm_session_destroy(ppm_session* s);
-/* Queue n_pass further passes (asynchronous, stream-ordered). */
+/* Run n_pass further passes; returns once they are done. */
 ppm_status  ppm_session_run(ppm_session* s, uint32_t n_pass);
 /* Per-pixel mean over the passes run so far (yreso x xreso x 3 doubles,
  * row-major) and, when var_out is not NULL, the unbiased per-pixel variance

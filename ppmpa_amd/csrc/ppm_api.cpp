@@ -26,13 +26,13 @@ using namespace ppm;
 // Streams of a context beside its own, kept until ppm_destroy, so that
 // creating and destroying sessions creates and destroys no streams: AUX_PIPE
 // + j - 1 runs pass pipeline j >= 1 (pipeline 0 runs on the context's
-// stream), AUX_CAPTURE and AUX_CAPTURE2 are the streams pass graphs are captured
-// on (made on first use).  The pipelines' streams are made with the context, right after
-// its own: HIP spreads a process's streams over four hardware queues in the
-// order they are made, and two pipelines on one queue run one after the
-// other (four pipelines whose streams were made after a capture stream: as
-// slow as two).  Calls on a context never overlap (each returns once its
-// work is done), so its sessions and batches may share them.
+// stream), AUX_CAPTURE and AUX_CAPTURE2 are the streams pass graphs are
+// captured on (made on first use).  The pipelines' streams are made with the
+// context, right after its own: HIP spreads a process's streams over four
+// hardware queues in the order they are made, and two pipelines on one queue
+// run one after the other (four pipelines whose streams were made after a
+// capture stream: as slow as two).  Calls on a context never overlap (each
+// returns once its work is done), so its sessions and batches may share them.
 constexpr int AUX_PIPE = 0, AUX_CAPTURE = MAX_PIPES - 1, AUX_CAPTURE2 = MAX_PIPES, AUX_N = MAX_PIPES + 1;
 
 // Pinned host memory a context keeps for the caller's arrays (stage_out,
@@ -394,7 +394,10 @@ hipError_t arena_alloc(ppm_ctx* c, void** mem, F&& layout) {
 // call so far, but at most WORK_KEEP bytes (a larger call allocates and frees
 // its own), given back by ppm_destroy and by block_alloc when memory runs
 // out.  Allocating them per call cost more than the calls' kernels: an eye
-// pass of 640x480 over 500k photons 22.1 -> 2.1 ms.
+// pass of 640x480 over 500k photons 22.1 -> 2.1 ms.  WORK_KEEP holds an
+// eye pass of 1280x720 at depth 10 (1.6 GB); at 1920x1080 (3.9 GB) calls pay
+// for their allocation: eye 6.2-19 ms a call, 5.2 with a larger block, classic
+// 117, 2.8.  More is not kept, since nothing but this context gives it back.
 constexpr size_t WORK_KEEP = 2ull << 30;
 struct Work {
   ppm_ctx* held = nullptr;  // whose block it is
@@ -566,11 +569,17 @@ uint32_t cam_tiles_max(const DevCamera& cam) {
 //   256x256, rough glass: eye 0.157 / 0.101 / 0.071, eight passes 1.62 / 1.49 / 1.46
 //   512x512, 40 shapes: eye 0.558 / 0.341 / 0.428
 //   640x400, 300 spheres: eye 2.08 / 1.32 / 1.05, eight passes 15.4 / 14.4 / 14.7
-//   640x400, 20k triangles: eye 3.35 / 1.83 / 1.13, eight passes 27.4 / 24.0 / 22.6
-//   1024x768, glass sphere: 64 passes 41.1 / 42.3 / 47.3
-//   1920x1080, 327k triangles: four passes 132.6 / 129.9 / 131.8
 //   256x256, a mirror sphere: 16 passes 2.06 / 2.13 / 2.16
-//   24 rooms of 128^2-512^2 in one batch: four rounds 41.4 / 41.7 / 43.9
+// and 16 passes with a glass sphere, by the tiles: 4096 4.53 / 4.13 / 4.52, 6144
+// 5.25 / 5.13 / 5.90, 7168 5.50 / 5.53 / 6.20, 8192 5.79 / 5.88 / 6.64, 10240
+// 6.72 / 6.87 / 7.94, 12288 7.48 / 7.84 / 9.05; eight with 20k triangles: 4000
+// 26.3 / 22.8 / 21.7, 8192 37.2 / 34.7 / 35.0, 12288 42.8 / 40.8 / 39.9; four
+// with 327k: 32400 132.6 / 129.9 / 131.8.  So the first line lies where halves
+// and whole tiles meet, between 7168 and 8192 within the runs' noise, and scenes of
+// many shapes go on one step finer.
+// A batch keeps its sessions' parts, so that its images are theirs bit for bit;
+// its many rooms need no sharing, and pay for the halves: 24 rooms, 12 rounds 103.4
+// / 105.2, 64 rooms about 0.45 of 17.2 a round.
 uint32_t eye_part_shift(const SceneBuf& sc, uint32_t tiles) {
   if (!sc.branches) return 0;
   const bool few = tiles <= 8192u;
@@ -578,7 +587,7 @@ uint32_t eye_part_shift(const SceneBuf& sc, uint32_t tiles) {
   return sc.n_shapes > BVH_SMALL_PRIMS ? (few ? 2 : 1) : (few ? 1 : 0);
 }
 
-// The eye buffers at tile shape `shift` (sized for any shape by eye_alloc);
+// The eye buffers at tile shape `shift` (sized for any shape by eye_layout);
 // the tiles' query counts of earlier passes, which only order the eye's
 // work, start again from zero.
 bool eye_tiles(EyeBuf& eb, const SceneBuf& sc, DevCamera& cam, uint32_t shift) {
@@ -2662,8 +2671,9 @@ ppm_status ppm_batch_create(ppm_ctx* c, uint32_t n, const ppm_scene* const* scen
   // pipelines: the smallest cfgs[i].pipelines, 3 where it is 0 (automatic):
   // three rounds in flight by default, since a full round keeps the GPU busy
   // and a third pipeline fills the tails of each stage, where the rooms with
-  // the most work are still running (64-room workload: 3.19 s with two,
-  // 3.11 s with three, 3.18 s with four; a session gains nothing past two)
+  // the most work are still running (12 rounds of 24 rooms with one pipeline
+  // 107.4 ms, two 101.4, three 98.9, four 97.8: a fourth set of buffers in every
+  // room for a hundredth)
   b->K = 4;
   for (uint32_t i = 0; i < n; ++i) b->K = std::min<uint32_t>(b->K, cfgs[i].pipelines ? cfgs[i].pipelines : 3u);
   if (b->K == 0) b->K = 1;

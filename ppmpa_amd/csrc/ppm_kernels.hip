@@ -1134,7 +1134,7 @@ static hipError_t onesweep_sort(hipStream_t s, const OneSweep& o, uint32_t* keys
 }
 
 // Leaves + tree.  The tree is a complete binary tree in heap order over
-// lpad = 2^depth leaves of 64 consecutive photons (empty leaves have empty
+// lpad = 2^depth leaves of LEAF consecutive photons (empty leaves have empty
 // boxes).  k_build_leaves: one block per 64 leaves; each wave gathers 16
 // leaves' photons into tree order (coalesced 32-byte writes), reduces their
 // boxes with cross-lane shuffles, and the block folds its 64 boxes up six
@@ -1835,8 +1835,9 @@ __device__ __forceinline__ uint64_t peer_mask(uint32_t key, bool pred) {
 // pixel, depth and path); the tile's per-pixel state lives in LDS: the
 // count of in-place deeper query slots used and the emitted radiance.  Slots
 // and sums are assigned in lane order within a step, and a wave holds one
-// tile at a time, so the schedule, and with it every slot and sum, depends
-// only on the tile: results are reproducible.  Deeper queries beyond a
+// part of a tile at a time, so the schedule, and with it every slot and sum,
+// depends only on the tile and the number of parts, which the scene and the
+// image size fix: results are reproducible.  Deeper queries beyond a
 // pixel's sec_max slots go to the overflow region (atomic slots, added in
 // any order).
 // CL: the classic ray tracer's tree instead (trace_ray_classic,
@@ -2112,11 +2113,9 @@ hipError_t launch_eye(hipStream_t s, const SceneBuf& sc, PassState* st, const Ey
                       int use_classic, int max_depth, int n_cu, const PassBegin& begin) {
   hipLaunchKernelGGL(k_tile_order, dim3((eb.n_tiles + 255) / 256 + (begin.stride != 0u ? 1u : 0u)), dim3(256), 0, s, eb,
                      st, begin);
-  // 6 persistent waves per CU: the eye's 123 registers allow 4 waves per
-  // SIMD, and a smaller grid leaves room beside it for the photon branch
-  // and the other pipeline's kernels (16 per CU filled every slot: caustic
-  // 0.855 -> 0.816 ms per pass, mesh 95.6 -> 87.8 ms; 4 and 8: 0.815-0.834
-  // and 90.6-94.5 ms)
+  // EYE_WAVES_PER_CU persistent waves per CU: the eye's registers allow 3 or 4
+  // waves per SIMD, and a smaller grid leaves room beside it for the other
+  // pipelines' kernels
   uint32_t n_waves = std::min<uint32_t>(std::min<uint32_t>(eb.n_tiles << eb.part_shift, (uint32_t)n_cu * EYE_WAVES_PER_CU), eb.estack_lanes / 64u);
   if (n_waves < 1) n_waves = 1;
   const uint32_t blocks = (n_waves + 3) / 4;

@@ -146,10 +146,12 @@ struct EyeBuf {
 constexpr uint32_t EYE_WAVES_PER_CU_MAX = 32;
 // Grid sizes of a session's persistent kernels, per CU: eye waves, shade
 // blocks of 4 waves, photon-tracing waves (= photon regions).  Each kernel
-// leaves slots free beside it for the other branch of its pass and the
-// other pipeline's pass: filling the GPU with every kernel (16 eye waves,
-// 8 shade blocks, 16 tracing waves) serialised them.  Caustic workload
-// 0.855 -> 0.730 ms per pass with these, mesh 95.6 -> 87.6 ms.
+// leaves slots free beside it for the other pipelines' passes.  With four
+// pipelines, 16 caustic passes in ms: 10.48 with these; eye 4 / 8 / 12 waves 10.55 /
+// 10.50 / 10.69; shade 3 / 4 / 6 / 8 blocks 10.38 / 10.43 / 10.80 / 11.12; tracing 4 / 6 /
+// 12 waves 10.67 / 10.60 / 10.56.  Four passes of the 327k-triangle mesh: 123.2 with
+// these, 122.1 to 124.1 with the others but 125.3 with 12 eye waves and 127.8 with
+// 4 tracing waves; small boxes and rooms within 2%.
 constexpr uint32_t EYE_WAVES_PER_CU = 6;
 constexpr uint32_t SHADE_BLOCKS_PER_CU = 5;
 constexpr uint32_t TRACE_WAVES_PER_CU = 8;
