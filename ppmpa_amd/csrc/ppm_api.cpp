@@ -2049,8 +2049,10 @@ static hipError_t session_clear(ppm_session* s, bool tiles) {
 
 // own_streams = false: a batch's session, whose passes the batch launches on
 // its own streams; the pipelines get no streams or events of their own.
+// n_pass: the passes it will run, where they are known (0: any number); an
+// automatic session needs no more sets of buffers than that.
 static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass_cfg* cfg, ppm_session** out,
-                                 bool own_streams) {
+                                 bool own_streams, uint32_t n_pass = 0) {
   if (!c || !sc || !cfg || !out) return fail(c, PPM_E_INVALID, "null argument");
   *out = nullptr;
   if (ppm_status s = check_cfg_depth(c, cfg->max_depth)) return s;
@@ -2100,7 +2102,7 @@ static ppm_status session_create(ppm_ctx* c, const ppm_scene* sc, const ppm_pass
     Arena a;
     Pipe p;
     pipe_layout(a, p, sc->buf.cam, total, cfg->max_depth, c->n_cu, false);
-    sets = session_sets(c, a.used);
+    sets = std::min(session_sets(c, a.used), n_pass ? n_pass : MAX_PIPES);
   }
   hipError_t e = hipSuccess;
   s->pipes.reserve(want);
@@ -2838,7 +2840,7 @@ ppm_status ppm_batch_timings(ppm_batch* b, ppm_timings* t) {
 ppm_status ppm_run_passes(ppm_ctx* c, const ppm_scene* sc, const ppm_pass_cfg* cfg, uint32_t n_pass, double* mean_out,
                           double* var_out, ppm_timings* t) {
   ppm_session* s = nullptr;
-  if (ppm_status st = ppm_session_create(c, sc, cfg, &s)) return st;
+  if (ppm_status st = session_create(c, sc, cfg, &s, true, std::max(n_pass, 1u))) return st;
   ppm_status st = ppm_session_run(s, n_pass);
   if (st == PPM_OK) st = ppm_session_image(s, mean_out, var_out, nullptr);
   if (st == PPM_OK && t) st = ppm_session_timings(s, t);

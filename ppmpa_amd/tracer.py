@@ -418,13 +418,14 @@ class Session:
 
 
 def run_passes(ctx, dscene, cfg, n_pass):
-    s = Session(ctx, dscene, cfg)
-    try:
-        s.run(n_pass)
-        mean, var, _ = s.image()
-        return mean, var, s.timings()
-    finally:
-        s.close()
+    """A session's image, variance and timings after n_pass passes
+    (ppm_run_passes)."""
+    cam = dscene.scene.camera
+    mean = np.zeros((cam.yreso, cam.xreso, 3))
+    var = np.zeros_like(mean)
+    t = A.Timings()
+    ctx.check(ctx.lib.ppm_run_passes(ctx.h, dscene.h, C.byref(cfg), int(n_pass), _dp(mean), _dp(var), C.byref(t)))
+    return mean, var, {k: getattr(t, k) for k, _ in A.Timings._fields_ if k != "reserved"}
 
 
 class Batch:
