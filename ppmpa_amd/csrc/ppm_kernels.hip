@@ -6,9 +6,10 @@
 //   FP64 per-pixel accumulation  (util/averager2.rb:49-62)
 //
 // Wavefront-64 design: one photon / pixel / query per lane; wave-wide ballots
-// compact live photons and stored records; the map is a balanced binary tree
-// over Morton-sorted 64-photon leaves, traversed wave-coherently so that one
-// leaf is staged once into LDS (coalesced loads) and tested by all 64 lanes.
+// compact live photons and stored records.  A pass gathers over a hashed grid
+// of its one radius; ppm_map_build, for any radius, makes a balanced binary
+// tree over Morton-sorted leaves of LEAF photons, walked by a lane, or the
+// four of a quad, per query.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -630,9 +631,9 @@ hipError_t launch_photons_out(hipStream_t s, const PhotonBuf& pb, uint32_t base,
 // ===========================================================================
 // Photon map build (photonmap.rs:23-29).  The reference inserts photons one
 // by one into the kdtree crate; here: Morton keys in the quantisation box ->
-// LSD radix sort (8-bit digits, device-side count) -> leaves of 64
-// consecutive photons -> balanced binary tree (heap order) of AABBs built
-// bottom-up with arrival counters.
+// LSD radix sort (8-bit digits, device-side count) -> leaves of LEAF
+// consecutive photons -> balanced binary tree (heap order) of AABBs, the
+// lowest six levels folded in LDS, the rest by one block.
 
 __device__ __forceinline__ uint32_t expand_bits10(uint32_t v) {
   v &= 0x3FFu;
